@@ -14,6 +14,8 @@
 
 #define HD __host__ __device__ __forceinline__
 
+#include "hamr_arith.h"
+
 namespace hamr {
 
 enum { RHO = 0, UU = 1, U1 = 2, U2 = 3, U3 = 4, B1 = 5, B2 = 6, B3 = 7, KTOT = 8, NPR = 9 };
@@ -33,19 +35,6 @@ constexpr double kGAMMAMAX = 80.;
 
 template <class T> HD T mymax(T a, T b) { return (a > b) ? a : b; }
 template <class T> HD T mymin(T a, T b) { return (a < b) ? a : b; }
-
-// Division, reciprocal square root and power in the arithmetic of R: IEEE
-// double operations for the FP64 step (the reference's), the hardware's
-// single-precision reciprocal, reciprocal square root and exp2/log2 (about
-// one ulp each) for the FP32 path.
-template <class R> HD R dv(R a, R b) { return a / b; }
-template <class R> HD R rsq(R a) { return R(1.) / sqrt(a); }
-template <class R> HD R rpow(R a, R e) { return pow(a, e); }
-#if defined(__HIP_DEVICE_COMPILE__)
-template <> HD float dv<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-template <> HD float rsq<float>(float a) { return __builtin_amdgcn_rsqf(a); }
-template <> HD float rpow<float>(float a, float e) { return __builtin_amdgcn_exp2f(e * __builtin_amdgcn_logf(a)); }
-#endif
 
 // Local geometry: packed symmetric gcov/gcon (00,01,02,03,11,12,13,22,23,33) and sqrt(-g).
 // oma = 1 - alpha (lapse alpha = 1/sqrt(-g^00)), formed in FP64 by the FP32 path only.
@@ -97,15 +86,17 @@ template <class R> HD void ucon_calc(const R *pr, const Geom<R> &G, R *ucon)
     alpha = rsq(-G.gcon[0]);
     for (int j = 1; j < 4; j++) beta[j] = G.gcon[j] * alpha * alpha;
     gamma_calc(pr, G.gcov, &gamma);
-    ucon[0] = dv(gamma, alpha);
-    for (int j = 1; j < 4; j++) ucon[j] = pr[U1 + j - 1] - dv(gamma * beta[j], alpha);
+    const Div<R> by_alpha(alpha);
+    ucon[0] = by_alpha(gamma);
+    for (int j = 1; j < 4; j++) ucon[j] = pr[U1 + j - 1] - by_alpha(gamma * beta[j]);
 }
 
 // GPU_phys_mhd.h:738
 template <class R> HD void bcon_calc(const R *pr, const R *ucon, const R *ucov, R *bcon)
 {
     bcon[0] = pr[B1] * ucov[1] + pr[B2] * ucov[2] + pr[B3] * ucov[3];
-    for (int j = 1; j < 4; j++) bcon[j] = dv(pr[B1 - 1 + j] + bcon[0] * ucon[j], ucon[0]);
+    const Div<R> by_ut(ucon[0]);
+    for (int j = 1; j < 4; j++) bcon[j] = by_ut(pr[B1 - 1 + j] + bcon[0] * ucon[j]);
 }
 
 // GPU_phys_mhd.h:692
@@ -129,8 +120,8 @@ template <class R> HD void vchar_coord(const R *pr, const State<R> &q, int dir, 
     if (dir == 1) { Acon_0 = G.gcon[1]; Acon_js = G.gcon[4]; }
     else if (dir == 2) { Acon_0 = G.gcon[2]; Acon_js = G.gcon[7]; }
     else { Acon_0 = G.gcon[3]; Acon_js = G.gcon[9]; }
-    cs2 = dv(gam * (gam - R(1.)) * pr[UU], w);
-    va2 = dv(bsq, eta);
+    cs2 = Div<R>(w)(gam * (gam - R(1.)) * pr[UU]);
+    va2 = Div<R>(eta)(bsq);
     cms2 = cs2 + va2 - cs2 * va2;
     if (cms2 < R(0.)) cms2 = R(kSMALL);
     if (cms2 > R(1.)) cms2 = R(1.);
@@ -149,8 +140,9 @@ template <class R> HD void vchar_coord(const R *pr, const State<R> &q, int dir, 
     if ((discr < R(0.0)) && (discr > R(-1.e-10))) discr = R(0.0);
     else if (discr < R(-1.e-10)) discr = R(0.);
     discr = sqrt(discr);
-    vp = dv(-(-B + discr), R(2.) * A);
-    vm = dv(-(-B - discr), R(2.) * A);
+    const Div<R> by_2A(R(2.) * A);
+    vp = by_2A(-(-B + discr));
+    vm = by_2A(-(-B - discr));
     *vmax = mymax(vp, vm);
     *vmin = mymin(vp, vm);
 }
@@ -248,7 +240,7 @@ template <class R> HD R mc_slope(R ym, R y0, R yp)
 // (GPU_interp.h:89-90): a_{c+1/2} = (y_c + y_{c+1})/2 - (dq_{c+1} - dq_c)/6.
 template <class R> HD R ppm_face(R ym, R yp, R dqm, R dqp)
 {
-    return R(0.5) * (yp + ym) - dv(dqp - dqm, R(6.0));
+    return R(0.5) * (yp + ym) - Div<R>(R(6.0))(dqp - dqm);
 }
 
 // CW84 monotonicity limits of the parabola of a cell with mean x3 and interface

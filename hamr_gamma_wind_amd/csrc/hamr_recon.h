@@ -55,9 +55,10 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
     const R cmin = fabs(mymax(mymax(R(0.), -cmin_l), -cmin_r));
     const R ctop = mymax(cmax, cmin);
     R *Fb = F + NPR * B.off + cell;
+    const Div<R> by_c(cmax + cmin + R(kSMALL));
 #pragma unroll
     for (int k = 0; k < NPR; k++)
-        Fb[(int64_t)k * K] = dv(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]), cmax + cmin + R(kSMALL));
+        Fb[(int64_t)k * K] = by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]));
     const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
     return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
 }
