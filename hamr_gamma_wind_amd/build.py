@@ -22,7 +22,13 @@ ARCH = os.environ.get("HAMR_OFFLOAD_ARCH", "gfx950")
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-Wall", "-Wno-unused-variable",
           "-Wno-unused-function", "-I" + CSRC]
-DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# No machine LICM: the kernels' outer loop walks work-list items and mostly runs
+# once, but the pass lifts the literals of its body (the FP64 polynomials, the
+# Newton constants) out of it, where they hold registers throughout: k_update
+# needs 155 VGPRs without it and spills at 168 with it, the FP64 HLLC fluxes 238
+# instead of 256 and 84 bytes of scratch.
+DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+          "-mllvm", "-disable-machine-licm"]
 
 SOURCES = [
     ("hamr_kernels.hip", True),

@@ -39,6 +39,8 @@ template <> HD float rpow<float>(float a, float e) { return __builtin_amdgcn_exp
 template <class R> struct Div {
     R d;
     HD explicit Div(R b) : d(b) {}
+    HD Div(R b, R) : d(b) {}  // with the reciprocal formed earlier
+    HD R recip() const { return R(0.); }
     HD R operator()(R a) const { return dv(a, d); }
 };
 #if HAMR_DEVICE_ARITH
@@ -50,6 +52,8 @@ template <> struct Div<double> {
         y = fma(y, fma(-b, y, 1.), y);
         y = fma(y, fma(-b, y, 1.), y);
     }
+    HD Div(double b, double r) : d(b), y(r) {}
+    HD double recip() const { return y; }
     HD double operator()(double a) const
     {
         const double q = a * y;

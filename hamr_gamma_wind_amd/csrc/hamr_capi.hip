@@ -76,6 +76,7 @@ struct hamr_ctx {
     double *gcov = nullptr, *gcon = nullptr, *gdet = nullptr, *conn = nullptr, *rcen = nullptr;
     double *tet = nullptr;         // face tetrads of the HLLC solver (96 per metric column)
     float *g32 = nullptr;          // the metric in FP32 (KParams::g32)
+    double *colc = nullptr;        // per-column values of the update (KParams::colc)
     BlockDev *blk = nullptr;
     int *ring = nullptr, *rside = nullptr;  // polar rings
     int nring = 0, ring_len = 0, ni_max = 0;
@@ -363,7 +364,7 @@ static int init_device(hamr_ctx *c)
     const size_t KC = (size_t)c->cols;
     if (dalloc(c, &c->gcov, NPOS * 10 * KC) || dalloc(c, &c->gcon, NPOS * 10 * KC) || dalloc(c, &c->gdet, NPOS * KC) ||
         dalloc(c, &c->conn, 40 * KC) || dalloc(c, &c->rcen, KC) || dalloc(c, &c->tet, 96 * KC) ||
-        dalloc(c, &c->g32, NPOS * G32N * KC) || dalloc(c, &c->blk, nb))
+        dalloc(c, &c->g32, NPOS * G32N * KC) || dalloc(c, &c->colc, COLN * KC) || dalloc(c, &c->blk, nb))
         return -1;
     {
         // (sets the blocks' kPushWhole flags before they are uploaded)
@@ -401,6 +402,7 @@ static int init_device(hamr_ctx *c)
     P.rcen = c->rcen;
     P.tet = c->tet;
     P.g32 = c->g32;
+    P.colc = c->colc;
     P.push3 = c->push3;
     P.tiled_push = c->amr ? 1 : 0;
     P.xp = c->p;
@@ -1022,6 +1024,9 @@ int hamr_upload_metric(hamr_ctx *c, int geo, const double *gcov, const double *g
     if (check_launch(c, "hamr_upload_metric")) return -1;
     if (h2d(c, c->conn + mo * 40, conn, 40 * KC * sizeof(double))) return -1;
     if (h2d(c, c->rcen + mo, rcen, KC * sizeof(double))) return -1;
+    launch_col_consts(c->gcon + mo * NPOS * 10, c->gdet + mo * NPOS, c->rcen + mo, c->d.rho_floor, c->d.u_floor,
+                      c->colc + mo * COLN, (int64_t)KC, c->s);
+    if (check_launch(c, "hamr_upload_metric")) return -1;
     // the HLLC solver's face tetrads follow the metric (set_Mud after set_grid)
     std::vector<double> tet(96 * KC);
     fill_tetrads(gcov, gcon, (int64_t)G.D1 * G.D2, (int64_t)KC, tet.data());

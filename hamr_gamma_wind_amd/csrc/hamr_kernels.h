@@ -20,6 +20,9 @@ struct KParams {
     // formed in FP64 first: g32[moff*NPOS*G32N + (pos*G32N + s)*kcol + col],
     // s = 0-9 gcov, 10-19 gcon, 20 gdet, 21 1 - 1/sqrt(-g^00).
     const float *g32;
+    // Values of each metric column at the cell centre that every cell of the column
+    // would otherwise form: colc[moff*COLN + v*kcol + col] (ColConst).
+    const double *colc;
     int riemann;        // HAMR_RIEMANN_HLL (0) or HAMR_RIEMANN_HLLC (1), in either arithmetic
     const PushEntry *push3;  // push table (rows from BlockDev::push3)
     int tiled_push;          // 1: a multi-level set (per-tile push entries); 0: every face one entry
@@ -68,6 +71,10 @@ struct Launch {
     int line = 0;  // flux launches: 1 = line-staged tiles (KC_LINE lists), 0 = one thread per face (KC_FLUX lists)
 };
 
+// KParams::colc: 1/sqrt(-g^00) and the reciprocal Div forms of it, beta^j = g^0j
+// alpha^2, n_0 = -sqrt(-1/g^00), the reciprocal Div forms of gdet, and the
+// floors of rho and u.
+enum ColConst : int { CC_ALPHA = 0, CC_RALPHA, CC_BETA1, CC_BETA2, CC_BETA3, CC_NCOV, CC_RG, CC_RHOFLR, CC_UFLR, COLN };
 constexpr int G32N = 22;  // FP32 metric values per column and position (KParams::g32)
 
 // Tiles of the line-staged flux kernel (kLineT threads per workgroup) of
@@ -200,6 +207,9 @@ void launch_rdump_unpack(const KParams &P, const int *blist, const int64_t *roff
 constexpr int DREC = 9;
 void launch_dump_pack(const KParams &P, const int *blist, const int64_t *doff, const int64_t *doff_host, int first,
                       int count, int64_t max_cells, const double *p, float *out, hipStream_t s);
+// The column values (KParams::colc) of one geometry slab from its metric.
+void launch_col_consts(const double *gcon, const double *gdet, const double *rcen, double rho_floor, double u_floor,
+                       double *colc, int64_t kcol, hipStream_t s);
 // The FP32 metric (KParams::g32) of ncol columns of one geometry slab from its
 // FP64 metric (the slab's pointers into gcov, gcon, gdet and g32).
 void launch_geom32(const double *gcov, const double *gcon, const double *gdet, float *g32, int64_t kcol,

@@ -62,6 +62,19 @@ __device__ __forceinline__ Geom<R> load_geom(const KParams &P, const BlockDev &B
     return G;
 }
 
+// Element g of a slab whose base is the same for the whole wavefront: the base
+// stays in scalar registers and g is a 32-bit offset, so that an access takes no
+// 64-bit vector address arithmetic (a slab holds fewer than 2^29 cells: the
+// memory of one GPU does not hold the arrays of a larger one).
+template <class T> __device__ __forceinline__ T gld(const T *base, uint32_t g)
+{
+    return *(const T *)((const char *)base + (uint32_t)(g * (uint32_t)sizeof(T)));
+}
+template <class T> __device__ __forceinline__ void gst(T *base, uint32_t g, T v)
+{
+    *(T *)((char *)base + (uint32_t)(g * (uint32_t)sizeof(T))) = v;
+}
+
 // The step Dt of block B: the launch's Dt (dt_ptr[0] dt_mult when the launch
 // reads dt from the device, else Dt_val), scaled by the block's time level in
 // a local-adaptive-time-stepping cycle (a block of time level tl advances by

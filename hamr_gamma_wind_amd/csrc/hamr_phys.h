@@ -79,17 +79,31 @@ template <class R> HD int gamma_calc(const R *pr, const R *gcov, R *gamma)
     return 0;
 }
 
+// Lapse and shift of a geometry: alpha = 1/sqrt(-g^00), beta^j = g^0j alpha^2.
+template <class R> struct Lapse {
+    R alpha, beta[4];
+    Div<R> by_alpha;
+    HD explicit Lapse(const Geom<R> &G) : alpha(rsq(-G.gcon[0])), by_alpha(alpha)
+    {
+        for (int j = 1; j < 4; j++) beta[j] = G.gcon[j] * alpha * alpha;
+    }
+    HD Lapse(R a, const Div<R> &by, R b1, R b2, R b3) : alpha(a), by_alpha(by)
+    {
+        beta[1] = b1;
+        beta[2] = b2;
+        beta[3] = b3;
+    }
+};
+
 // GPU_phys_mhd.h:714
-template <class R> HD void ucon_calc(const R *pr, const Geom<R> &G, R *ucon)
+template <class R> HD void ucon_calc(const R *pr, const Geom<R> &G, const Lapse<R> &L, R *ucon)
 {
-    R alpha, gamma, beta[4];
-    alpha = rsq(-G.gcon[0]);
-    for (int j = 1; j < 4; j++) beta[j] = G.gcon[j] * alpha * alpha;
+    R gamma;
     gamma_calc(pr, G.gcov, &gamma);
-    const Div<R> by_alpha(alpha);
-    ucon[0] = by_alpha(gamma);
-    for (int j = 1; j < 4; j++) ucon[j] = pr[U1 + j - 1] - by_alpha(gamma * beta[j]);
+    ucon[0] = L.by_alpha(gamma);
+    for (int j = 1; j < 4; j++) ucon[j] = pr[U1 + j - 1] - L.by_alpha(gamma * L.beta[j]);
 }
+template <class R> HD void ucon_calc(const R *pr, const Geom<R> &G, R *ucon) { ucon_calc(pr, G, Lapse<R>(G), ucon); }
 
 // GPU_phys_mhd.h:738
 template <class R> HD void bcon_calc(const R *pr, const R *ucon, const R *ucov, R *bcon)
@@ -100,14 +114,15 @@ template <class R> HD void bcon_calc(const R *pr, const R *ucon, const R *ucov, 
 }
 
 // GPU_phys_mhd.h:692
-template <class R> HD void get_state(const R *pr, const Geom<R> &G, State<R> &q)
+template <class R> HD void get_state(const R *pr, const Geom<R> &G, const Lapse<R> &L, State<R> &q)
 {
-    ucon_calc(pr, G, q.ucon);
+    ucon_calc(pr, G, L, q.ucon);
     lower10(q.ucon, G.gcov, q.ucov);
     bcon_calc(pr, q.ucon, q.ucov, q.bcon);
     lower10(q.bcon, G.gcov, q.bcov);
     if constexpr (sizeof(R) == 4) q.opu = one_plus_ut(pr, G);
 }
+template <class R> HD void get_state(const R *pr, const Geom<R> &G, State<R> &q) { get_state(pr, G, Lapse<R>(G), q); }
 
 template <class R> HD R dot4(const R *a, const R *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3]; }
 
@@ -271,9 +286,21 @@ struct InvPre {
     double Bsq, QdotB, QdotBsq, Qtsq, Qdotn, D;
 };
 
-HD void inv_prepare(const double *Ut, const double *gcov, const double *gcon, InvPre &s)
+// Quantities of one metric column the inversions use: 1/sqrt(-g^00), n_0 =
+// -sqrt(-1/g^00) and quotients by gdet.
+struct InvCol {
+    double alpha, ncov;
+    Div<double> by_g;
+    HD InvCol(const double *gcon, double gdet)
+        : alpha(1.0 / sqrt(-gcon[0])), ncov(-sqrt(-1. / gcon[0])), by_g(gdet)
+    {
+    }
+    HD InvCol(double a, double n, const Div<double> &g) : alpha(a), ncov(n), by_g(g) {}
+};
+
+HD void inv_prepare(const double *Ut, const double *gcov, const double *gcon, double ncov, InvPre &s)
 {
-    double Bcov[4], Qcov[4], ncov, Qsq;
+    double Bcov[4], Qcov[4], Qsq;
     s.Bcon[0] = 0.;
     for (int i = 1; i < 4; i++) s.Bcon[i] = Ut[B1 + i - 1];
     lower10(s.Bcon, gcov, Bcov);
@@ -284,7 +311,6 @@ HD void inv_prepare(const double *Ut, const double *gcov, const double *gcon, In
     s.QdotB = 0.;
     for (int i = 0; i < 4; i++) s.QdotB += Qcov[i] * s.Bcon[i];
     s.QdotBsq = s.QdotB * s.QdotB;
-    ncov = -sqrt(-1. / gcon[0]);
     s.ncon[0] = gcon[0] * ncov;
     s.ncon[1] = gcon[1] * ncov;
     s.ncon[2] = gcon[2] * ncov;
@@ -309,9 +335,11 @@ HD double utsq_of(const double *prim, const double *gcov)
 
 HD void set_utcon(const InvPre &s, double gamma, double W, double *prim)
 {
+    const double f = gamma / (W + s.Bsq);
+    const Div<double> by_W(W);
     for (int i = 1; i < 4; i++) {
         double Qtcon = s.Qcon[i] + s.ncon[i] * s.Qdotn;
-        prim[U1 + i - 1] = gamma / (W + s.Bsq) * (Qtcon + s.QdotB * s.Bcon[i] / W);
+        prim[U1 + i - 1] = f * (Qtcon + by_W(s.QdotB * s.Bcon[i]));
     }
 }
 
@@ -327,26 +355,29 @@ HD int gnr_2d(double *x, const InvPre &s, double gam)
     double dx[2], x_old[2], errx = 1., f = 1., df = 1.;
     int n_iter = 0, i_extra = 0, doing_extra = 0, keep = 1;
     const double Bsq = s.Bsq, Qtsq = s.Qtsq, QdotBsq = s.QdotBsq, Qdotn = s.Qdotn, D = s.D;
+    const Div<double> by_gam(gam);
+    Div<double> by_W(x[0]);  // of the current x[0]: 1/x[0] here, the relative change at the loop's end
     while (keep) {
         double Wsq, p_tmp, dPdvsq, dPdW, gtmp, t11, t16, t18, t2, t21, t23, t24, t25, t3, t35, t36, t4, t40, t9;
         Wsq = x[0] * x[0];
         gtmp = 1. - x[1];
-        p_tmp = (gam - 1.) * (fma(x[0], gtmp, -D * sqrt(gtmp))) / gam;
-        dPdW = (gam - 1.) * (1. - x[1]) / gam;
-        dPdvsq = (gam - 1.) * (fma(0.5, D / sqrt(1. - x[1]), -x[0])) / gam;
+        const double sg = sqrt(gtmp);
+        p_tmp = by_gam((gam - 1.) * (fma(x[0], gtmp, -D * sg)));
+        dPdW = by_gam((gam - 1.) * gtmp);
+        dPdvsq = by_gam((gam - 1.) * (fma(0.5, Div<double>(sg)(D), -x[0])));
         t2 = -0.5 * Bsq + dPdvsq;
         t3 = Bsq + x[0];
         t4 = t3 * t3;
-        t9 = 1. / Wsq;
+        t9 = Div<double>(Wsq)(1.);
         t11 = Qtsq - x[1] * t4 + QdotBsq * (Bsq + 2.0 * x[0]) * t9;
         t16 = QdotBsq * t9;
         t18 = -Qdotn - 0.5 * Bsq * (1.0 + x[1]) + 0.5 * t16 - x[0] + p_tmp;
-        t21 = 1. / t3;
-        t23 = 1. / x[0];
+        t21 = Div<double>(t3)(1.);
+        t23 = by_W(1.);
         t24 = t16 * t23;
         t25 = -1.0 + dPdW - t24;
         t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (QdotBsq + x[1] * Wsq * x[0]) * t9 * t23;
-        t36 = 1. / t35;
+        t36 = Div<double>(t35)(1.);
         dx[0] = -(t2 * t11 + t4 * t18) * t21 * t36;
         t40 = (x[1] + t24) * t3;
         dx[1] = -(-t25 * t11 - 2.0 * t40 * t18) * t21 * t36;
@@ -360,7 +391,8 @@ HD int gnr_2d(double *x, const InvPre &s, double gam)
         x[0] = (x[0] > kW_TOO_BIG) ? x_old[0] : x[0];
         x[1] = (x[1] < 0.) ? 0. : x[1];
         x[1] = (x[1] > 1.) ? (1. - 1.e-15) : x[1];
-        errx = (x[0] == 0.) ? fabs(x[0] - x_old[0]) : fabs((x[0] - x_old[0]) / x[0]);
+        by_W = Div<double>(x[0]);
+        errx = (x[0] == 0.) ? fabs(x[0] - x_old[0]) : fabs(by_W(x[0] - x_old[0]));
         if ((fabs(errx) <= kNEWT_TOL) && (doing_extra == 0) && (kEXTRA_NEWT_ITER > 0)) doing_extra = 1;
         if (doing_extra == 1) i_extra++;
         if (((fabs(errx) <= kNEWT_TOL) && (doing_extra == 0)) || (i_extra > kEXTRA_NEWT_ITER) || (n_iter >= (kMAX_NEWT_ITER - 1))) keep = 0;
@@ -373,12 +405,12 @@ HD int gnr_2d(double *x, const InvPre &s, double gam)
 }
 
 // GPU_utoprim_2d.h Utoprim_new_body
-HD int body_2d(const double *Ut, const double *gcov, const double *gcon, double *prim, double gam)
+HD int body_2d(const double *Ut, const double *gcov, const double *gcon, double ncov, double *prim, double gam)
 {
     InvPre s;
     double x[2], utsq, gammasq, gamma, rho0, u, p, w, W_last, W, vsq, gtmp, xv;
     int i_increase, retval;
-    inv_prepare(Ut, gcov, gcon, s);
+    inv_prepare(Ut, gcov, gcon, ncov, s);
     utsq = utsq_of(prim, gcov);
     if ((utsq < 0.) && (fabs(utsq) < 1.0e-13)) utsq = fabs(utsq);
     if (utsq < 0. || utsq > kUTSQ_TOO_BIG) return 2;
@@ -464,12 +496,12 @@ HD int gnr_1dvsq2(double *x, const InvPre &s, double K, double gam)
 }
 
 // GPU_utoprim_1dvsq2fix1.h Utoprim_new_body2
-HD int body_1dvsq2(const double *Ut, const double *gcov, const double *gcon, double *prim, double K, double gam)
+HD int body_1dvsq2(const double *Ut, const double *gcov, const double *gcon, double ncov, double *prim, double K, double gam)
 {
     InvPre s;
     double x[1], utsq, gammasq, gamma, rho0, u, p, W, vsq, gtmp;
     int retval;
-    inv_prepare(Ut, gcov, gcon, s);
+    inv_prepare(Ut, gcov, gcon, ncov, s);
     utsq = utsq_of(prim, gcov);
     if ((utsq < 0.) && (fabs(utsq) < 1.0e-13)) utsq = fabs(utsq);
     if (utsq < 0. || utsq > kUTSQ_TOO_BIG) return 2;
@@ -578,12 +610,12 @@ HD int gnr_1dfix(double *x, const InvPre &s, double K, double rho_g0, double gam
 }
 
 // GPU_utoprim_1dfix1.h Utoprim_new_body3
-HD int body_1dfix(const double *Ut, const double *gcov, const double *gcon, double *prim, double K, double gam)
+HD int body_1dfix(const double *Ut, const double *gcov, const double *gcon, double ncov, double *prim, double K, double gam)
 {
     InvPre s;
     double x[1], utsq, gammasq, gamma, rho0, u, p, w, W_last, W, vsq, gtmp;
     int i_increase, retval;
-    inv_prepare(Ut, gcov, gcon, s);
+    inv_prepare(Ut, gcov, gcon, ncov, s);
     utsq = utsq_of(prim, gcov);
     if ((utsq < 0.) && (fabs(utsq) < 1.0e-13)) utsq = fabs(utsq);
     if (utsq < 0. || utsq > kUTSQ_TOO_BIG) return 2;
@@ -621,23 +653,23 @@ HD int body_1dfix(const double *Ut, const double *gcov, const double *gcon, doub
 
 // Utoprim_2d / _1dvsq2fix1 / _1dfix1 wrappers: normal-observer frame transform,
 // body, write-back only on success (face fields always rewritten).
-HD int utoprim(int which, const double *U, const double *gcov, const double *gcon, double gdet, double gam,
+HD int utoprim(int which, const double *U, const double *gcov, const double *gcon, const InvCol &C, double gam,
                double *prim)
 {
-    double Ut[NPR], pt[5], alpha, K = 0.;
+    double Ut[NPR], pt[5], K = 0.;
+    const double alpha = C.alpha, ncov = C.ncov;
     int ret;
     if (U[0] <= 0.) return -100;
-    for (int i = B1; i <= B3; i++) prim[i] = U[i] / gdet;
-    alpha = 1.0 / sqrt(-gcon[0]);
-    Ut[RHO] = alpha * U[RHO] / gdet;
-    Ut[UU] = alpha * (U[UU] - U[RHO]) / gdet;
-    for (int i = U1; i <= U3; i++) Ut[i] = alpha * U[i] / gdet;
-    for (int i = B1; i <= B3; i++) Ut[i] = alpha * U[i] / gdet;
+    for (int i = B1; i <= B3; i++) prim[i] = C.by_g(U[i]);
+    Ut[RHO] = C.by_g(alpha * U[RHO]);
+    Ut[UU] = C.by_g(alpha * (U[UU] - U[RHO]));
+    for (int i = U1; i <= U3; i++) Ut[i] = C.by_g(alpha * U[i]);
+    for (int i = B1; i <= B3; i++) Ut[i] = C.by_g(alpha * U[i]);
     for (int i = 0; i < B1; i++) pt[i] = prim[i];
     if (which != 0) K = U[KTOT] / U[RHO];
-    if (which == 0) ret = body_2d(Ut, gcov, gcon, pt, gam);
-    else if (which == 1) ret = body_1dvsq2(Ut, gcov, gcon, pt, K, gam);
-    else ret = body_1dfix(Ut, gcov, gcon, pt, K, gam);
+    if (which == 0) ret = body_2d(Ut, gcov, gcon, ncov, pt, gam);
+    else if (which == 1) ret = body_1dvsq2(Ut, gcov, gcon, ncov, pt, K, gam);
+    else ret = body_1dfix(Ut, gcov, gcon, ncov, pt, K, gam);
     if (ret == 0)
         for (int i = 0; i < B1; i++) prim[i] = pt[i];
     return ret;
