@@ -34,10 +34,20 @@ enum TuneSlot : int {
 constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_CORNER, KC_CORNER, KC_INTERIOR,
                                    KC_INTERIOR, KC_INTERIOR, KC_BOUND1, KC_BOUND2, KC_BOUND3, -1};
 
+// Default item order of a class.  In chunks per XCD where tiles share what they
+// read with the next tiles (the stencils of fluxes, EMFs and face update, the
+// rows of the x1 and x2 ghost copies): plain -> chunked order 950 -> 803 us (x1
+// fluxes, mixed, 384x192x192), 292 -> 231 (256x128x128), 61 -> 44 (126x100x78
+// as 42x25x39 blocks), 445 -> 323 (722 blocks); corner EMFs 32 -> 24 us and 155 ->
+// 151, x2 ghosts 236 -> 208, the others 0-7%.  Plain for the interior updates, whose
+// tiles share almost nothing (1.80 -> 1.81 ms, 904 -> 930 us on 722 blocks) and take
+// unequal times, and for the x3 ghost rows (11 -> 19 us on 64x32x32).
+static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_BOUND3 ? 0 : 1; }
+
 struct TuneCfg {
     int tile = kDefaultTile;  // index into kTiles
     int grid = 0;             // workgroups; 0: one per item
-    int swz = 0;              // XCD-contiguous item order
+    int swz = 0;              // item order in chunks per XCD (WorkList; the default: default_swz)
     int march = 0;            // TS_CONS only: the x1-marching form (tile, grid, swz unused)
     int alt = 0;              // the slot's second form: flux slots line-staged tiles (KC_LINE lists)
                               // instead of one thread per face; TS_CONS k_cons + k_invert instead of k_update
@@ -321,7 +331,7 @@ static Launch block_launch(const hamr_ctx *c, int cls, int n)
     x.threads = kTiles[kDefaultTile];
     x.wl.items = L.items[kDefaultTile] ? L.items[kDefaultTile] + L.start[kDefaultTile][n] : nullptr;
     x.wl.n = L.count[kDefaultTile][n];
-    x.wl.swz = 0;
+    x.wl.swz = default_swz(cls);
     x.grid = x.wl.n;
     x.lds_cols = L.lds_cols[kDefaultTile];
     x.line = (cls >= KC_LINE1 && cls <= KC_LINE3) ? 1 : 0;
@@ -389,6 +399,8 @@ static int init_device(hamr_ctx *c)
     if (h2d(c, c->io_roff, c->roff.data(), (nb + 1) * sizeof(int64_t))) return -1;
     if (h2d(c, c->io_doff, c->doff.data(), (nb + 1) * sizeof(int64_t))) return -1;
     if (build_class_lists(c)) return -1;
+    for (int slot = 0; slot < TS_N; slot++)
+        if (kSlotClass[slot] >= 0) c->tune[slot].swz = default_swz(kSlotClass[slot]);
     KParams &P = c->P;
     P.gam = c->d.gam;
     P.cour = c->d.cour;
@@ -1826,7 +1838,7 @@ static Launch las_launch(const hamr_ctx *c, int cls, int s, int ph)
     x.threads = kTiles[kDefaultTile];
     x.wl.items = c->las_items ? c->las_items + o[0] : nullptr;
     x.wl.n = (int)o[1];
-    x.wl.swz = 0;
+    x.wl.swz = default_swz(cls);
     x.grid = x.wl.n;
     x.lds_cols = c->cl[cls].lds_cols[kDefaultTile];
     x.line = 0;

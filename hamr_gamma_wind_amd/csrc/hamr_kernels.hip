@@ -538,7 +538,7 @@ __global__ void __launch_bounds__(256) k_invert(KParams P, WorkList wl, int full
 // cell, 2592 -> 2010 VALU instructions, and the literals are left in the loop
 // (build.py): 2.09 -> 1.60 ms.
 template <class R, bool TILED>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILED ? 2 : 3)))
 k_update(KParams P, WorkList wl, int full, double Dt_val, const double *__restrict__ dt_ptr, double dt_mult,
          const double *__restrict__ pi, const double *__restrict__ pb, double *__restrict__ pf_out,
          double *__restrict__ U0, double *__restrict__ Unew, const double *__restrict__ psf, const R *__restrict__ F1,

@@ -19,8 +19,15 @@ __device__ __forceinline__ void region_index(int t, int n2, int n3, int &a, int 
 __device__ __forceinline__ int2 wl_get(const WorkList &wl, int w)
 {
     if (wl.swz) {
-        const int q = wl.n >> 3, r = wl.n & 7, x = w & 7, k = w >> 3;
-        w = x * q + (x < r ? x : r) + k;
+        constexpr int LC = 5;  // log2 of the items per chunk
+        const int full = wl.n >> (LC + 3), body = full << (LC + 3);
+        if (w < body) {
+            const int x = w & 7, k = w >> 3;
+            w = ((((k >> LC) << 3) + x) << LC) + (k & ((1 << LC) - 1));
+        } else {  // the last, partial round: one contiguous range per XCD
+            const int v = w - body, m = wl.n - body, q = m >> 3, r = m & 7, x = v & 7, k = v >> 3;
+            w = body + x * q + (x < r ? x : r) + k;
+        }
     }
     return wl.items[w];
 }

@@ -385,7 +385,7 @@ int hamr_time_stage(hamr_ctx *ctx, int stage, int nrep, double *avg_ms);
  * Every kernel of the step walks a work list of (block, tile) items.  For each
  * kernel (HAMR_TUNE_*) the tuner times, on the current state, the tile sizes
  * 64/128/256 threads, grids of one workgroup per item or 1024/2048/4096
- * persistent workgroups, and item orders plain or XCD-contiguous, and keeps the
+ * persistent workgroups, and item orders plain or in chunks per XCD, and keeps the
  * fastest (nrep timed launches each).  Results do not depend on the choice.
  * The step graph is re-captured after a change. */
 enum {
@@ -395,7 +395,7 @@ enum {
 };
 int hamr_autotune(hamr_ctx *ctx, int nrep);
 /* cfg[3]: threads per workgroup, workgroups (0: one per item), flags; ms:
- * tuned time (-1: not tuned).  Flags bit 0: XCD-contiguous item order; bit 1,
+ * tuned time (-1: not tuned).  Flags bit 0: item order in chunks per XCD; bit 1,
  * the slot's second form: for HAMR_TUNE_FLUX1-3 line-staged tiles of 256
  * threads (each cell's slope, interface and limited parabola formed once per
  * tile) instead of one thread per face; for HAMR_TUNE_CONS the conserved
