@@ -32,7 +32,7 @@ enum TuneSlot : int {
     TS_BOUND1, TS_BOUND2, TS_BOUND3, TS_EXCHANGE, TS_N
 };
 constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_CORNER, KC_CORNER, KC_INTERIOR,
-                                   KC_INTERIOR, KC_INTERIOR, KC_BOUND1, KC_BOUND2, KC_BOUND3, -1};
+                                   KC_INTERIOR, KC_FLAGS, KC_BOUND1, KC_BOUND2, KC_BOUND3, -1};
 
 // Default item order of a class.  In chunks per XCD where tiles share what they
 // read with the next tiles (the stencils of fluxes, EMFs and face update, the
@@ -42,7 +42,7 @@ constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_COR
 // 151, x2 ghosts 236 -> 208, the others 0-7%.  Plain for the interior updates, whose
 // tiles share almost nothing (1.80 -> 1.81 ms, 904 -> 930 us on 722 blocks) and take
 // unequal times, and for the x3 ghost rows (11 -> 19 us on 64x32x32).
-static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_BOUND3 ? 0 : 1; }
+static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_FLAGS || cls == KC_BOUND3 ? 0 : 1; }
 
 struct TuneCfg {
     int tile = kDefaultTile;  // index into kTiles
@@ -1496,13 +1496,11 @@ int hamr_ct_update(hamr_ctx *c, int flag, double Dt, int n)
 int hamr_update(hamr_ctx *c, int flag, int n, double Dt)
 {
     if (!c || !valid_block(c, n)) return fail(c, "hamr_update: bad block");
-    const Launch L = block_launch(c, KC_INTERIOR, n);
-    if (flag)
-        launch_update(c->P, L, 1, Dt, nullptr, 1.0, c->ph, c->ph, c->p, c->U0, c->Un, c->ps, c->F[0], c->F[1], c->F[2],
-                      c->pflag, c->failcnt, c->prec, c->s);
-    else
-        launch_update(c->P, L, 0, Dt, nullptr, 1.0, c->p, c->p, c->ph, c->U0, c->Un, c->psh, c->F[0], c->F[1], c->F[2],
-                      c->pflag, c->failcnt, c->prec, c->s);
+    double *in = flag ? c->ph : c->p, *out = flag ? c->p : c->ph, *psf = flag ? c->ps : c->psh;
+    for (int part : {3, 2})
+        launch_update_part(c->P, part, block_launch(c, part == 2 ? KC_FLAGS : KC_INTERIOR, n), flag ? 1 : 0, Dt, nullptr,
+                           1.0, in, in, out, c->U0, c->Un, psf, c->F[0], c->F[1], c->F[2], c->pflag, c->failcnt, c->prec,
+                           c->s);
     return check_launch(c, "hamr_update");
 }
 
@@ -1717,7 +1715,8 @@ static int stepping_levels(int s)
 }
 
 // the kernel classes a cycle launches over filtered lists
-constexpr int kLasClasses[] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_CORNER, KC_INTERIOR, KC_BOUND1, KC_BOUND2};
+constexpr int kLasClasses[] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_CORNER, KC_INTERIOR, KC_FLAGS, KC_BOUND1,
+                              KC_BOUND2};
 
 static int log2i(int v)
 {
@@ -1922,7 +1921,7 @@ static void enqueue_las_cycle(hamr_ctx *c, int maxtl)
             if (!L.wl.n) continue;
             const int full = ph == LAS_FULL;
             for (int part : {3, 2})
-                launch_update_part(P, part, L, full, 0., c->dt, full ? 1.0 : 0.5, las_in(c, ph), las_in(c, ph),
+                launch_update_part(P, part, part == 2 ? las_launch(c, KC_FLAGS, s, ph) : L, full, 0., c->dt, full ? 1.0 : 0.5, las_in(c, ph), las_in(c, ph),
                                    las_out(c, ph), c->U0, c->Un, las_outs(c, ph), c->F[0], c->F[1], c->F[2], c->pflag,
                                    c->failcnt, mixed, st);
         }

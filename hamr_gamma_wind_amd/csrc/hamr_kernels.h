@@ -115,8 +115,10 @@ enum KClass : int {
     KC_INTERIOR,                       // interior cells               (update, inversion, fallback)
     KC_BOUND1, KC_BOUND2, KC_BOUND3,   // ghost layers of one direction
     KC_LINE1, KC_LINE2, KC_LINE3,      // line-staged flux tiles of one direction (line_tiles)
+    KC_FLAGS,                          // the flag slab, kFlagsPerThread cells per thread (fallback)
     KC_N
 };
+constexpr int kFlagsPerThread = 16;
 // Threads a block needs in a kernel class.
 int64_t class_work(const BlockDev &B, int cls);
 // Metric columns a tile of `threads` interior cells of a block with bs3 cells
@@ -140,10 +142,6 @@ void launch_pole(const KParams &P, const int *ring, const int *rside, int nring,
                  const double *dt_ptr, void *E, int mixed, hipStream_t s);
 void launch_ct_update(const KParams &P, const Launch &L, double Dt_val, const double *dt_ptr, double dt_mult,
                       const double *psi, double *psf, const void *E, int mixed, hipStream_t s);
-void launch_update(const KParams &P, const Launch &L, int full, double Dt_val, const double *dt_ptr, double dt_mult,
-                   const double *pi, const double *pb, double *pf, double *U0, double *Unew, const double *psf,
-                   const void *F1, const void *F2, const void *F3, int *pflag, int *failcnt, int mixed,
-                   hipStream_t s);
 // Conserved update only (k_cons, predictor form with step Dt): U(p) -> U0,
 // U(p) - Dt div F + Dt S(p) with the face average of psf -> Unew.
 void launch_cons(const KParams &P, const Launch &L, double Dt, const double *p, double *U0, double *Unew,
@@ -156,8 +154,7 @@ void launch_cons_march(const KParams &P, int nblk, int max_plane, int min_bs3, i
                        double *Unew, const double *psf, const void *F1, const void *F2, const void *F3, int mixed,
                        hipStream_t s);
 // The kernels of the update one at a time: part 0 k_cons, 1 k_invert, 2
-// k_fallback, 3 k_update (k_cons and k_invert in one kernel).  launch_update
-// runs parts 3 and 2.
+// k_fallback (a KC_FLAGS list), 3 k_update (k_cons and k_invert in one kernel).
 void launch_update_part(const KParams &P, int part, const Launch &L, int full, double Dt_val, const double *dt_ptr,
                         double dt_mult, const double *pi, const double *pb, double *pf, double *U0, double *Unew,
                         const double *psf, const void *F1, const void *F2, const void *F3, int *pflag, int *failcnt,

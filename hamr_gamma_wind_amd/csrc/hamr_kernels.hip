@@ -25,6 +25,7 @@ int64_t class_work(const BlockDev &B, int cls)
     case KC_ECENT: return (b1 + 2) * (b2 + 2) * (b3 + 2);
     case KC_CORNER: return (b1 + 1) * (b2 + 1) * (b3 + 1);
     case KC_INTERIOR: return b1 * b2 * b3;
+    case KC_FLAGS: return (B.ks + kFlagsPerThread - 1) / kFlagsPerThread;
     case KC_BOUND1: return 2 * NG * d2 * d3;
     case KC_BOUND2: return 2 * NG * d1 * d3;
     default: return 2 * NG * (d1 * d2 + 1);
@@ -602,43 +603,66 @@ k_update(KParams P, WorkList wl, int full, double Dt_val, const double *__restri
     }
 }
 
-// The rest of the cascade for the cells k_invert marked: entropy-based 1D
-// (GPU_utoprim_1dvsq2fix1.h), then 1D (GPU_utoprim_1dfix1.h), then floors.
+// The rest of the cascade for the cells k_update or k_invert marked:
+// entropy-based 1D (GPU_utoprim_1dvsq2fix1.h), then 1D (GPU_utoprim_1dfix1.h),
+// then floors.  A tile looks over blockDim.x * kFlagsPerThread flags of the
+// block's slab (64 bytes per thread, ghosts and padding among them: those are
+// never marked), gathers the marked cells in LDS and inverts them, one per
+// thread.  Bound by reading the flags while few cells are marked: with a thread
+// per interior cell the launch of mostly idle workgroups with this kernel's
+// registers took 209 us on 384x192x192 (95 MB of flags).
 __global__ void __launch_bounds__(256) k_fallback(KParams P, WorkList wl, const double *__restrict__ Unew,
                                                   double *__restrict__ pf_out, int *__restrict__ pflag,
                                                   int *__restrict__ failcnt)
 {
+    __shared__ int cells[256 * kFlagsPerThread];
+    __shared__ int count;
     FOR_ITEMS(wl)
     {
         const int2 it = wl_get(wl, w_);
         const int n = it.x;
         const BlockDev &B = P.blk[n];
-        const int t = it.y * blockDim.x + threadIdx.x;
-        if (t >= B.bs[0] * B.bs[1] * B.bs[2]) continue;
-        int a, b, c;
-        region_index(t, B.bs[1], B.bs[2], a, b, c);
-        const int i = a + NG, j = b + NG, z = c + NG;
-        const int64_t K = B.ks;
-        const int64_t g = ((int64_t)i * B.D[1] + j) * B.D[2] + z, col = (int64_t)i * B.D[1] + j;
-        if (pflag[B.off + g] != kFallbackPending) continue;
-        const int64_t base = NPR * B.off + g;
-        const Geom<double> G = load_geom(P, B, CENT, col);
-        double pf[NPR], U[NPR];
+        if (threadIdx.x == 0) count = 0;
+        __syncthreads();
+        const int g0 = (it.y * (int)blockDim.x) * kFlagsPerThread + 4 * (int)threadIdx.x;
+        int4 f[kFlagsPerThread / 4];
 #pragma unroll
-        for (int k = 0; k < NPR; k++) {
-            U[k] = Unew[base + k * K];
-            pf[k] = pf_out[base + k * K];
+        for (int q = 0; q < kFlagsPerThread / 4; q++) {
+            const int g = g0 + q * 4 * (int)blockDim.x;
+            f[q] = g < B.ks ? *(const int4 *)(pflag + B.off + g) : make_int4(0, 0, 0, 0);
         }
-        const InvCol C(G.gcon, G.g);
-        int flag = utoprim(1, U, G.gcov, G.gcon, C, P.gam, pf);
-        if (flag) {
-            atomicAdd(&failcnt[n * 4 + 1], 1);
-            flag = utoprim(2, U, G.gcov, G.gcon, C, P.gam, pf);
-            if (flag) atomicAdd(&failcnt[n * 4 + 2], 1);
+#pragma unroll
+        for (int q = 0; q < kFlagsPerThread / 4; q++) {
+            const int g = g0 + q * 4 * (int)blockDim.x;
+            if (f[q].x == kFallbackPending) cells[atomicAdd(&count, 1)] = g;
+            if (f[q].y == kFallbackPending) cells[atomicAdd(&count, 1)] = g + 1;
+            if (f[q].z == kFallbackPending) cells[atomicAdd(&count, 1)] = g + 2;
+            if (f[q].w == kFallbackPending) cells[atomicAdd(&count, 1)] = g + 3;
         }
-        const double *cc = P.colc + B.moff * COLN + col;
-        finish_cell(P, B, n, i, j, g, z, flag, cc[(int64_t)CC_RHOFLR * B.kcol], cc[(int64_t)CC_UFLR * B.kcol], pf, pf_out,
-                    pflag, failcnt);
+        __syncthreads();
+        for (int e = threadIdx.x; e < count; e += blockDim.x) {
+            const int g = cells[e], row = g / B.D[2], z = g - row * B.D[2], i = row / B.D[1], j = row - i * B.D[1];
+            if (i < NG || i >= NG + B.bs[0] || j < NG || j >= NG + B.bs[1] || z < NG || z >= NG + B.bs[2]) continue;
+            const int64_t K = B.ks, col = row, base = NPR * B.off + g;
+            const Geom<double> G = load_geom(P, B, CENT, col);
+            const double *cc = P.colc + B.moff * COLN + col;
+            const int64_t KC = B.kcol;
+            const InvCol C(cc[CC_ALPHA * KC], cc[CC_NCOV * KC], Div<double>(G.g, cc[CC_RG * KC]));
+            double pf[NPR], U[NPR];
+#pragma unroll
+            for (int k = 0; k < NPR; k++) {
+                U[k] = Unew[base + k * K];
+                pf[k] = pf_out[base + k * K];
+            }
+            int flag = utoprim(1, U, G.gcov, G.gcon, C, P.gam, pf);
+            if (flag) {
+                atomicAdd(&failcnt[n * 4 + 1], 1);
+                flag = utoprim(2, U, G.gcov, G.gcon, C, P.gam, pf);
+                if (flag) atomicAdd(&failcnt[n * 4 + 2], 1);
+            }
+            finish_cell(P, B, n, i, j, g, z, flag, cc[CC_RHOFLR * KC], cc[CC_UFLR * KC], pf, pf_out, pflag, failcnt);
+        }
+        __syncthreads();  // the list is no longer read
     }
 }
 
@@ -1278,15 +1302,6 @@ void launch_update_part(const KParams &P, int part, const Launch &L, int full, d
     } else {
         hipLaunchKernelGGL(k_fallback, gdim(L), bdim(L), 0, s, P, L.wl, Unew, pf, pflag, failcnt);
     }
-}
-
-void launch_update(const KParams &P, const Launch &L, int full, double Dt_val, const double *dt_ptr, double dt_mult,
-                   const double *pi, const double *pb, double *pf, double *U0, double *Unew, const double *psf,
-                   const void *F1, const void *F2, const void *F3, int *pflag, int *failcnt, int mixed, hipStream_t s)
-{
-    for (int part : {3, 2})
-        launch_update_part(P, part, L, full, Dt_val, dt_ptr, dt_mult, pi, pb, pf, U0, Unew, psf, F1, F2, F3, pflag,
-                           failcnt, mixed, s);
 }
 
 void launch_cons(const KParams &P, const Launch &L, double Dt, const double *p, double *U0, double *Unew,

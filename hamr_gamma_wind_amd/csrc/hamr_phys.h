@@ -454,19 +454,21 @@ HD double W_of_vsq2(double vsq, double &p, double &rho, double &u, double D, dou
 {
     double gtmp = (1. - vsq);
     rho = D * sqrt(gtmp);
-    p = K * pow(rho, gam);
+    p = K * rpow(rho, gam);
     u = p / (gam - 1.);
     return ((rho + u + p) / gtmp);
 }
 
-// GPU_utoprim_1dvsq2fix1.h general_newton_raphson2 + func_1d_gnr2 + validate_x2
+// GPU_utoprim_1dvsq2fix1.h general_newton_raphson2 + func_1d_gnr2 +
+// validate_x2.  W, p and rho at x[0] are formed once: the iterate an iteration
+// ends with is the one the next begins with.
 HD int gnr_1dvsq2(double *x, const InvPre &s, double K, double gam)
 {
     double dx, x_old, errx = 1., W = 0., W_old = 0., p, rho, u, f = 1., df = 1.;
     int n_iter = 0, i_extra = 0, doing_extra = 0, keep = 1;
+    double Wf = W_of_vsq2(x[0], p, rho, u, s.D, K, gam);
     while (keep) {
-        double Wf, Wsq, dWdvsq, fact_tmp, resid, jac;
-        Wf = W_of_vsq2(x[0], p, rho, u, s.D, K, gam);
+        double Wsq, dWdvsq, fact_tmp, resid, jac;
         Wsq = Wf * Wf;
         dWdvsq = (gam * (2. - gam) * p + (gam - 1.) * rho) / (2. * (gam - 1.) * (1. - x[0]) * (1. - x[0]));
         fact_tmp = (s.Bsq + Wf);
@@ -481,7 +483,7 @@ HD int gnr_1dvsq2(double *x, const InvPre &s, double K, double gam)
         x[0] = (x[0] < -1.e-10) ? (0.5 * x_old) : x[0];
         x[0] = fabs(x[0]);
         W_old = W;
-        W = W_of_vsq2(x[0], p, rho, u, s.D, K, gam);
+        W = Wf = W_of_vsq2(x[0], p, rho, u, s.D, K, gam);
         errx = (W == 0.) ? fabs(W - W_old) : fabs((W - W_old) / W);
         errx += (x[0] == 0.) ? fabs(x[0] - x_old) : fabs((x[0] - x_old) / x[0]);
         if ((fabs(errx) <= kNEWT_TOL) && (doing_extra == 0) && (kEXTRA_NEWT_ITER > 0)) doing_extra = 1;
