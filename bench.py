@@ -65,8 +65,8 @@ def kernel_bytes(kernel, bs, mixed=False):
     b1, b2, b3 = bs
     w = 4 if mixed else 8
     nz = b1 * b2 * b3
-    ghosts = {"bound1": 2 * 3 * (b2 + 6) * (b3 + 6), "bound2": 2 * 3 * (b1 + 6) * (b3 + 6),
-              "bound3": 2 * 3 * (b1 + 6) * (b2 + 6)}
+    # a uniform grid's ghost fill is one kernel, in the bound1 slot
+    ghosts = {"bound1": (b1 + 6) * (b2 + 6) * (b3 + 6) - nz, "bound2": 0, "bound3": 0}
     table = {
         "flux1": 10 * 8 + 9 * w, "flux2": 10 * 8 + 9 * w, "flux3": 10 * 8 + 9 * w,
         "emf_centre": 6 * 8 + 3 * w,        # U1-3, B1-3 read; 3 centre EMFs written

@@ -26,13 +26,15 @@ constexpr int kTiles[3] = {64, 128, 256};   // tile sizes (threads per workgroup
 constexpr int kDefaultTile = 2;
 static_assert(kTiles[kDefaultTile] == kLineT, "line-staged flux tiles use the default tile size");
 
-// Kernels the autotuner configures (each walks the work list of one class).
+// Kernels the autotuner configures (each walks the work list of one class).  A
+// uniform grid's ghost fill is one kernel, in TS_BOUND1; a multi-level set's
+// radial and polar faces are TS_BOUND1 and TS_BOUND2.  TS_BOUND3 has no kernel.
 enum TuneSlot : int {
     TS_FLUX1 = 0, TS_FLUX2, TS_FLUX3, TS_ECENT, TS_ECORNER, TS_CT, TS_CONS, TS_INVERT, TS_FALLBACK,
     TS_BOUND1, TS_BOUND2, TS_BOUND3, TS_EXCHANGE, TS_N
 };
 constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_CORNER, KC_CORNER, KC_INTERIOR,
-                                   KC_INTERIOR, KC_FLAGS, KC_BOUND1, KC_BOUND2, KC_BOUND3, -1};
+                                   KC_INTERIOR, KC_FLAGS, KC_BOUND1, KC_BOUND2, -1, -1};
 
 // Default item order of a class.  In chunks per XCD where tiles share what they
 // read with the next tiles (the stencils of fluxes, EMFs and face update, the
@@ -41,8 +43,8 @@ constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_COR
 // as 42x25x39 blocks), 445 -> 323 (722 blocks); corner EMFs 32 -> 24 us and 155 ->
 // 151, x2 ghosts 236 -> 208, the others 0-7%.  Plain for the interior updates, whose
 // tiles share almost nothing (1.80 -> 1.81 ms, 904 -> 930 us on 722 blocks) and take
-// unequal times, and for the x3 ghost rows (11 -> 19 us on 64x32x32).
-static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_FLAGS || cls == KC_BOUND3 ? 0 : 1; }
+// unequal times.
+static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_FLAGS ? 0 : 1; }
 
 struct TuneCfg {
     int tile = kDefaultTile;  // index into kTiles
@@ -252,8 +254,9 @@ static int build_class_lists(hamr_ctx *c)
 {
     const int nb = nblk_of(c);
     for (int cls = 0; cls < KC_N; cls++) {
-        // block list of the class: every block, except the ghost fill of a
-        // multi-level set, whose kernels serve only the outflow and polar faces
+        // block list of the class: every block, except that the ghost fill of a
+        // multi-level set has its own kernels, which serve only the outflow and
+        // polar faces
         std::vector<int> bl;
         for (int n : c->order) {
             const BlockDev &B = c->blocks[n];
@@ -261,7 +264,9 @@ static int build_class_lists(hamr_ctx *c)
             if (c->amr) {
                 if (cls == KC_BOUND1) use = B.kind[0] == FK_OUTFLOW || B.kind[1] == FK_OUTFLOW;
                 else if (cls == KC_BOUND2) use = B.kind[2] == FK_POLE || B.kind[3] == FK_POLE;
-                else if (cls == KC_BOUND3) use = false;
+                else if (cls == KC_FILL || cls == KC_FILLROWS) use = false;
+            } else if (cls == KC_BOUND1 || cls == KC_BOUND2) {
+                use = false;
             }
             if (use) bl.push_back(n);
         }
@@ -303,15 +308,19 @@ static int build_class_lists(hamr_ctx *c)
 static bool line_flux(const hamr_ctx *c, int slot) { return slot <= TS_FLUX3 && c->tune[slot].alt; }
 static int slot_class(const hamr_ctx *c, int slot)
 {
+    if (slot == TS_BOUND1 && !c->amr) return KC_FILL;
     return line_flux(c, slot) ? KC_LINE1 + slot - TS_FLUX1 : kSlotClass[slot];
 }
 
-// Launch of a tune slot over its whole block list with the tuned configuration.
-static Launch all_launch(const hamr_ctx *c, int slot)
+// Launch of a tune slot over its whole block list (of class cls, when given)
+// with the tuned configuration.
+static Launch all_launch(const hamr_ctx *c, int slot, int cls = -1)
 {
     const TuneCfg &t = c->tune[slot];
-    const ClassList &L = c->cl[slot_class(c, slot)];
-    Launch x;
+    if (cls < 0) cls = slot_class(c, slot);
+    Launch x{};
+    if (cls < 0) return x;  // a slot without a kernel
+    const ClassList &L = c->cl[cls];
     x.line = line_flux(c, slot) ? 1 : 0;
     const int ti = x.line ? kDefaultTile : t.tile;  // line-staged tiles are kLineT threads
     x.threads = kTiles[ti];
@@ -447,7 +456,7 @@ static void pole(hamr_ctx *c, double dt_val, const double *dt_ptr)
     launch_pole(c->P, c->ring, c->rside, c->nring, c->ring_len, c->ni_max, dt_val, dt_ptr, c->E, c->prec, c->s);
 }
 
-// Ghost fill of all blocks.  Uniform grid: x1, x2, x3 stages of k_bound.
+// Ghost fill of all blocks.  Uniform grid: one kernel (k_fill).
 // Multi-level set: outflow faces, exchange stage 1, polar faces, exchange
 // stages 2 and 3, and the final outflow pass over the radial ghosts that the
 // later stages left (see hamr_amr.cpp).
@@ -460,8 +469,7 @@ static void bound_all(hamr_ctx *c, double *p, double *ps, bool x3_rows_done = fa
 {
     const int T = kTiles[c->tune[TS_EXCHANGE].tile], G = c->tune[TS_EXCHANGE].grid;
     if (!c->amr) {
-        for (int dir = 1; dir <= 3; dir++)
-            launch_bound(c->P, dir, all_launch(c, TS_BOUND1 + dir - 1), p, ps, c->pflag, 0, c->s, x3_rows_done ? 1 : 0);
+        launch_fill(c->P, all_launch(c, TS_BOUND1, x3_rows_done ? KC_FILLROWS : KC_FILL), p, ps, c->pflag, c->s);
         return;
     }
     launch_bound(c->P, 1, all_launch(c, TS_BOUND1), p, ps, c->pflag, 0, c->s);
@@ -2076,8 +2084,14 @@ static void run_slot(hamr_ctx *c, int slot, const Launch &L, int T_ex, int G_ex)
                            c->F[1], c->F[2], c->pflag, c->failcnt, c->prec, s);
         break;
     case TS_BOUND1:
-    case TS_BOUND2:
-    case TS_BOUND3: launch_bound(P, slot - TS_BOUND1 + 1, L, c->p, c->ps, c->pflag, 0, s); break;
+        if (!c->amr) {
+            launch_fill(P, L, c->p, c->ps, c->pflag, s);
+            break;
+        }
+        launch_bound(P, 1, L, c->p, c->ps, c->pflag, 0, s);
+        break;
+    case TS_BOUND2: launch_bound(P, 2, L, c->p, c->ps, c->pflag, 0, s); break;
+    case TS_BOUND3: break;
     default:
         for (int st = 0; st < 3; st++)
             launch_amr_exchange(P, st + 1, c->ex[st], c->nex[st], c->pro[st], c->npro[st], c->p, c->ps, c->pflag, T_ex, G_ex, s);
@@ -2138,7 +2152,7 @@ int hamr_autotune(hamr_ctx *c, int nrep)
     static const int grids[4] = {0, 1024, 2048, 4096};
     for (int slot = 0; slot < TS_N; slot++) {
         if (slot == TS_EXCHANGE && !c->amr) continue;
-        if (slot != TS_EXCHANGE && c->cl[kSlotClass[slot]].n[kDefaultTile] == 0) continue;
+        if (slot != TS_EXCHANGE && (slot_class(c, slot) < 0 || c->cl[slot_class(c, slot)].n[kDefaultTile] == 0)) continue;
         TuneCfg best;
         // second forms: the fluxes line-staged, the update k_cons + k_invert
         const int nform = (slot <= TS_FLUX3 || slot == TS_CONS) ? 2 : 1;
@@ -2186,7 +2200,7 @@ int hamr_autotune(hamr_ctx *c, int nrep)
 int hamr_time_kernel(hamr_ctx *c, int slot, int nrep, double *avg_ms)
 {
     if (!c || !avg_ms || nrep < 1 || slot < 0 || slot >= TS_N) return fail(c, "hamr_time_kernel: bad arguments");
-    if (slot == TS_EXCHANGE && !c->amr) {
+    if (slot == TS_BOUND3 || (!c->amr && (slot == TS_EXCHANGE || slot == TS_BOUND2))) {  // no such kernel
         *avg_ms = 0.;
         return 0;
     }

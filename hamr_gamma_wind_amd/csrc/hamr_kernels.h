@@ -113,7 +113,9 @@ enum KClass : int {
     KC_ECENT,                          // cells [NG-1, NG+BS]
     KC_CORNER,                         // corners/faces [NG, NG+BS]   (corner EMF, face-B update)
     KC_INTERIOR,                       // interior cells               (update, inversion, fallback)
-    KC_BOUND1, KC_BOUND2, KC_BOUND3,   // ghost layers of one direction
+    KC_BOUND1, KC_BOUND2,              // ghost layers of one direction (multi-level sets)
+    KC_FILL, KC_FILLROWS,              // ghost cells of a uniform grid's block: all, or without the x3 ghosts
+                                       // inside its x1 and x2 range
     KC_LINE1, KC_LINE2, KC_LINE3,      // line-staged flux tiles of one direction (line_tiles)
     KC_FLAGS,                          // the flag slab, kFlagsPerThread cells per thread (fallback)
     KC_N
@@ -166,15 +168,16 @@ void launch_adjoint(const KParams &P, const BlockDev &B, double Dt, const double
                     const double *F1, const double *F2, const double *F3, const double *w, double *lP, double *lps,
                     double *lpsf, double *lE, double *lEc, double *lF1, double *lF2, double *lF3, hipStream_t s);
 
-// Ghost fill of one direction over the faces whose kind is FK_COPY, FK_OUTFLOW
-// or FK_POLE (FK_AMR faces are left to the exchange tables).  With
-// outflow_only = 1 only radial outflow faces are filled, and not at the ghost
-// rows of a polar face (the final pass of the multi-level fill).
-// With x3_rows_done = 1 the x3 fill skips the rows inside the block's x1 and
-// x2 range whose ghosts the update (k_invert, k_fallback) and face-field
-// (k_ct_update) kernels of the step wrote from the periodic neighbour.
+// Ghost fill of direction dir (1 or 2) of a multi-level set over the faces whose
+// kind is FK_COPY, FK_OUTFLOW or FK_POLE (FK_AMR faces are left to the exchange
+// tables).  With outflow_only = 1 only radial outflow faces are filled, and not
+// at the ghost rows of a polar face (the final pass of the multi-level fill).
 void launch_bound(const KParams &P, int dir, const Launch &L, double *p, double *ps, int *pflag, int outflow_only,
-                  hipStream_t s, int x3_rows_done = 0);
+                  hipStream_t s);
+// Ghost fill of a uniform grid's blocks in one launch.  L: a KC_FILL list, or a
+// KC_FILLROWS list when the update and face-field kernels of the step already
+// wrote the x3 ghosts of the rows inside each block's x1 and x2 range.
+void launch_fill(const KParams &P, const Launch &L, double *p, double *ps, int *pflag, hipStream_t s);
 // Flux correction at level jumps along direction dir (1..3): each entry's
 // coarse face takes the mean of its four finer faces (F: the direction's flux
 // array, FP32 when mixed); dt from dt_ptr if non-null.

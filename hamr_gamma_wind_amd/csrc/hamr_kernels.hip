@@ -28,7 +28,9 @@ int64_t class_work(const BlockDev &B, int cls)
     case KC_FLAGS: return (B.ks + kFlagsPerThread - 1) / kFlagsPerThread;
     case KC_BOUND1: return 2 * NG * d2 * d3;
     case KC_BOUND2: return 2 * NG * d1 * d3;
-    default: return 2 * NG * (d1 * d2 + 1);
+    case KC_FILL: return 2 * NG * (d2 * d3 + b1 * d3 + b1 * (b2 + 1));
+    case KC_FILLROWS: return 2 * NG * (d2 * d3 + b1 * d3);
+    default: return 0;
     }
 }
 
@@ -666,19 +668,14 @@ __global__ void __launch_bounds__(256) k_fallback(KParams P, WorkList wl, const 
     }
 }
 
-// Ghost fill of one direction for the listed blocks: same-level copy, radial
-// outflow with inflow check, or the polar mirror from the pi-shifted partner.
-// Stage order x1, x2, x3, each over the full extent of the others.  Faces of
-// kind FK_AMR are left to the multi-level exchange.
-//
-// Thread mapping: for x1 and x2 the fastest thread index runs along z, so
-// every access of a wavefront is contiguous.  For x3 the ghosts are the first
-// and last NG cells of each z-row; a group of 2*NG consecutive threads writes
-// the upper ghosts of row r-1 and the lower ghosts of row r, which are adjacent
-// in memory, so each group stores one contiguous 48-byte segment.
+// Ghost fill of one direction for the listed blocks of a multi-level set:
+// same-level copy, radial outflow with inflow check, or the polar mirror from the
+// pi-shifted partner, over the full extent of the other directions.  Faces of
+// kind FK_AMR are left to the multi-level exchange.  The fastest thread index
+// runs along z, so every access of a wavefront is contiguous.
 template <int DIR>
 __global__ void __launch_bounds__(256) k_bound(KParams P, WorkList wl, double *p, double *ps, int *pflag,
-                                               int outflow_only, int x3_rows_done)
+                                               int outflow_only)
 {
     FOR_ITEMS(wl)
     {
@@ -687,33 +684,12 @@ __global__ void __launch_bounds__(256) k_bound(KParams P, WorkList wl, double *p
         const BlockDev &B = P.blk[n];
         const int d1 = B.D[0], d2 = B.D[1], d3 = B.D[2];
         const int t = it.y * blockDim.x + threadIdx.x;
-        int aa, bb, gg, side;
-        if (DIR == 3) {
-            const int nrow = d1 * d2;
-            if (t >= 2 * NG * (nrow + 1)) continue;
-            const int g6 = t % (2 * NG), r = t / (2 * NG);
-            side = (g6 < NG) ? 1 : 0;
-            gg = side ? g6 : g6 - NG;
-            const int row = side ? r - 1 : r;
-            if (row < 0 || row >= nrow) continue;
-            aa = row / d2;
-            bb = row % d2;
-        } else {
-            const int ta = (DIR == 1) ? d2 : d1, tb = d3;
-            if (t >= 2 * NG * ta * tb) continue;
-            bb = t % tb;
-            aa = (t / tb) % ta;
-            gg = (t / (tb * ta)) % NG;
-            side = t / (tb * ta * NG);
-        }
+        const int ta = (DIR == 1) ? d2 : d1, tb = d3;
+        if (t >= 2 * NG * ta * tb) continue;
+        const int bb = t % tb, aa = (t / tb) % ta, gg = (t / (tb * ta)) % NG, side = t / (tb * ta * NG);
         const int face = 2 * (DIR - 1) + side;
         const int kind = B.kind[face];
         if (kind == FK_AMR) continue;
-        // rows inside the block's x1 and x2 range whose x3 ghosts the update
-        // and face-field kernels already wrote from the periodic neighbour
-        if (DIR == 3 && x3_rows_done && aa >= NG && aa < NG + B.bs[0] && bb >= NG && bb < NG + B.bs[1] &&
-            x3_row_pushed(P, B, n, face, aa, bb))
-            continue;
         if (outflow_only) {
             if (kind != FK_OUTFLOW) continue;
             // rows beyond a polar face keep the mirror image of the partner's ghosts
@@ -728,8 +704,7 @@ __global__ void __launch_bounds__(256) k_bound(KParams P, WorkList wl, double *p
         else sidx = side ? NG + bsd - 1 - gg : 2 * NG - 1 - gg;
         int i, j, z, is, js, zs;
         if (DIR == 1) { i = gidx; j = aa; z = bb; is = sidx; js = j; zs = z; }
-        else if (DIR == 2) { i = aa; j = gidx; z = bb; is = i; js = sidx; zs = z; }
-        else { i = aa; j = bb; z = gidx; is = i; js = j; zs = sidx; }
+        else { i = aa; j = gidx; z = bb; is = i; js = sidx; zs = z; }
         // a block that is its own pole partner (one block around the axis): shift by half a turn
         if (kind == FK_POLE && src == n) zs = ((z - NG + B.bs[2] / 2) % B.bs[2] + B.bs[2]) % B.bs[2] + NG;
         const BlockDev &S = P.blk[src];
@@ -768,6 +743,132 @@ __global__ void __launch_bounds__(256) k_bound(KParams P, WorkList wl, double *p
             sd[2 * K + cg] = -ssrc[2 * KS + cs];
             if (pflag) pflag[B.off + cg] = pflag[S.off + cs];
         }
+    }
+}
+
+// The whole ghost fill of a uniform grid's block set in one launch: the three
+// stages x1 (copy, or outflow with inflow check), x2 (copy, or the polar mirror)
+// and x3 (copy) composed per ghost cell, last stage first.  Each stage copies a
+// cell of a neighbour's slab that the earlier stages filled; followed back through
+// the stages, every ghost ends at an interior cell of some block (with the inflow
+// check of the radial ghost column it passes, then the mirror's signs), which no
+// thread writes.  The two face-field components that a stage leaves alone (B^1
+// across a radial edge, B^2 across the axis) stop there: their source is the
+// stored, never filled value of that block's ghost, which the later stages copy.
+//
+// Bound by memory: 0.69 GB each way for the rows beside the update's own x3
+// ghosts on 384x192x192.  Along z first, so that the x1 ghost planes and the x2
+// ghost rows are whole runs of memory with their x3 ghosts; the three stages'
+// kernels wrote those in pieces of 24 bytes and passed the corners through
+// memory twice or three times.  All blocks have one shape.
+struct FillSrc {
+    int blk;
+    int i, j, z;
+};
+__global__ void __launch_bounds__(256) k_fill(KParams P, WorkList wl, double *p, double *ps, int *pflag)
+{
+    FOR_ITEMS(wl)
+    {
+        const int2 it = wl_get(wl, w_);
+        const int n = it.x;
+        const BlockDev &B = P.blk[n];
+        const int d2 = B.D[1], d3 = B.D[2], b1 = B.bs[0], b2 = B.bs[1], b3 = B.bs[2];
+        const int nA = 2 * NG * d2 * d3, nB = b1 * 2 * NG * d3, nC = b1 * (b2 + 1) * 2 * NG;
+        int t = it.y * (int)blockDim.x + (int)threadIdx.x;
+        int i, j, z;
+        if (t < nA) {  // x1 ghost planes
+            const int q = t / d3;
+            z = t - q * d3;
+            i = q / d2;
+            j = q - i * d2;
+            if (i >= NG) i += b1;
+        } else if (t < nA + nB) {  // x2 ghost rows
+            t -= nA;
+            const int q = t / d3;
+            z = t - q * d3;
+            i = q / (2 * NG);
+            j = q - i * (2 * NG);
+            i += NG;
+            if (j >= NG) j += b2;
+        } else {  // x3 ghosts of the other rows: the upper of one row and the lower of the next are adjacent
+            t -= nA + nB;
+            if (t >= nC) continue;
+            const int q = t / (2 * NG), g6 = t - q * (2 * NG);
+            i = q / (b2 + 1);
+            const int r = q - i * (b2 + 1);
+            i += NG;
+            if (g6 < NG ? r == 0 : r == b2) continue;
+            j = NG + (g6 < NG ? r - 1 : r);
+            z = g6 < NG ? NG + b3 + g6 : g6 - NG;
+        }
+        // the stages backwards; a: the primitives, the flag and B^3, f1 and f2: B^1 and B^2
+        FillSrc a{n, i, j, z};
+        if (z < NG) {
+            a.blk = B.nbr[4];
+            a.z = z + b3;
+        } else if (z >= NG + b3) {
+            a.blk = B.nbr[5];
+            a.z = z - b3;
+        }
+        FillSrc f2 = a;
+        bool mirror = false;
+        if (j < NG || j >= NG + b2) {
+            const int side = j >= NG, nb = P.blk[a.blk].nbr[2 + side];
+            mirror = P.blk[a.blk].kind[2 + side] == FK_POLE;
+            if (mirror) {
+                a.j = side ? 2 * (NG + b2) - 1 - j : 2 * NG - 1 - j;
+                // a block that is its own pole partner (one block around the axis): shift by half a turn
+                if (nb == a.blk) a.z = (a.z - NG + b3 / 2) % b3 + NG;
+                a.blk = nb;
+            } else {
+                a.j = side ? j - b2 : j + b2;
+                a.blk = nb;
+                f2 = a;
+            }
+        }
+        FillSrc f1 = a;
+        int out = -1;  // the radial edge the cell lies beyond (0 inner, 1 outer)
+        const int cblk = a.blk, cj = a.j;
+        if (i < NG || i >= NG + b1) {
+            const int side = i >= NG;
+            if (P.blk[a.blk].kind[side] == FK_OUTFLOW) {
+                out = side;
+                a.i = f2.i = side ? NG + b1 - 1 : NG;
+            } else {
+                a.i = f2.i = side ? i - b1 : i + b1;
+                a.blk = P.blk[a.blk].nbr[side];
+                f2.blk = P.blk[f2.blk].nbr[side];
+                f1 = a;
+            }
+        }
+        auto cell = [&](const FillSrc &s) { return (s.i * d2 + s.j) * d3 + s.z; };
+        const int64_t K = B.ks, oa = P.blk[a.blk].off, o1 = P.blk[f1.blk].off, o2 = P.blk[f2.blk].off;
+        const int cg = (i * d2 + j) * d3 + z, ca = cell(a), c1 = cell(f1), c2 = cell(f2);
+        double pr[NPR];
+#pragma unroll
+        for (int k = 0; k < NPR; k++) pr[k] = p[NPR * oa + k * K + ca];
+        const double s1 = ps[3 * o1 + c1], s2 = ps[3 * o2 + K + c2];
+        double s3 = ps[3 * oa + 2 * K + ca];
+        const int fl = pflag ? pflag[oa + ca] : 0;
+        if (out >= 0) {
+            const Geom<double> G = load_geom(P, P.blk[cblk], CENT, (int64_t)i * d2 + cj);
+            inflow_check(pr, G, out);
+        }
+        if (mirror) {
+            pr[U2] *= -1.0;
+            pr[U3] *= -1.0;
+            pr[B2] *= -1.0;
+            pr[B3] *= -1.0;
+            s3 = -s3;
+        }
+#pragma unroll
+        for (int k = 0; k < NPR; k++) p[NPR * B.off + k * K + cg] = pr[k];
+        double *sd = ps + 3 * B.off;
+        // (a component that no stage fills is its own source)
+        if (o1 != B.off || c1 != cg) sd[cg] = s1;
+        if (o2 != B.off || c2 != cg) sd[K + cg] = s2;
+        sd[2 * K + cg] = s3;
+        if (pflag) pflag[B.off + cg] = fl;
     }
 }
 
@@ -1312,12 +1413,17 @@ void launch_cons(const KParams &P, const Launch &L, double Dt, const double *p, 
 }
 
 void launch_bound(const KParams &P, int dir, const Launch &L, double *p, double *ps, int *pflag, int outflow_only,
-                  hipStream_t s, int x3_rows_done)
+                  hipStream_t s)
 {
     if (L.wl.n <= 0) return;
-    if (dir == 1) hipLaunchKernelGGL(k_bound<1>, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag, outflow_only, 0);
-    else if (dir == 2) hipLaunchKernelGGL(k_bound<2>, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag, outflow_only, 0);
-    else hipLaunchKernelGGL(k_bound<3>, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag, outflow_only, x3_rows_done);
+    if (dir == 1) hipLaunchKernelGGL(k_bound<1>, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag, outflow_only);
+    else hipLaunchKernelGGL(k_bound<2>, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag, outflow_only);
+}
+
+void launch_fill(const KParams &P, const Launch &L, double *p, double *ps, int *pflag, hipStream_t s)
+{
+    if (L.wl.n <= 0) return;
+    hipLaunchKernelGGL(k_fill, gdim(L), bdim(L), 0, s, P, L.wl, p, ps, pflag);
 }
 
 void launch_amr_exchange(const KParams &P, int dir, const AmrEntry *e, int64_t n, const AmrProlong *pe, int64_t npro,

@@ -157,23 +157,6 @@ __device__ __forceinline__ bool x3_push_target(const KParams &P, const BlockDev 
     return true;
 }
 
-// Whether the x3 ghosts of row (i, j) of block n (inside its x1 and x2 range)
-// beyond face f (4: lower, 5: upper) are written by the update of the copy
-// neighbour across f (its push table names n for that row's tile).
-__device__ __forceinline__ bool x3_row_pushed(const KParams &P, const BlockDev &B, int n, int f, int i, int j)
-{
-    const int s = B.nbr[f];
-    if (P.las_s >= 0 || s < 0) return false;
-    const BlockDev &S = P.blk[s];
-    const int row = S.push3[f == 4 ? 1 : 0];
-    if (row < 0) return false;
-    const int is = i + B.o[0] - S.o[0], js = j + B.o[1] - S.o[1];
-    if (is < NG || is >= NG + S.bs[0] || js < NG || js >= NG + S.bs[1]) return false;
-    if (row & kPushWhole) return P.push3[row & ~kPushWhole].m == n;
-    const int t2n = (S.bs[1] + kPushTile - 1) / kPushTile;
-    return P.push3[row + ((is - NG) / kPushTile) * t2n + (js - NG) / kPushTile].m == n;
-}
-
 // launch geometry of a work-list launch
 static inline dim3 gdim(const Launch &L) { return dim3((unsigned)L.grid); }
 static inline dim3 bdim(const Launch &L) { return dim3((unsigned)L.threads); }

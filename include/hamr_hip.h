@@ -408,7 +408,10 @@ int hamr_tune_get(const hamr_ctx *ctx, int slot, int *cfg, double *ms);
 int hamr_tune_set(hamr_ctx *ctx, int slot, const int *cfg);
 /* Average device time (ms, HIP events on the context stream) of one launch of
  * kernel `slot` over all blocks with its tuned shape and predictor-step
- * operands (HAMR_TUNE_EXCHANGE: the three exchange stages of a multi-level set).
+ * operands (HAMR_TUNE_EXCHANGE: the three exchange stages of a multi-level set;
+ * HAMR_TUNE_BOUND1: the whole ghost fill of a uniform grid, or the radial faces of
+ * a multi-level set, whose polar faces are HAMR_TUNE_BOUND2; 0 for a slot that the
+ * set has no kernel for).
  * Like hamr_autotune it keeps p/ps, the flags and the failure counters of the
  * last step, and leaves p/ps and ph/psh with their ghosts filled; the
  * intermediate arrays (fluxes, EMFs, U0, Un, ph, psh) hold the timed launches'
