@@ -73,8 +73,9 @@ template <class R> HD void vchar_ft(const R *pr, const R *ucon, const R *bcon, i
     if ((discr < R(0.0)) && (discr > R(-1.e-10))) discr = R(0.0);
     else if (discr < R(-1.e-10)) discr = R(0.);
     discr = sqrt(discr);
-    const R vp = dv(-(-B + discr), R(2.) * A);
-    const R vm = dv(-(-B - discr), R(2.) * A);
+    const Div<R> by_2A(R(2.) * A);
+    const R vp = by_2A(-(-B + discr));
+    const R vm = by_2A(-(-B - discr));
     if (vp > vm) { *vmax = vp; *vmin = vm; }
     else { *vmax = vm; *vmin = vp; }
 }
@@ -132,13 +133,14 @@ HD void hllc_hydro(const FtFace<R> &f, R int_velocity, R cmin_roe, R cmax_roe, R
     const R ptot = -(-H[1][UU]) * vcon + H[1][Y::U_1];
     const bool fail = !(fabs(ptot) > R(0.)) || (vcon < cmin_roe) || (vcon > cmax_roe) || !(fabs(vcon) > R(0.));
     if (cmax_roe > int_velocity && vcon <= int_velocity && !fail) {
-        const R s = dv(cmax_roe - dv(f.rud, f.ru0), cmax_roe - vcon + R(kSMALL));
+        const Div<R> by_den(cmax_roe - vcon + R(kSMALL));
+        const R s = by_den(cmax_roe - dv(f.rud, f.ru0));
         FT[0][RHO] = s * f.U_r[RHO];
         if constexpr (TAU) {
-            FT[0][UU] = dv(cmax_roe * f.U_r[UU] + f.smd_r - ptot * vcon, cmax_roe - vcon + R(kSMALL));
+            FT[0][UU] = by_den(cmax_roe * f.U_r[UU] + f.smd_r - ptot * vcon);
             FT[0][Y::U_1] = (-(FT[0][UU] - FT[0][RHO]) + ptot) * vcon;
         } else {
-            FT[0][UU] = dv(cmax_roe * f.U_r[UU] + f.U_r[Y::U_1] - ptot * vcon, cmax_roe - vcon + R(kSMALL));
+            FT[0][UU] = by_den(cmax_roe * f.U_r[UU] + f.U_r[Y::U_1] - ptot * vcon);
             FT[0][Y::U_1] = (-FT[0][UU] + ptot) * vcon;
         }
         FT[0][Y::U_2] = s * f.U_r[Y::U_2];
@@ -149,13 +151,14 @@ HD void hllc_hydro(const FtFace<R> &f, R int_velocity, R cmin_roe, R cmax_roe, R
         FT[0][KTOT] = s * f.U_r[KTOT];
         for (int k = 0; k < NPR; k++) FT[1][k] = (f.F_r[k] + cmax_roe * (FT[0][k] - f.U_r[k]));
     } else if (cmin_roe < int_velocity && vcon >= int_velocity && !fail) {
-        const R s = dv(cmin_roe - dv(f.lud, f.lu0), cmin_roe - vcon + R(kSMALL));
+        const Div<R> by_den(cmin_roe - vcon + R(kSMALL));
+        const R s = by_den(cmin_roe - dv(f.lud, f.lu0));
         FT[0][RHO] = s * f.U_l[RHO];
         if constexpr (TAU) {
-            FT[0][UU] = dv(cmin_roe * f.U_l[UU] + f.smd_l - ptot * vcon, cmin_roe - vcon + R(kSMALL));
+            FT[0][UU] = by_den(cmin_roe * f.U_l[UU] + f.smd_l - ptot * vcon);
             FT[0][Y::U_1] = (-(FT[0][UU] - FT[0][RHO]) + ptot) * vcon;
         } else {
-            FT[0][UU] = dv(cmin_roe * f.U_l[UU] + f.U_l[Y::U_1] - ptot * vcon, cmin_roe - vcon + R(kSMALL));
+            FT[0][UU] = by_den(cmin_roe * f.U_l[UU] + f.U_l[Y::U_1] - ptot * vcon);
             FT[0][Y::U_1] = (-FT[0][UU] + ptot) * vcon;
         }
         FT[0][Y::U_2] = s * f.U_l[Y::U_2];
@@ -197,51 +200,55 @@ HD void hllc_mhd(const FtFace<R> &f, R int_velocity, R cmin_roe, R cmax_roe, R (
     const R D = B * B - R(4.) * A * C;
     vcon[0] = R(0.);
     vcon[Y::g1] = TAU ? dv(R(2.) * C, -B + R(sqrt(D))) : dv(-B - R(sqrt(D)), R(2.) * A);
-    vcon[Y::g2] = dv(H[0][Y::B_2] * vcon[Y::g1] - H[1][Y::B_2], H[0][Y::B_1]);
-    vcon[Y::g3] = dv(H[0][Y::B_3] * vcon[Y::g1] - H[1][Y::B_3], H[0][Y::B_1]);
+    const Div<R> by_Bn(H[0][Y::B_1]);
+    vcon[Y::g2] = by_Bn(H[0][Y::B_2] * vcon[Y::g1] - H[1][Y::B_2]);
+    vcon[Y::g3] = by_Bn(H[0][Y::B_3] * vcon[Y::g1] - H[1][Y::B_3]);
     const R gammasq = dv(R(1.), R(1.) - (vcon[1] * vcon[1] + vcon[2] * vcon[2] + vcon[3] * vcon[3]));
+    const Div<R> by_gsq(gammasq);
     const R v_dot_B = (vcon[1] * H[0][B1] + vcon[2] * H[0][B2] + vcon[3] * H[0][B3]);
     const R ptot = -(-H[1][UU] - H[0][Y::B_1] * (v_dot_B)) * vcon[DIR] + H[1][Y::U_1]
-        + dv(H[0][Y::B_1] * H[0][Y::B_1], gammasq);
+        + by_gsq(H[0][Y::B_1] * H[0][Y::B_1]);
     const R vn = vcon[DIR];
     const bool fail = !(fabs(ptot) > R(0.)) || (vn < cmin_roe) || (vn > cmax_roe) || !(fabs(vn) > R(0.));
     if (cmax_roe > int_velocity && vn <= int_velocity && !fail) {
-        const R den = cmax_roe - vn + R(kSMALL);
-        FT[0][RHO] = dv(cmax_roe - dv(f.rud, f.ru0), den) * f.U_r[RHO];
+        const Div<R> by_den(cmax_roe - vn + R(kSMALL));
+        const R s = by_den(cmax_roe - dv(f.rud, f.ru0));
+        FT[0][RHO] = s * f.U_r[RHO];
         if constexpr (TAU) {
-            FT[0][UU] = dv(cmax_roe * f.U_r[UU] + f.smd_r - ptot * vn + v_dot_B * H[0][Y::B_1], den);
+            FT[0][UU] = by_den(cmax_roe * f.U_r[UU] + f.smd_r - ptot * vn + v_dot_B * H[0][Y::B_1]);
             FT[0][Y::U_1] = (-(FT[0][UU] - FT[0][RHO]) + ptot) * vn - v_dot_B * H[0][Y::B_1];
         } else {
-            FT[0][UU] = dv(cmax_roe * f.U_r[UU] + f.U_r[Y::U_1] - ptot * vn + v_dot_B * H[0][Y::B_1], den);
+            FT[0][UU] = by_den(cmax_roe * f.U_r[UU] + f.U_r[Y::U_1] - ptot * vn + v_dot_B * H[0][Y::B_1]);
             FT[0][Y::U_1] = (-FT[0][UU] + ptot) * vn - v_dot_B * H[0][Y::B_1];
         }
-        FT[0][Y::U_2] = dv(-H[0][Y::B_1] * (dv(H[0][Y::B_2], gammasq) + v_dot_B * vcon[Y::g2])
-                               + cmax_roe * f.U_r[Y::U_2] - f.F_r[Y::U_2], den);
-        FT[0][Y::U_3] = dv(-H[0][Y::B_1] * (dv(H[0][Y::B_3], gammasq) + v_dot_B * vcon[Y::g3])
-                               + cmax_roe * f.U_r[Y::U_3] - f.F_r[Y::U_3], den);
+        FT[0][Y::U_2] = by_den(-H[0][Y::B_1] * (by_gsq(H[0][Y::B_2]) + v_dot_B * vcon[Y::g2])
+                               + cmax_roe * f.U_r[Y::U_2] - f.F_r[Y::U_2]);
+        FT[0][Y::U_3] = by_den(-H[0][Y::B_1] * (by_gsq(H[0][Y::B_3]) + v_dot_B * vcon[Y::g3])
+                               + cmax_roe * f.U_r[Y::U_3] - f.F_r[Y::U_3]);
         FT[0][Y::B_1] = H[0][Y::B_1];
         FT[0][Y::B_2] = H[0][Y::B_2];
         FT[0][Y::B_3] = H[0][Y::B_3];
-        FT[0][KTOT] = dv(cmax_roe - dv(f.rud, f.ru0), den) * f.U_r[KTOT];
+        FT[0][KTOT] = s * f.U_r[KTOT];
         for (int k = 0; k < NPR; k++) FT[1][k] = (f.F_r[k] + cmax_roe * (FT[0][k] - f.U_r[k]));
     } else if (cmin_roe < int_velocity && vn >= int_velocity && !fail) {
-        const R den = cmin_roe - vn + R(kSMALL);
-        FT[0][RHO] = dv(cmin_roe - dv(f.lud, f.lu0), den) * f.U_l[RHO];
+        const Div<R> by_den(cmin_roe - vn + R(kSMALL));
+        const R s = by_den(cmin_roe - dv(f.lud, f.lu0));
+        FT[0][RHO] = s * f.U_l[RHO];
         if constexpr (TAU) {
-            FT[0][UU] = dv(cmin_roe * f.U_l[UU] + f.smd_l - ptot * vn + v_dot_B * H[0][Y::B_1], den);
+            FT[0][UU] = by_den(cmin_roe * f.U_l[UU] + f.smd_l - ptot * vn + v_dot_B * H[0][Y::B_1]);
             FT[0][Y::U_1] = (-(FT[0][UU] - FT[0][RHO]) + ptot) * vn - v_dot_B * H[0][Y::B_1];
         } else {
-            FT[0][UU] = dv(cmin_roe * f.U_l[UU] + f.U_l[Y::U_1] - ptot * vn + v_dot_B * H[0][Y::B_1], den);
+            FT[0][UU] = by_den(cmin_roe * f.U_l[UU] + f.U_l[Y::U_1] - ptot * vn + v_dot_B * H[0][Y::B_1]);
             FT[0][Y::U_1] = (-FT[0][UU] + ptot) * vn - v_dot_B * H[0][Y::B_1];
         }
-        FT[0][Y::U_2] = dv(-H[0][Y::B_1] * (dv(H[0][Y::B_2], gammasq) + v_dot_B * vcon[Y::g2])
-                               + cmin_roe * f.U_l[Y::U_2] - f.F_l[Y::U_2], den);
-        FT[0][Y::U_3] = dv(-H[0][Y::B_1] * (dv(H[0][Y::B_3], gammasq) + v_dot_B * vcon[Y::g3])
-                               + cmin_roe * f.U_l[Y::U_3] - f.F_l[Y::U_3], den);
+        FT[0][Y::U_2] = by_den(-H[0][Y::B_1] * (by_gsq(H[0][Y::B_2]) + v_dot_B * vcon[Y::g2])
+                               + cmin_roe * f.U_l[Y::U_2] - f.F_l[Y::U_2]);
+        FT[0][Y::U_3] = by_den(-H[0][Y::B_1] * (by_gsq(H[0][Y::B_3]) + v_dot_B * vcon[Y::g3])
+                               + cmin_roe * f.U_l[Y::U_3] - f.F_l[Y::U_3]);
         FT[0][Y::B_1] = H[0][Y::B_1];
         FT[0][Y::B_2] = H[0][Y::B_2];
         FT[0][Y::B_3] = H[0][Y::B_3];
-        FT[0][KTOT] = dv(cmin_roe - dv(f.lud, f.lu0), den) * f.U_l[KTOT];
+        FT[0][KTOT] = s * f.U_l[KTOT];
         for (int k = 0; k < NPR; k++) FT[1][k] = (f.F_l[k] + cmin_roe * (FT[0][k] - f.U_l[k]));
     } else {
         for (int k = 0; k < NPR; k++) {
@@ -301,12 +308,11 @@ HD void hllc_frame_flux(const R *pl, const R *pr, const R *ucl, const R *bcl, co
         for (int k = 0; k < NPR; k++) FT[0][k] = f.U_l[k];
         for (int k = 0; k < NPR; k++) FT[1][k] = f.F_l[k];
     } else {
+        const Div<R> by_c(cmax_roe - cmin_roe + R(kSMALL));
         for (int k = 0; k < NPR; k++)
-            f.HLL[0][k] = dv(f.F_l[k] - f.F_r[k] + cmax_roe * f.U_r[k] - cmin_roe * f.U_l[k],
-                             cmax_roe - cmin_roe + R(kSMALL));
+            f.HLL[0][k] = by_c(f.F_l[k] - f.F_r[k] + cmax_roe * f.U_r[k] - cmin_roe * f.U_l[k]);
         for (int k = 0; k < NPR; k++)
-            f.HLL[1][k] = dv(cmax_roe * f.F_l[k] - cmin_roe * f.F_r[k] + cmax_roe * cmin_roe * (f.U_r[k] - f.U_l[k]),
-                             cmax_roe - cmin_roe + R(kSMALL));
+            f.HLL[1][k] = by_c(cmax_roe * f.F_l[k] - cmin_roe * f.F_r[k] + cmax_roe * cmin_roe * (f.U_r[k] - f.U_l[k]));
         const R bn = f.HLL[0][DIR + B1 - 1];
         const R e0 = TAU ? f.HLL[0][UU] - f.HLL[0][RHO] : f.HLL[0][UU];  // the total energy
         const bool do_hydro = (fabs(bn * bn * l_ucon[0] * r_ucon[0]) < R(1.e-10) * fabs(e0));

@@ -40,35 +40,6 @@ __device__ __forceinline__ int2 wl_get(const WorkList &wl, int w)
 __device__ __forceinline__ int64_t mg10(const BlockDev &B, int pos, int s) { return B.moff * (NPOS * 10) + ((int64_t)pos * 10 + s) * B.kcol; }
 __device__ __forceinline__ int64_t mg1(const BlockDev &B, int pos) { return B.moff * NPOS + (int64_t)pos * B.kcol; }
 
-// Metric at one position of one column in the arithmetic R: the FP64 metric,
-// or for R = float its FP32 copy (the FP64 values rounded, and 1 - alpha
-// formed in FP64 and rounded, by k_geom32 when the metric was uploaded).
-template <class R = double>
-__device__ __forceinline__ Geom<R> load_geom(const KParams &P, const BlockDev &B, int pos, int64_t col)
-{
-    Geom<R> G;
-    if constexpr (sizeof(R) == 4) {
-        const float *g = P.g32 + B.moff * (NPOS * G32N) + (int64_t)pos * G32N * B.kcol + col;
-#pragma unroll
-        for (int s = 0; s < 10; s++) {
-            G.gcov[s] = g[s * B.kcol];
-            G.gcon[s] = g[(10 + s) * B.kcol];
-        }
-        G.g = g[20 * B.kcol];
-        G.oma = g[21 * B.kcol];
-    } else {
-        const double *gc = P.gcov + mg10(B, pos, 0) + col;
-        const double *gi = P.gcon + mg10(B, pos, 0) + col;
-#pragma unroll
-        for (int s = 0; s < 10; s++) {
-            G.gcov[s] = gc[s * B.kcol];
-            G.gcon[s] = gi[s * B.kcol];
-        }
-        G.g = P.gdet[mg1(B, pos) + col];
-    }
-    return G;
-}
-
 // Element g of a slab whose base is the same for the whole wavefront: the base
 // stays in scalar registers and g is a 32-bit offset, so that an access takes no
 // 64-bit vector address arithmetic (a slab holds fewer than 2^29 cells: the
@@ -80,6 +51,34 @@ template <class T> __device__ __forceinline__ T gld(const T *base, uint32_t g)
 template <class T> __device__ __forceinline__ void gst(T *base, uint32_t g, T v)
 {
     *(T *)((char *)base + (uint32_t)(g * (uint32_t)sizeof(T))) = v;
+}
+
+// Metric at one position of one column in the arithmetic R: the FP64 metric,
+// or for R = float its FP32 copy (the FP64 values rounded, and 1 - alpha
+// formed in FP64 and rounded, by k_geom32 when the metric was uploaded).
+template <class R = double>
+__device__ __forceinline__ Geom<R> load_geom(const KParams &P, const BlockDev &B, int pos, int64_t col)
+{
+    Geom<R> G;
+    if constexpr (sizeof(R) == 4) {
+        const float *g = P.g32 + B.moff * (NPOS * G32N) + (int64_t)pos * G32N * B.kcol;
+#pragma unroll
+        for (int s = 0; s < 10; s++) {
+            G.gcov[s] = gld(g + s * B.kcol, (uint32_t)col);
+            G.gcon[s] = gld(g + (10 + s) * B.kcol, (uint32_t)col);
+        }
+        G.g = gld(g + 20 * B.kcol, (uint32_t)col);
+        G.oma = gld(g + 21 * B.kcol, (uint32_t)col);
+    } else {
+        const double *gc = P.gcov + mg10(B, pos, 0), *gi = P.gcon + mg10(B, pos, 0);
+#pragma unroll
+        for (int s = 0; s < 10; s++) {
+            G.gcov[s] = gld(gc + s * B.kcol, (uint32_t)col);
+            G.gcon[s] = gld(gi + s * B.kcol, (uint32_t)col);
+        }
+        G.g = gld(P.gdet + mg1(B, pos), (uint32_t)col);
+    }
+    return G;
 }
 
 // The step Dt of block B: the launch's Dt (dt_ptr[0] dt_mult when the launch

@@ -25,23 +25,21 @@ namespace hamr {
 
 // HLL flux through face `cell` (cell index of the face's upper cell; (i, j) its
 // metric column) from the reconstructed states pl (lower side) and pr (upper
-// side), fluxcalc2D2's flux and speed part (GPU_program1.cu:811-1045).  Stores
-// the 9 fluxes and returns the face's Courant dt, or 1e9 where it is not a
+// side), fluxcalc2D2's flux and speed part (GPU_program1.cu:811-1045).  G: the
+// metric at the face, bn: the face's normal field.  Stores the 9 fluxes and returns the face's Courant dt, or 1e9 where it is not a
 // valid bound (no signal speed).
 template <int DIR, class R>
 __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
-                                           R *pr, int i, int j, int64_t cell, R *__restrict__ F)
+                                           R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
+                                           const R bn)
 {
     const int64_t K = B.ks;
-    const R bn = (R)ps[3 * B.off + (DIR - 1) * K + cell];
     pl[B1 + DIR - 1] = bn;
     pr[B1 + DIR - 1] = bn;
     if (DIR == 2 && (((B.pole & 1) && j == NG) || ((B.pole & 2) && j == NG + B.bs[1]))) {
         pl[B1] = R(0.);
         pr[B1] = R(0.);
     }
-    const int64_t col = (int64_t)i * B.D[1] + j;
-    const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, col);
     const R gam = (R)P.gam;
     R t1[NPR], t2[NPR], t3[NPR], t4[NPR], cmax_l = R(0.), cmin_l = R(0.), cmax_r = R(0.), cmin_r = R(0.), dum;
     State<R> q;
@@ -54,11 +52,11 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
     const R cmax = fabs(mymax(mymax(R(0.), cmax_l), cmax_r));
     const R cmin = fabs(mymax(mymax(R(0.), -cmin_l), -cmin_r));
     const R ctop = mymax(cmax, cmin);
-    R *Fb = F + NPR * B.off + cell;
+    R *Fb = F + NPR * B.off;
     const Div<R> by_c(cmax + cmin + R(kSMALL));
 #pragma unroll
     for (int k = 0; k < NPR; k++)
-        Fb[(int64_t)k * K] = by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]));
+        gst(Fb + (int64_t)k * K, (uint32_t)cell, by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k])));
     const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
     return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
 }
@@ -68,10 +66,10 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
 // orthonormal-frame solver of hamr_hllc.h with the face's tetrad.
 template <int DIR, class R>
 __device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
-                                            R *pr, int i, int j, int64_t cell, R *__restrict__ F)
+                                            R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
+                                            const R bn)
 {
     const int64_t K = B.ks;
-    const R bn = (R)ps[3 * B.off + (DIR - 1) * K + cell];
     pl[B1 + DIR - 1] = bn;
     pr[B1 + DIR - 1] = bn;
     if (DIR == 2 && (((B.pole & 1) && j == NG) || ((B.pole & 2) && j == NG + B.bs[1]))) {
@@ -79,7 +77,6 @@ __device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B,
         pr[B1] = R(0.);
     }
     const int64_t col = (int64_t)i * B.D[1] + j;
-    const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, col);
     const R gam = (R)P.gam;
     State<R> ql, qr;
     get_state(pl, G, ql);
@@ -113,12 +110,21 @@ __device__ __forceinline__ void dt_reduce(double vdt, unsigned long long *__rest
     if ((threadIdx.x & 63) == 0 && vdt < 1.e9) atomicMin(&dtmin[slot], (unsigned long long)__double_as_longlong(vdt));
 }
 
-// One thread per face: both parabolas of the face's two cells.  At least 3
-// waves per SIMD (<= 168 VGPRs): the FP64 flux needs 169 registers
-// unconstrained (the FP32 flux needs 96, five waves).  A variant that marches
-// each thread through a segment of faces along x1 or x2 and forms each cell's
-// parabola once issues 29% fewer FP32 VALU instructions per face, but its
-// carried state takes 157 registers (three waves) and it ran 7-35% slower.
+// One thread per face: both parabolas of the face's two cells.
+//
+// Bound by the VALU (FP32: 1.55e3 instructions per face, x3 fluxes at 97% of the
+// issue rate; FP64: 1.98e3) and, beside it, by the latency of the stencil loads:
+// the limiter's branches keep the compiler from moving a load above the previous
+// variable's parabola, so that the 7 variables' loads waited one after another.
+// With all 42 issued first and the metric's 21 in the middle: x1, x2, x3 fluxes
+// 418, 435, 400 -> 339, 346, 320 us (FP64, 256x128x128), 818, 855, 690 -> 768, 727,
+// 594 us (mixed, 384x192x192).  At least 3 waves per SIMD (FP64: 162 VGPRs; FP32
+// 92-104, four or five waves); held at four in FP64, or at five or six in FP32,
+// they spill and run 8-25% slower.  Without the limiter's branches (selects) the
+// loads are hoisted too far: spills, 15% slower.  A variant that marches each
+// thread through a segment of faces along x1 or x2 and forms each cell's parabola
+// once issues 29% fewer FP32 VALU instructions per face, but its carried state
+// takes 157 registers (three waves) and it ran 7-35% slower.
 // RS selects the Riemann solver: 0 HLL, 1 HLLC.  The FP64 HLLC kernel is held
 // at two waves per SIMD: 256 VGPRs with about 20 spilled to scratch ran 1.4x
 // faster than one wave with none spilled.  The FP32 HLLC kernel at four waves
@@ -147,20 +153,34 @@ k_flux(KParams P, WorkList wl, const double *__restrict__ p, const double *__res
             const int64_t sd = (DIR == 1) ? (int64_t)B.D[1] * B.D[2] : (DIR == 2) ? (int64_t)B.D[2] : 1;
             const double *pb = p + NPR * B.off;
             R pl[NPR], pr[NPR];
+            // every stencil value first, then the parabolas (KTOT enters no flux)
+            double y[KTOT][6];
 #pragma unroll
-            for (int k = 0; k < NPR; k++) {
-                if (k == B1 + DIR - 1) continue;  // the face-normal field comes from ps
-                const double *q = pb + (int64_t)k * K + cell;
-                const R ym3 = (R)q[-3 * sd], ym2 = (R)q[-2 * sd], ym1 = (R)q[-sd], y0 = (R)q[0], yp1 = (R)q[sd],
-                        yp2 = (R)q[2 * sd];
+            for (int k = 0; k < KTOT; k++) {
+                if (k == B1 + DIR - 1) continue;
+                const double *q = pb + (int64_t)k * K;
+#pragma unroll
+                for (int m = 0; m < 6; m++) y[k][m] = gld(q + (m - 3) * sd, (uint32_t)cell);
+            }
+            auto one = [&](int k) {
+                if (k == B1 + DIR - 1) return;  // the face-normal field comes from ps
+                const R ym3 = (R)y[k][0], ym2 = (R)y[k][1], ym1 = (R)y[k][2], y0 = (R)y[k][3], yp1 = (R)y[k][4],
+                        yp2 = (R)y[k][5];
                 R l, r;
                 para(ym3, ym2, ym1, y0, yp1, l, r);
                 pl[k] = r;
                 para(ym2, ym1, y0, yp1, yp2, l, r);
                 pr[k] = l;
-            }
-            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F);
-            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F);
+            };
+#pragma unroll
+            for (int k = 0; k < 4; k++) one(k);
+            // the metric while the rest is reconstructed, in the registers the first stencils left
+            const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
+            const R bn = (R)gld(ps + 3 * B.off + (DIR - 1) * K, (uint32_t)cell);
+#pragma unroll
+            for (int k = 4; k < KTOT; k++) one(k);
+            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
         }
         if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
     }
@@ -285,8 +305,10 @@ k_flux_lines(KParams P, WorkList wl, const double *__restrict__ p, const double 
         else line_tile_states<DIR, R, 0>(B, it.y, p, sm, pl, pr, fact, cell, i, j);
         double vdt = 1.e9;
         if (fact) {
-            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F);
-            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F);
+            const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
+            const R bn = (R)ps[3 * B.off + (DIR - 1) * (int64_t)B.ks + cell];
+            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
         }
         if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
         // the next item's first barrier orders its LDS writes after these reads
