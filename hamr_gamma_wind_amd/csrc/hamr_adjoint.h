@@ -1,9 +1,9 @@
 // hamr_adjoint.h -- hand-written reverse-mode derivatives of the pointwise
 // physics of one forward stage (FP64): the MHD state and fluxes of a
 // reconstructed face state, the HLL combination, the cell-centre EMF, and the
-// forward-mode Jacobian of the PPM reconstruction through the limiter's active
-// branch.  Every function recomputes the primal quantities it needs from its
-// inputs (nothing of the forward pass is stored).
+// PPM reconstruction through the limiter's active branch.  Every function
+// recomputes the primal quantities it needs from its inputs (nothing of the
+// forward pass is stored).
 //
 // Conventions follow hamr_phys.h: prims RHO, UU, U1-U3 (relative 4-velocity),
 // B1-B3, KTOT; packed symmetric metric; fluxes and conserved variables times
@@ -150,120 +150,182 @@ HD void para_jacobian(const double *x, double *l, double *r, double *Jl, double 
     }
 }
 
+// mc_slope(ym, y0, yp) with the choice it makes: the slope is 2 (y0 - ym), 2 (yp -
+// y0) or (yp - ym) / 2 itself, as the three agree in sign where it is not zero.
+struct SlopeChoice {
+    double dq;
+    bool on, centred, upper;
+    HD SlopeChoice(double ym, double y0, double yp)
+    {
+        const double Dqm = 2. * (y0 - ym), Dqp = 2. * (yp - y0), Dqc = 0.5 * (yp - ym);
+        on = Dqm * Dqp > 0.;
+        upper = fabs(Dqp) < fabs(Dqm);
+        const double one_sided = upper ? Dqp : Dqm;
+        centred = !(fabs(one_sided) < fabs(Dqc));
+        dq = on ? (centred ? Dqc : one_sided) : 0.;
+    }
+    // adds lam d(dq)/d(ym, y0, yp) to v[0..2]
+    HD void vjp(double lam, double *v) const
+    {
+        const double h = on ? (centred ? 0.5 : 2.) * lam : 0.;
+        const double lo = !centred && upper ? 0. : h, hi = centred || upper ? h : 0.;
+        v[0] -= lo;
+        v[1] += lo - hi;
+        v[2] += hi;
+    }
+};
+
+// Reverse of para for one cell: adds lam_l dl/dx + lam_r dr/dx to v[0..4], along
+// the branches para_jacobian takes.
+HD void para_vjp(const double *x, double ll, double lr, double *v)
+{
+    const SlopeChoice s0(x[0], x[1], x[2]), s1(x[1], x[2], x[3]), s2(x[2], x[3], x[4]);
+    const double x3 = x[2];
+    const double lo = ppm_face(x[1], x3, s0.dq, s1.dq), hi = ppm_face(x3, x[3], s1.dq, s2.dq);
+    const double qa = (hi - x3) * (x3 - lo), qd = hi - lo, qe = 6.0 * (x3 - 0.5 * (lo + hi));
+    const bool low = qd * (qd - qe) < 0., high = !low && qd * (qd + qe) < 0., flat = qa <= 0.;
+    // low: l = 3 x3 - 2 r, high: r = 3 x3 - 2 l
+    const double fl = low ? 0. : high ? ll - 2.0 * lr : ll, fr = high ? 0. : low ? lr - 2.0 * ll : lr;
+    const double l3 = low ? 3.0 * ll : high ? 3.0 * lr : 0.;
+    // flat: l = r = x3, else the interface values
+    const double gl = flat ? 0. : 0.5 * fl, gr = flat ? 0. : 0.5 * fr, third = 1. / 3.;
+    v[1] += gl;
+    v[2] += l3 + (flat ? fl + fr : gl + gr);
+    v[3] += gr;
+    s0.vjp(gl * third, v);
+    s1.vjp((gr - gl) * third, v + 1);
+    s2.vjp(-gr * third, v + 2);
+}
+
 // ---------------------------------------------------------------------------
 // Adjoints of the MHD state of one set of primitives (ucon, ucov, bcon, bcov,
-// rho, u), accumulated by the flux and speed adjoints and pulled back to the
-// primitives by state_pullback.
+// rho, u), pulled back to the primitives by state_pullback.
 struct StateAdj {
     double ucon[4], ucov[4], bcon[4], bcov[4], rho, u, bsq;
 };
 
-HD void state_adj_zero(StateAdj &a)
-{
-    for (int k = 0; k < 4; k++) a.ucon[k] = a.ucov[k] = a.bcon[k] = a.bcov[k] = 0.;
-    a.rho = a.u = a.bsq = 0.;
-}
-
-// primtoflux (GPU_phys_mhd.h:432) in direction dir, reverse: lF are the
-// adjoints of the nine (gdet-weighted) outputs.
-HD void primtoflux_vjp(const double *pr, const State<double> &q, int dir, const Geom<double> &G, double gam,
-                       const double *lF, StateAdj &a)
-{
-    const double rho = pr[RHO], u = pr[UU], P = (gam - 1.) * u;
-    const double bsq = dot4(q.bcon, q.bcov), eta = rho + P + u + bsq;
-    const double ud = q.ucon[dir], bd = q.bcon[dir];
-    double lf[NPR];
-    for (int k = 0; k < NPR; k++) lf[k] = G.g * lF[k];
-    // f[KTOT] = f[RHO] * entr, entr = P rho^-gam; f[UU] = mhd[0] + f[RHO]
-    const double rmg = pow(rho, -gam), entr = P * rmg, fr = rho * ud;
-    const double lfr = lf[RHO] + lf[UU] + lf[KTOT] * entr;
-    const double lentr = lf[KTOT] * fr;
-    a.rho += lfr * ud - lentr * gam * entr / rho;
-    a.u += lentr * (gam - 1.) * rmg;
-    a.ucon[dir] += lfr * rho;
-    // mhd[j] = eta ud u_j + ptot delta(dir, j) - bd b_j
-    double leta = 0., lptot = 0.;
-    for (int j = 0; j < 4; j++) {
-        const double lm = (j == 0) ? lf[UU] : lf[U1 + j - 1];
-        leta += lm * ud * q.ucov[j];
-        a.ucon[dir] += lm * eta * q.ucov[j];
-        a.ucov[j] += lm * eta * ud;
-        if (j == dir) lptot += lm;
-        a.bcon[dir] -= lm * q.bcov[j];
-        a.bcov[j] -= lm * bd;
+// One state's flux along d (0: its conserved variables; primtoflux,
+// GPU_phys_mhd.h:432), contracted with weights lf of its nine components that
+// hold the factor gdet:
+//   S(d) = u^d Q - b^d R + ptot lf_d,
+//   Q = rho (lf_rho + lf_u + lf_K entr) + eta lf_j u_j + lf_Bj b^j,  R = lf_j b_j + lf_Bj u^j,
+// lf_j the weights of T^d_j.  The HLL adjoint needs no flux by itself, only
+// these sums, and its weights of a state's flux and of its conserved variables
+// are lf times one number each; so Q, R and their factors serve both.
+struct Contraction {
+    double eta, ptot, mu, Q, R, rmg, entr, bsq, w;
+    HD Contraction(const double *pr, const State<double> &q, double gam, const double *lf)
+    {
+        const double rho = pr[RHO], u = pr[UU], P = (gam - 1.) * u;
+        w = rho + P + u;
+        bsq = dot4(q.bcon, q.bcov);
+        eta = w + bsq;
+        ptot = P + 0.5 * bsq;
+        rmg = rpow(rho, -gam);
+        entr = P * rmg;
+        const double *m = lf + UU, *n = lf + B1;
+        mu = dot4(m, q.ucov);
+        Q = rho * (lf[RHO] + lf[UU] + lf[KTOT] * entr) + eta * mu
+            + (n[0] * q.bcon[1] + n[1] * q.bcon[2] + n[2] * q.bcon[3]);
+        R = dot4(m, q.bcov) + (n[0] * q.ucon[1] + n[1] * q.ucon[2] + n[2] * q.ucon[3]);
     }
-    // f[Bj] = b^j ud - bd u^j
+    HD double S(const State<double> &q, const double *lf, int d) const
+    {
+        return q.ucon[d] * Q - q.bcon[d] * R + ptot * lf[UU + d];
+    }
+};
+static_assert(U1 == UU + 1 && U2 == UU + 2 && U3 == UU + 3 && B2 == B1 + 1 && B3 == B1 + 2, "order of the components");
+
+// The adjoint of sF S(dir) + sU S(0): sets a.
+HD void contraction_vjp(const double *pr, const State<double> &q, const Contraction &c, int dir, double gam,
+                        const double *lf, double sF, double sU, StateAdj &a)
+{
+    const double Wu = sF * q.ucon[dir] + sU * q.ucon[0], Wb = sF * q.bcon[dir] + sU * q.bcon[0];
+    const double Wm = sF * lf[UU + dir] + sU * lf[UU];
+    const double *m = lf + UU, *n = lf + B1;
+    a.ucon[0] = sU * c.Q;
+    a.bcon[0] = -sU * c.R;
     for (int j = 1; j < 4; j++) {
-        const double l = lf[B1 + j - 1];
-        a.bcon[j] += l * ud;
-        a.ucon[dir] += l * q.bcon[j];
-        a.bcon[dir] -= l * q.ucon[j];
-        a.ucon[j] -= l * bd;
+        a.ucon[j] = -Wb * n[j - 1];
+        a.bcon[j] = Wu * n[j - 1];
     }
-    // eta = rho + gam u + bsq, ptot = (gam - 1) u + bsq / 2
-    a.rho += leta;
-    a.u += leta * gam + lptot * (gam - 1.);
-    a.bsq += leta + 0.5 * lptot;
+    for (int j = 0; j < 4; j++) {
+        a.ucov[j] = Wu * c.eta * m[j];
+        a.bcov[j] = -Wb * m[j];
+    }
+    a.ucon[dir] += sF * c.Q;
+    a.bcon[dir] -= sF * c.R;
+    const double leta = Wu * c.mu;
+    a.rho = Wu * (lf[RHO] + lf[UU] + (1. - gam) * lf[KTOT] * c.entr) + leta;
+    a.u = Wu * lf[KTOT] * pr[RHO] * (gam - 1.) * c.rmg + leta * gam + Wm * (gam - 1.);
+    a.bsq = leta + 0.5 * Wm;
 }
 
-// Magnetosonic speeds of primtoflux (GPU_phys_mhd.h:550-617), reverse.
-HD void speeds_vjp(const double *pr, const State<double> &q, int dir, const Geom<double> &G, double gam, double lvmax,
-                   double lvmin, StateAdj &a)
-{
-    const double rho = pr[RHO], u = pr[UU], P = (gam - 1.) * u, w = rho + P + u;
-    const double bsq = dot4(q.bcon, q.bcov), eta = w + bsq;
-    double Acon_0, Acon_js;
-    if (dir == 1) { Acon_0 = G.gcon[1]; Acon_js = G.gcon[4]; }
-    else if (dir == 2) { Acon_0 = G.gcon[2]; Acon_js = G.gcon[7]; }
-    else { Acon_0 = G.gcon[3]; Acon_js = G.gcon[9]; }
-    const double cs2 = gam * (gam - 1.) * u / w, va2 = bsq / eta;
-    double cms2 = cs2 + va2 - cs2 * va2;
-    bool clamped = false;
-    if (cms2 < 0.) { cms2 = kSMALL; clamped = true; }
-    if (cms2 > 1.) { cms2 = 1.; clamped = true; }
-    const double Asq = Acon_js, Bsq = G.gcon[0], Au = q.ucon[dir], Bu = q.ucon[0], AB = Acon_0;
-    const double Au2 = Au * Au, Bu2 = Bu * Bu, AuBu = Au * Bu;
-    const double A = Bu2 - (Bsq + Bu2) * cms2;
-    const double B = 2. * (AuBu - (AB + AuBu) * cms2);
-    const double C = Au2 - (Asq + Au2) * cms2;
-    double discr = B * B - 4. * A * C;
-    const bool dclamp = !(discr > 0.);
-    if (dclamp) discr = 0.;
-    const double sd = sqrt(discr);
-    const double vp = -(-B + sd) / (2. * A), vm = -(-B - sd) / (2. * A);
-    // vmax = max(vp, vm), vmin = min(vp, vm)
-    double lvp, lvm;
-    if (vp > vm) { lvp = lvmax; lvm = lvmin; }
-    else { lvp = lvmin; lvm = lvmax; }
-    // vp = (B - sd) / (2A), vm = (B + sd) / (2A)
-    double lB = (lvp + lvm) / (2. * A);
-    const double lsd = (lvm - lvp) / (2. * A);
-    double lA = -(lvp * vp + lvm * vm) / A;
-    double lC = 0.;
-    if (!dclamp) {
-        const double ld = lsd / (2. * sd);
-        lB += ld * 2. * B;
-        lA += -4. * C * ld;
-        lC += -4. * A * ld;
+// Magnetosonic speeds of a state along dir (vchar_coord, GPU_phys_mhd.h:550-617)
+// with what their reverse uses.
+struct Speeds {
+    double vp, vm, A, B, C, sd, cms2, cs2, va2, Acon_0, Acon_js;
+    Div<double> by_w, by_eta, by_2A;
+    bool clamped, dclamp;
+    HD Speeds(const double *pr, const State<double> &q, const Contraction &c, int dir, const Geom<double> &G, double gam)
+        : by_w(c.w), by_eta(c.eta), by_2A(1.)
+    {
+        if (dir == 1) { Acon_0 = G.gcon[1]; Acon_js = G.gcon[4]; }
+        else if (dir == 2) { Acon_0 = G.gcon[2]; Acon_js = G.gcon[7]; }
+        else { Acon_0 = G.gcon[3]; Acon_js = G.gcon[9]; }
+        cs2 = by_w(gam * (gam - 1.) * pr[UU]);
+        va2 = by_eta(c.bsq);
+        cms2 = cs2 + va2 - cs2 * va2;
+        clamped = false;
+        if (cms2 < 0.) { cms2 = kSMALL; clamped = true; }
+        if (cms2 > 1.) { cms2 = 1.; clamped = true; }
+        const double Bsq = G.gcon[0], Au = q.ucon[dir], Bu = q.ucon[0];
+        A = Bu * Bu - (Bsq + Bu * Bu) * cms2;
+        B = 2. * (Au * Bu - (Acon_0 + Au * Bu) * cms2);
+        C = Au * Au - (Acon_js + Au * Au) * cms2;
+        double discr = B * B - 4. * A * C;
+        dclamp = !(discr > 0.);
+        if (dclamp) discr = 0.;
+        sd = sqrt(discr);
+        by_2A = Div<double>(2. * A);
+        vp = by_2A(B - sd);
+        vm = by_2A(B + sd);
     }
-    const double om = 1. - cms2;
-    a.ucon[0] += lA * 2. * Bu * om + lB * 2. * Au * om;
-    a.ucon[dir] += lB * 2. * Bu * om + lC * 2. * Au * om;
-    if (clamped) return;
-    const double lcms2 = -lA * (Bsq + Bu2) - lB * 2. * (AB + AuBu) - lC * (Asq + Au2);
-    const double lcs2 = lcms2 * (1. - va2), lva2 = lcms2 * (1. - cs2);
-    // cs2 = gam (gam - 1) u / w, w = rho + gam u
-    a.u += lcs2 * (gam * (gam - 1.) / w - cs2 * gam / w);
-    a.rho += -lcs2 * cs2 / w;
-    // va2 = bsq / eta, eta = rho + gam u + bsq
-    const double leta = -lva2 * va2 / eta;
-    a.bsq += lva2 / eta + leta;
-    a.rho += leta;
-    a.u += leta * gam;
-}
+    HD double vmax() const { return mymax(vp, vm); }
+    HD double vmin() const { return mymin(vp, vm); }
+
+    // adds the adjoint of lvmax vmax + lvmin vmin to a
+    HD void vjp(const State<double> &q, int dir, const Geom<double> &G, double gam, double lvmax, double lvmin,
+                StateAdj &a) const
+    {
+        const double lvp = vp > vm ? lvmax : lvmin, lvm = vp > vm ? lvmin : lvmax;
+        double lB = by_2A(lvp + lvm), lA = -2. * by_2A(lvp * vp + lvm * vm), lC = 0.;
+        if (!dclamp) {
+            const double ld = Div<double>(2. * sd)(by_2A(lvm - lvp));
+            lB += ld * 2. * B;
+            lA += -4. * C * ld;
+            lC = -4. * A * ld;
+        }
+        const double Bsq = G.gcon[0], Au = q.ucon[dir], Bu = q.ucon[0], om = 1. - cms2;
+        a.ucon[0] += lA * 2. * Bu * om + lB * 2. * Au * om;
+        a.ucon[dir] += lB * 2. * Bu * om + lC * 2. * Au * om;
+        if (clamped) return;
+        const double lcms2 = -lA * (Bsq + Bu * Bu) - lB * 2. * (Acon_0 + Au * Bu) - lC * (Acon_js + Au * Au);
+        const double lw = by_w(lcms2 * (1. - va2)), le = by_eta(lcms2 * (1. - cs2));
+        // cs2 = gam (gam - 1) u / w, w = rho + gam u
+        a.u += lw * gam * ((gam - 1.) - cs2);
+        a.rho -= lw * cs2;
+        // va2 = bsq / eta, eta = rho + gam u + bsq
+        const double leta = -le * va2;
+        a.bsq += le + leta;
+        a.rho += leta;
+        a.u += leta * gam;
+    }
+};
 
 // get_state (GPU_phys_mhd.h:692-760), reverse: adds the primitives' adjoints to lpr.
-HD void state_pullback(const double *pr, const State<double> &q, const Geom<double> &G, StateAdj &a, double *lpr)
+HD void state_pullback(const double *pr, const State<double> &q, const Geom<double> &G, const Lapse<double> &L,
+                       StateAdj &a, double *lpr)
 {
     // bsq = bcon . bcov
     for (int m = 0; m < 4; m++) {
@@ -277,14 +339,15 @@ HD void state_pullback(const double *pr, const State<double> &q, const Geom<doub
         for (int m = 0; m < 4; m++) a.bcon[m] += t[m];
     }
     // bcon[j] = (B_j + b0 u^j) / u0, b0 = B . ucov(1..3)
-    const double u0 = q.ucon[0], b0 = q.bcon[0];
+    const Div<double> by_u0(q.ucon[0]);
+    const double b0 = q.bcon[0];
     double lb0 = a.bcon[0];
     for (int j = 1; j < 4; j++) {
-        const double l = a.bcon[j];
-        lpr[B1 + j - 1] += l / u0;
-        lb0 += l * q.ucon[j] / u0;
-        a.ucon[j] += l * b0 / u0;
-        a.ucon[0] -= l * q.bcon[j] / u0;
+        const double l = by_u0(a.bcon[j]);
+        lpr[B1 + j - 1] += l;
+        lb0 += l * q.ucon[j];
+        a.ucon[j] += l * b0;
+        a.ucon[0] -= l * q.bcon[j];
     }
     for (int i = 1; i < 4; i++) {
         lpr[B1 + i - 1] += lb0 * q.ucov[i];
@@ -297,68 +360,93 @@ HD void state_pullback(const double *pr, const State<double> &q, const Geom<doub
         for (int m = 0; m < 4; m++) a.ucon[m] += t[m];
     }
     // ucon[0] = gamma / alpha, ucon[j] = U_j - gamma beta_j / alpha
-    const double alpha = 1. / sqrt(-G.gcon[0]);
-    double lgam = a.ucon[0] / alpha;
+    double lgam = a.ucon[0];
     for (int j = 1; j < 4; j++) {
-        const double beta = G.gcon[j] * alpha * alpha;
-        lgam -= a.ucon[j] * beta / alpha;
+        lgam -= a.ucon[j] * L.beta[j];
         lpr[U1 + j - 1] += a.ucon[j];
     }
+    lgam = L.by_alpha(lgam);
     // gamma = sqrt(1 + qsq), qsq = U . g_spatial . U (no derivative where clamped)
     const double *g = G.gcov;
     const double U[3] = {pr[U1], pr[U2], pr[U3]};
+    const double v0 = g[4] * U[0] + g[5] * U[1] + g[6] * U[2], v1 = g[5] * U[0] + g[7] * U[1] + g[8] * U[2],
+                 v2 = g[6] * U[0] + g[8] * U[1] + g[9] * U[2];
     const double qsq = g[4] * U[0] * U[0] + g[7] * U[1] * U[1] + g[9] * U[2] * U[2]
         + 2. * (g[5] * U[0] * U[1] + g[6] * U[0] * U[2] + g[8] * U[1] * U[2]);
     if (qsq >= 0.) {
-        const double gamma = sqrt(1. + qsq);
-        const double lq = lgam / (2. * gamma);
-        lpr[U1] += lq * 2. * (g[4] * U[0] + g[5] * U[1] + g[6] * U[2]);
-        lpr[U2] += lq * 2. * (g[5] * U[0] + g[7] * U[1] + g[8] * U[2]);
-        lpr[U3] += lq * 2. * (g[6] * U[0] + g[8] * U[1] + g[9] * U[2]);
+        const double lq = Div<double>(sqrt(1. + qsq))(lgam);
+        lpr[U1] += lq * v0;
+        lpr[U2] += lq * v1;
+        lpr[U3] += lq * v2;
     }
     lpr[RHO] += a.rho;
     lpr[UU] += a.u;
 }
 
-// One face state: fluxes F (dir), conserved U (dir 0) and speeds, reverse.
-HD void face_state_vjp(const double *pr, const Geom<double> &G, int dir, double gam, const double *lF, const double *lU,
-                       double lvmax, double lvmin, double *lpr)
+// Conserved variables U(P) (primtoflux, dir 0) with weights lU, and the
+// cell-centre EMF E_i = -gdet (u^j b^k - u^k b^j) (GPU_const_trans.h:63-119) with
+// weights lE, reverse: sets lpr.
+HD void cell_vjp(const double *pr, const Geom<double> &G, double gam, const double *lU, const double *lE, double *lpr)
 {
+    const Lapse<double> L(G);
     State<double> q;
-    get_state(pr, G, q);
+    get_state(pr, G, L, q);
+    double lf[NPR];
+    for (int k = 0; k < NPR; k++) {
+        lf[k] = G.g * lU[k];
+        lpr[k] = 0.;
+    }
+    const Contraction c(pr, q, gam, lf);
     StateAdj a;
-    state_adj_zero(a);
-    primtoflux_vjp(pr, q, dir, G, gam, lF, a);
-    primtoflux_vjp(pr, q, 0, G, gam, lU, a);
-    speeds_vjp(pr, q, dir, G, gam, lvmax, lvmin, a);
-    state_pullback(pr, q, G, a, lpr);
-}
-
-// Conserved variables U(P) (primtoflux, dir 0), reverse.
-HD void conserved_vjp(const double *pr, const Geom<double> &G, double gam, const double *lU, double *lpr)
-{
-    State<double> q;
-    get_state(pr, G, q);
-    StateAdj a;
-    state_adj_zero(a);
-    primtoflux_vjp(pr, q, 0, G, gam, lU, a);
-    state_pullback(pr, q, G, a, lpr);
-}
-
-// Cell-centre EMF E_i = -gdet (u^j b^k - u^k b^j) (GPU_const_trans.h:63-119), reverse.
-HD void ecent_vjp(const double *pr, const Geom<double> &G, const double *lE, double *lpr)
-{
-    State<double> q;
-    get_state(pr, G, q);
-    StateAdj a;
-    state_adj_zero(a);
+    contraction_vjp(pr, q, c, 0, gam, lf, 0., 1., a);
     const double *u = q.ucon, *b = q.bcon;
     // E1 = -g (u2 b3 - u3 b2), E2 = -g (u3 b1 - u1 b3), E3 = -g (u1 b2 - u2 b1)
     const double l1 = -G.g * lE[0], l2 = -G.g * lE[1], l3 = -G.g * lE[2];
-    a.ucon[2] += l1 * b[3]; a.bcon[3] += l1 * u[2]; a.ucon[3] -= l1 * b[2]; a.bcon[2] -= l1 * u[3];
-    a.ucon[3] += l2 * b[1]; a.bcon[1] += l2 * u[3]; a.ucon[1] -= l2 * b[3]; a.bcon[3] -= l2 * u[1];
-    a.ucon[1] += l3 * b[2]; a.bcon[2] += l3 * u[1]; a.ucon[2] -= l3 * b[1]; a.bcon[1] -= l3 * u[2];
-    state_pullback(pr, q, G, a, lpr);
+    a.ucon[1] += l3 * b[2] - l2 * b[3];
+    a.ucon[2] += l1 * b[3] - l3 * b[1];
+    a.ucon[3] += l2 * b[1] - l1 * b[2];
+    a.bcon[1] += l2 * u[3] - l3 * u[2];
+    a.bcon[2] += l3 * u[1] - l1 * u[3];
+    a.bcon[3] += l1 * u[2] - l2 * u[1];
+    state_pullback(pr, q, G, L, a, lpr);
+}
+
+// HLL flux through a face (nine components with weights lf) of the states pl
+// and pr, reverse: sets lpl and lpr.
+HD void hll_vjp(const double *pl, const double *pr, const Geom<double> &G, int dir, double gam, double *lf, double *lpl,
+                double *lpr)
+{
+    for (int k = 0; k < NPR; k++) {
+        lf[k] *= G.g;
+        lpl[k] = lpr[k] = 0.;
+    }
+    const Lapse<double> L(G);
+    State<double> ql, qr;
+    get_state(pl, G, L, ql);
+    get_state(pr, G, L, qr);
+    const Contraction cl(pl, ql, gam, lf), cr(pr, qr, gam, lf);
+    const Speeds vl(pl, ql, cl, dir, G, gam), vr(pr, qr, cr, dir, G, gam);
+    const double vxl = vl.vmax(), vnl = vl.vmin(), vxr = vr.vmax(), vnr = vr.vmin();
+    const double m1 = mymax(0., vxl), cmax = fabs(mymax(m1, vxr));
+    const double n1 = mymax(0., -vnl), cmin = fabs(mymax(n1, -vnr));
+    const Div<double> by_den(cmax + cmin + kSMALL);
+    // reverse of F = (cmax FL + cmin FR - cmax cmin (UR - UL)) / den
+    const double SL = cl.S(ql, lf, dir), SR = cr.S(qr, lf, dir), D = cr.S(qr, lf, 0) - cl.S(ql, lf, 0);
+    const double sL = by_den(cmax), sR = by_den(cmin), sU = by_den(cmax * cmin);
+    const double F = by_den(cmax * SL + cmin * SR - cmax * cmin * D);
+    const double lcmax = by_den((SL - cmin * D) - F), lcmin = by_den((SR - cmax * D) - F);
+    double lvxl = 0., lvxr = 0., lvnl = 0., lvnr = 0.;
+    if (m1 > vxr) { if (!(0. > vxl)) lvxl = lcmax; }
+    else lvxr = lcmax;
+    if (n1 > -vnr) { if (!(0. > -vnl)) lvnl = -lcmin; }
+    else lvnr = -lcmin;
+    StateAdj a;
+    contraction_vjp(pl, ql, cl, dir, gam, lf, sL, sU, a);
+    vl.vjp(ql, dir, G, gam, lvxl, lvnl, a);
+    state_pullback(pl, ql, G, L, a, lpl);
+    contraction_vjp(pr, qr, cr, dir, gam, lf, sR, -sU, a);
+    vr.vjp(qr, dir, G, gam, lvxr, lvnr, a);
+    state_pullback(pr, qr, G, L, a, lpr);
 }
 
 }  // namespace hamr

@@ -9,389 +9,326 @@
 // field at the start of the stage) in reverse order, recomputing the
 // reconstructed states, fluxes and EMF selections from P instead of storing
 // them.  The source term is zero in the flat metric the adjoint serves (a
-// periodic box of one block); ghost cells are folded back onto the interior
-// cells they copy.
+// periodic box of one block).
+//
+// Every kernel gathers: a thread owns a cell, face or edge and reads what
+// reaches it, with indices wrapped into the periodic box, so each of the box's
+// n1 n2 n3 faces of a direction is taken once (its ghost copies and the copies on
+// the upper boundary add up in their common weight) and nothing is
+// accumulated by atomics: a call gives the same bits every time.
 #include "hamr_adjoint.h"
-#include "hamr_kernels.h"
+#include "hamr_kernels_dev.h"
 
 namespace hamr {
 
 namespace {
 
+// components of P that are reconstructed at a face: all but KTOT (which does not
+// enter the stage) and the normal field; each takes two slabs of the faces' buffer
+constexpr int kAdjRec = 7;
+static_assert(kAdjXSlabs == 2 * kAdjRec, "two slabs per reconstructed component");
+
 struct AdjArgs {
     int D[3], bs[3];
-    int64_t K;           // slab length
+    int n;               // interior cells
+    int64_t K;           // slab length of the context's arrays and the scratch
+    int64_t Kw, Kg;      // slab length of the weights and of the gradients
     double dx[3], Dt, gam;
     const double *gcov, *gcon, *gdet;  // geometry slab 0
     int64_t kcol;
 };
 
-__device__ __forceinline__ int64_t cell_of(const AdjArgs &A, int i, int j, int z)
+// periodic image inside the interior of an index at most bs cells outside
+__device__ __forceinline__ int wrap1(int i, int bs) { return i < NG ? i + bs : i >= NG + bs ? i - bs : i; }
+
+__device__ __forceinline__ uint32_t cell_of(const AdjArgs &A, int i, int j, int z)
 {
-    return ((int64_t)i * A.D[1] + j) * A.D[2] + z;
+    return ((uint32_t)i * A.D[1] + j) * A.D[2] + z;
 }
 
-// periodic image of a (possibly ghost) index inside the interior
-__device__ __forceinline__ int wrap(int i, int bs) { return ((i - NG) % bs + bs) % bs + NG; }
-
-__device__ __forceinline__ int64_t fold(const AdjArgs &A, int i, int j, int z)
+// Interior cell number t (z fastest).
+__device__ __forceinline__ void decode(const AdjArgs &A, int t, int &i, int &j, int &z)
 {
-    return cell_of(A, wrap(i, A.bs[0]), wrap(j, A.bs[1]), wrap(z, A.bs[2]));
+    int a, b, c;
+    region_index(t, A.bs[1], A.bs[2], a, b, c);
+    i = a + NG;
+    j = b + NG;
+    z = c + NG;
 }
 
-__device__ __forceinline__ void decode(int64_t t, int e1, int e2, int e3, int &a, int &b, int &c)
-{
-    c = (int)(t % e3);
-    const int64_t q = t / e3;
-    b = (int)(q % e2);
-    a = (int)(q / e2);
-}
-
-__device__ __forceinline__ Geom<double> geom_at(const AdjArgs &A, int pos, int64_t col)
+__device__ __forceinline__ Geom<double> geom_at(const AdjArgs &A, int pos, uint32_t col)
 {
     Geom<double> G;
+#pragma unroll
     for (int s = 0; s < 10; s++) {
-        G.gcov[s] = A.gcov[((int64_t)pos * 10 + s) * A.kcol + col];
-        G.gcon[s] = A.gcon[((int64_t)pos * 10 + s) * A.kcol + col];
+        G.gcov[s] = gld(A.gcov + ((int64_t)pos * 10 + s) * A.kcol, col);
+        G.gcon[s] = gld(A.gcon + ((int64_t)pos * 10 + s) * A.kcol, col);
     }
-    G.g = A.gdet[(int64_t)pos * A.kcol + col];
+    G.g = gld(A.gdet + (int64_t)pos * A.kcol, col);
     return G;
 }
 
-__device__ __forceinline__ bool interior(const AdjArgs &A, int i, int j, int z)
+// 1 where a mass flux selects the lower side (the corner EMF's upwinding)
+__device__ __forceinline__ double sel(const double *F, uint32_t g) { return (double)(gld(F, g) <= 0.0); }
+
+// Adjoint of the field flux component of a face along DIR (stride sd) whose
+// transverse direction has stride st: from the corner EMFs at both ends, e the
+// EMF's adjoint and F the mass flux along the transverse direction.
+__device__ __forceinline__ double field_flux(const double *e, const double *F, uint32_t g, uint32_t sd, uint32_t st)
 {
-    return i >= NG && i < NG + A.bs[0] && j >= NG && j < NG + A.bs[1] && z >= NG && z < NG + A.bs[2];
+    return 0.25 * (gld(e, g) * (1. + sel(F, g) + sel(F, g - sd))
+                   + gld(e, g + st) * (3. - sel(F, g + st) - sel(F, g + st - sd)));
+}
+
+// Adjoint of a centre EMF component whose two transverse directions have strides
+// sa, sb: from the four corners around the cell; Fa, Fb the mass fluxes along them.
+__device__ __forceinline__ double centre_emf(const double *e, const double *Fa, const double *Fb, uint32_t g, uint32_t sa,
+                                             uint32_t sb)
+{
+    const double a0 = sel(Fa, g), a1 = 1. - sel(Fa, g + sa), b0 = sel(Fb, g), b1 = 1. - sel(Fb, g + sb);
+    return -0.25 * (gld(e, g) * (a0 + b0) + gld(e, g + sa) * (a1 + b0) + gld(e, g + sb) * (a0 + b1)
+                    + gld(e, g + sa + sb) * (a1 + b1));
 }
 
 }  // namespace
 
-// lam_psf: adjoint of the updated face fields from w[B] (the face average of U'[B]).
-__global__ void __launch_bounds__(256) k_adj_seed(AdjArgs A, const double *__restrict__ w, double *__restrict__ lpsf)
+// lE, the adjoint of the corner EMFs, at the corners [NG, NG + bs] (transpose of
+// the face-field update and of the face average of U'[B]), and lps, the part of
+// dL/dB_f that the updated face field carries over; zero in the ghosts.
+__global__ void __launch_bounds__(256) k_adj_edge(AdjArgs A, const double *__restrict__ w, double *__restrict__ lE,
+                                                  double *__restrict__ lps)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)A.D[0] * A.D[1] * A.D[2];
-    if (t >= N) return;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= A.D[0] * A.D[1] * A.D[2]) return;
     int i, j, z;
-    decode(t, A.D[0], A.D[1], A.D[2], i, j, z);
-    const int64_t col = (int64_t)i * A.D[1] + j;
-    const int64_t K = A.K, si = (int64_t)A.D[1] * A.D[2], sj = A.D[2];
-    for (int d = 0; d < 3; d++) {
-        const int pos = d == 0 ? FACE1 : d == 1 ? FACE2 : FACE3;
-        const int64_t sd = d == 0 ? si : d == 1 ? sj : 1;
-        const double gf = A.gdet[(int64_t)pos * A.kcol + col];
-        double v = 0.;
-        if (interior(A, i, j, z)) v += w[(B1 + d) * K + t];
-        const int im = i - (d == 0), jm = j - (d == 1), zm = z - (d == 2);
-        if (interior(A, im, jm, zm)) v += w[(B1 + d) * K + t - sd];
-        lpsf[d * K + t] = gf * v / 2.;
+    region_index(t, A.D[1], A.D[2], i, j, z);
+    if (i < NG || i > NG + A.bs[0] || j < NG || j > NG + A.bs[1] || z < NG || z > NG + A.bs[2]) {
+        for (int d = 0; d < 3; d++) gst(lps + d * A.Kg, (uint32_t)t, 0.);
+        return;
     }
+    const int i0 = wrap1(i, A.bs[0]), j0 = wrap1(j, A.bs[1]), z0 = wrap1(z, A.bs[2]);
+    const int im = wrap1(i0 - 1, A.bs[0]), jm = wrap1(j0 - 1, A.bs[1]), zm = wrap1(z0 - 1, A.bs[2]);
+    const double *w0 = w + B1 * A.Kw, *w1 = w + B2 * A.Kw, *w2 = w + B3 * A.Kw;
+    // face averages at the corner's cell c and its lower neighbours
+    const uint32_t c = cell_of(A, i0, j0, z0), ci = cell_of(A, im, j0, z0), cj = cell_of(A, i0, jm, z0),
+                   cz = cell_of(A, i0, j0, zm), cij = cell_of(A, im, jm, z0), ciz = cell_of(A, im, j0, zm),
+                   cjz = cell_of(A, i0, jm, zm);
+    const double v0 = 0.5 * (gld(w0, c) + gld(w0, ci)), v1 = 0.5 * (gld(w1, c) + gld(w1, cj)),
+                 v2 = 0.5 * (gld(w2, c) + gld(w2, cz));
+    const double v0j = 0.5 * (gld(w0, cj) + gld(w0, cij)), v0z = 0.5 * (gld(w0, cz) + gld(w0, ciz));
+    const double v1i = 0.5 * (gld(w1, ci) + gld(w1, cij)), v1z = 0.5 * (gld(w1, cz) + gld(w1, cjz));
+    const double v2i = 0.5 * (gld(w2, ci) + gld(w2, ciz)), v2j = 0.5 * (gld(w2, cj) + gld(w2, cjz));
+    const double r1 = A.Dt / A.dx[0], r2 = A.Dt / A.dx[1], r3 = A.Dt / A.dx[2];
+    gst(lE, (uint32_t)t, r3 * (v1 - v1z) - r2 * (v2 - v2j));
+    gst(lE + A.K, (uint32_t)t, r1 * (v2 - v2i) - r3 * (v0 - v0z));
+    gst(lE + 2 * A.K, (uint32_t)t, r2 * (v0 - v0j) - r1 * (v1 - v1i));
+    const bool in = i == i0 && j == j0 && z == z0;
+    const uint32_t col = (uint32_t)i * A.D[1] + j;
+    gst(lps, (uint32_t)t, in ? gld(A.gdet + FACE1 * A.kcol, col) * v0 : 0.);
+    gst(lps + A.Kg, (uint32_t)t, in ? gld(A.gdet + FACE2 * A.kcol, col) * v1 : 0.);
+    gst(lps + 2 * A.Kg, (uint32_t)t, in ? gld(A.gdet + FACE3 * A.kcol, col) * v2 : 0.);
 }
 
-// lam_E from lam_psf (transpose of the face-field update), and the direct part
-// of lam_ps (the updated face field carries the old one with weight 1).
-__global__ void __launch_bounds__(256) k_adj_ct(AdjArgs A, const double *__restrict__ lpsf, double *__restrict__ lE,
-                                                double *__restrict__ lps)
+// lP (initialised here, zero in the ghosts) from U(P) and the centre EMF.
+__global__ void __launch_bounds__(256) k_adj_cell(AdjArgs A, const double *__restrict__ p, const double *__restrict__ w,
+                                                  const double *__restrict__ lE, const double *__restrict__ F1,
+                                                  const double *__restrict__ F2, const double *__restrict__ F3,
+                                                  double *__restrict__ lP)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)A.D[0] * A.D[1] * A.D[2];
-    if (t >= N) return;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= A.D[0] * A.D[1] * A.D[2]) return;
     int i, j, z;
-    decode(t, A.D[0], A.D[1], A.D[2], i, j, z);
-    const int64_t K = A.K, si = (int64_t)A.D[1] * A.D[2], sj = A.D[2];
-    const int64_t col = (int64_t)i * A.D[1] + j;
-    const double Dt = A.Dt, dx1 = A.dx[0], dx2 = A.dx[1], dx3 = A.dx[2];
-    auto gF = [&](int pos, int64_t c) { return A.gdet[(int64_t)pos * A.kcol + c]; };
-    auto L0 = [&](int64_t g) { return lpsf[g]; };
-    auto L1 = [&](int64_t g) { return lpsf[K + g]; };
-    auto L2 = [&](int64_t g) { return lpsf[2 * K + g]; };
-    // faces the forward updates (psf0: i in [NG, NG+bs1], j, z interior; cyclic for 1, 2)
-    auto ok0 = [&](int a, int b, int c) { return a >= NG && a <= NG + A.bs[0] && b >= NG && b < NG + A.bs[1] && c >= NG && c < NG + A.bs[2]; };
-    auto ok1 = [&](int a, int b, int c) { return a >= NG && a < NG + A.bs[0] && b >= NG && b <= NG + A.bs[1] && c >= NG && c < NG + A.bs[2]; };
-    auto ok2 = [&](int a, int b, int c) { return a >= NG && a < NG + A.bs[0] && b >= NG && b < NG + A.bs[1] && c >= NG && c <= NG + A.bs[2]; };
-    // direct part (faces on the upper block boundary are ghost copies: folded)
-    if (ok0(i, j, z)) atomicAdd(&lps[fold(A, i, j, z)], L0(t));
-    if (ok1(i, j, z)) atomicAdd(&lps[K + fold(A, i, j, z)], L1(t));
-    if (ok2(i, j, z)) atomicAdd(&lps[2 * K + fold(A, i, j, z)], L2(t));
-    if (i < NG || i > NG + A.bs[0] || j < NG || j > NG + A.bs[1] || z < NG || z > NG + A.bs[2]) return;
-    double e1 = 0., e2 = 0., e3 = 0.;
-    // psf0[g] = (ps0 gF1 - Dt/dx2 (E3[g+sj] - E3[g]) + Dt/dx3 (E2[g+1] - E2[g])) / gF1
-    if (ok0(i, j, z)) {
-        const double l = L0(t) / gF(FACE1, col);
-        e3 += l * Dt / dx2;
-        e2 -= l * Dt / dx3;
+    region_index(t, A.D[1], A.D[2], i, j, z);
+    const uint32_t g = t;
+    if (i < NG || i >= NG + A.bs[0] || j < NG || j >= NG + A.bs[1] || z < NG || z >= NG + A.bs[2]) {
+        for (int k = 0; k < NPR; k++) gst(lP + k * A.Kg, g, 0.);
+        return;
     }
-    if (ok0(i, j - 1, z)) e3 -= L0(t - sj) / gF(FACE1, col - 1) * Dt / dx2;
-    if (ok0(i, j, z - 1)) e2 += L0(t - 1) / gF(FACE1, col) * Dt / dx3;
-    // psf2[g] = (ps2 gF3 - Dt/dx1 (E2[g+si] - E2[g]) + Dt/dx2 (E1[g+sj] - E1[g])) / gF3
-    if (ok2(i, j, z)) {
-        const double l = L2(t) / gF(FACE3, col);
-        e2 += l * Dt / dx1;
-        e1 -= l * Dt / dx2;
-    }
-    if (ok2(i - 1, j, z)) e2 -= L2(t - si) / gF(FACE3, col - A.D[1]) * Dt / dx1;
-    if (ok2(i, j - 1, z)) e1 += L2(t - sj) / gF(FACE3, col - 1) * Dt / dx2;
-    // psf1[g] = (ps1 gF2 + Dt/dx1 (E3[g+si] - E3[g]) - Dt/dx3 (E1[g+1] - E1[g])) / gF2
-    if (ok1(i, j, z)) {
-        const double l = L1(t) / gF(FACE2, col);
-        e3 -= l * Dt / dx1;
-        e1 += l * Dt / dx3;
-    }
-    if (ok1(i - 1, j, z)) e3 += L1(t - si) / gF(FACE2, col - A.D[1]) * Dt / dx1;
-    if (ok1(i, j, z - 1)) e1 -= L1(t - 1) / gF(FACE2, col) * Dt / dx3;
-    lE[t] = e1;
-    lE[K + t] = e2;
-    lE[2 * K + t] = e3;
-}
-
-// lam_F (all components) from the flux divergence of U' (the field components
-// of U' are the face averages, not the divergence).
-__global__ void __launch_bounds__(256) k_adj_div(AdjArgs A, const double *__restrict__ w, double *__restrict__ lF1,
-                                                 double *__restrict__ lF2, double *__restrict__ lF3)
-{
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)A.D[0] * A.D[1] * A.D[2];
-    if (t >= N) return;
-    int i, j, z;
-    decode(t, A.D[0], A.D[1], A.D[2], i, j, z);
-    const int64_t K = A.K, si = (int64_t)A.D[1] * A.D[2], sj = A.D[2];
-    const bool in0 = interior(A, i, j, z);
-    const bool in1 = interior(A, i - 1, j, z), in2 = interior(A, i, j - 1, z), in3 = interior(A, i, j, z - 1);
+    double pr[NPR], lU[NPR], lpr[NPR];
+#pragma unroll
     for (int k = 0; k < NPR; k++) {
-        const bool fld = (k == B1 || k == B2 || k == B3);
-        const double w0 = (in0 && !fld) ? w[k * K + t] : 0.;
-        const double wi = (in1 && !fld) ? w[k * K + t - si] : 0.;
-        const double wj = (in2 && !fld) ? w[k * K + t - sj] : 0.;
-        const double wz = (in3 && !fld) ? w[k * K + t - 1] : 0.;
-        lF1[k * K + t] = A.Dt / (A.dx[0] * 1.0) * (w0 - wi);
-        lF2[k * K + t] = A.Dt / (A.dx[1] * 1.0) * (w0 - wj);
-        lF3[k * K + t] = A.Dt / (A.dx[2] * 1.0) * (w0 - wz);
+        const bool fld = k == B1 || k == B2 || k == B3;
+        pr[k] = k == KTOT ? 0. : gld(p + k * A.K, g);
+        lU[k] = fld ? 0. : gld(w + k * A.Kw, g);
     }
+    const uint32_t sj = A.D[2], si = sj * A.D[1];
+    const double e[3] = {centre_emf(lE, F2, F3, g, sj, 1), centre_emf(lE + A.K, F3, F1, g, 1, si),
+                         centre_emf(lE + 2 * A.K, F2, F1, g, sj, si)};
+    const Geom<double> G = geom_at(A, CENT, (uint32_t)i * A.D[1] + j);
+    cell_vjp(pr, G, A.gam, lU, e, lpr);
+    for (int k = 0; k < NPR; k++) gst(lP + k * A.Kg, g, lpr[k]);
 }
 
-// lam_P (initialised here) from U(P) of the interior cells.
-__global__ void __launch_bounds__(256) k_adj_u0(AdjArgs A, const double *__restrict__ p, const double *__restrict__ w,
-                                                double *__restrict__ lP)
+// Reconstructed component number v of the faces along DIR.
+template <int DIR> __device__ __forceinline__ constexpr int rec_comp(int v)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t N = (int64_t)A.D[0] * A.D[1] * A.D[2];
-    if (t >= N) return;
-    int i, j, z;
-    decode(t, A.D[0], A.D[1], A.D[2], i, j, z);
-    const int64_t K = A.K;
-    double lpr[NPR];
-    for (int k = 0; k < NPR; k++) lpr[k] = 0.;
-    if (interior(A, i, j, z)) {
-        double pr[NPR], lU[NPR];
-        for (int k = 0; k < NPR; k++) {
-            pr[k] = p[k * K + t];
-            lU[k] = (k == B1 || k == B2 || k == B3) ? 0. : w[k * K + t];
-        }
-        const Geom<double> G = geom_at(A, CENT, (int64_t)i * A.D[1] + j);
-        conserved_vjp(pr, G, A.gam, lU, lpr);
-    }
-    for (int k = 0; k < NPR; k++) lP[k * K + t] = lpr[k];
+    return v < B1 ? v : v == 5 ? (DIR == 1 ? B2 : B1) : (DIR == 3 ? B2 : B3);
 }
 
-// Corner EMF (upwind selections from the mass fluxes), transposed: scatter
-// lam_E into the flux field components and the centre EMFs.
-__global__ void __launch_bounds__(256) k_adj_emf(AdjArgs A, const double *__restrict__ F1, const double *__restrict__ F2,
-                                                 const double *__restrict__ F3, const double *__restrict__ lE,
-                                                 double *lF1, double *lF2, double *lF3, double *lEc)
-{
-    const int e = A.bs[0] + 1, f = A.bs[1] + 1, h = A.bs[2] + 1;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= (int64_t)e * f * h) return;
-    int a, b, c;
-    decode(t, e, f, h, a, b, c);
-    const int i = a + NG, j = b + NG, z = c + NG;
-    const int64_t K = A.K, si = (int64_t)A.D[1] * A.D[2], sj = A.D[2];
-    const int64_t g = cell_of(A, i, j, z);
-    auto L = [](double x) { return (double)(x <= 0.0); };
-    const double q1 = 0.25 * lE[g], q2 = 0.25 * lE[K + g], q3 = 0.25 * lE[2 * K + g];
-    const double *F1R = F1 + RHO * K, *F2R = F2 + RHO * K, *F3R = F3 + RHO * K;
-    double *lF1B2 = lF1 + B2 * K, *lF1B3 = lF1 + B3 * K, *lF2B1 = lF2 + B1 * K, *lF2B3 = lF2 + B3 * K;
-    double *lF3B1 = lF3 + B1 * K, *lF3B2 = lF3 + B2 * K;
-    double *lE1c = lEc, *lE2c = lEc + K, *lE3c = lEc + 2 * K;
-    {   // E1
-        const double aa = L(F2R[g]), bb = L(F2R[g - 1]), cc = L(F3R[g]), dd = L(F3R[g - sj]);
-        atomicAdd(&lF2B3[g], q1 * (-1. - cc - dd));
-        atomicAdd(&lF2B3[g - 1], q1 * (-1. - (1. - cc) - (1. - dd)));
-        atomicAdd(&lF3B2[g], q1 * (aa + bb + 1.));
-        atomicAdd(&lF3B2[g - sj], q1 * ((1. - aa) + (1. - bb) + 1.));
-        atomicAdd(&lE1c[g], q1 * (-aa - cc));
-        atomicAdd(&lE1c[g - sj], q1 * (-(1. - aa) - dd));
-        atomicAdd(&lE1c[g - 1], q1 * (-bb - (1. - cc)));
-        atomicAdd(&lE1c[g - sj - 1], q1 * (-(1. - bb) - (1. - dd)));
-    }
-    {   // E2
-        const double aa = L(F3R[g]), bb = L(F3R[g - si]), cc = L(F1R[g]), dd = L(F1R[g - 1]);
-        atomicAdd(&lF3B1[g], q2 * (-1. - cc - dd));
-        atomicAdd(&lF3B1[g - si], q2 * (-1. - (1. - cc) - (1. - dd)));
-        atomicAdd(&lF1B3[g], q2 * (aa + bb + 1.));
-        atomicAdd(&lF1B3[g - 1], q2 * ((1. - aa) + (1. - bb) + 1.));
-        atomicAdd(&lE2c[g], q2 * (-aa - cc));
-        atomicAdd(&lE2c[g - 1], q2 * (-(1. - aa) - dd));
-        atomicAdd(&lE2c[g - si], q2 * (-bb - (1. - cc)));
-        atomicAdd(&lE2c[g - si - 1], q2 * (-(1. - bb) - (1. - dd)));
-    }
-    {   // E3
-        const double aa = L(F2R[g]), bb = L(F2R[g - si]), cc = L(F1R[g]), dd = L(F1R[g - sj]);
-        atomicAdd(&lF2B1[g], q3 * (1. + cc + dd));
-        atomicAdd(&lF2B1[g - si], q3 * (1. + (1. - cc) + (1. - dd)));
-        atomicAdd(&lF1B2[g], q3 * (-aa - bb - 1.));
-        atomicAdd(&lF1B2[g - sj], q3 * (-(1. - aa) - (1. - bb) - 1.));
-        atomicAdd(&lE3c[g], q3 * (-aa - cc));
-        atomicAdd(&lE3c[g - sj], q3 * (-(1. - aa) - dd));
-        atomicAdd(&lE3c[g - si], q3 * (-bb - (1. - cc)));
-        atomicAdd(&lE3c[g - si - sj], q3 * (-(1. - bb) - (1. - dd)));
-    }
-}
-
-// Centre EMF of the cells [NG-1, NG+BS], transposed into lam_P (folded).
-__global__ void __launch_bounds__(256) k_adj_ecent(AdjArgs A, const double *__restrict__ p, const double *__restrict__ lEc,
-                                                   double *lP)
-{
-    const int e = A.bs[0] + 2, f = A.bs[1] + 2, h = A.bs[2] + 2;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= (int64_t)e * f * h) return;
-    int a, b, c;
-    decode(t, e, f, h, a, b, c);
-    const int i = a + NG - 1, j = b + NG - 1, z = c + NG - 1;
-    const int64_t K = A.K, g = cell_of(A, i, j, z);
-    const double lE[3] = {lEc[g], lEc[K + g], lEc[2 * K + g]};
-    if (lE[0] == 0. && lE[1] == 0. && lE[2] == 0.) return;
-    double pr[NPR], lpr[NPR];
-    for (int k = 0; k < NPR; k++) {
-        pr[k] = p[k * K + g];
-        lpr[k] = 0.;
-    }
-    const Geom<double> G = geom_at(A, CENT, (int64_t)i * A.D[1] + j);
-    ecent_vjp(pr, G, lE, lpr);
-    const int64_t fg = fold(A, i, j, z);
-    for (int k = 0; k < NPR; k++)
-        if (lpr[k] != 0.) atomicAdd(&lP[k * K + fg], lpr[k]);
-}
-
-// One face of direction DIR: HLL, the two face states and the PPM
-// reconstruction of every primitive, transposed into lam_P (folded) and the
-// normal face field into lam_ps.  Held at two waves per SIMD (a few registers
-// spilled): 1.3x faster than one wave with none spilled.
+// One face of direction DIR: the flux's adjoint (from the divergence and the EMFs),
+// HLL and the two face states, transposed into the adjoints of the face's
+// reconstructed values: X[2 v] of the lower cell's upper value (left state), X[2 v
+// + 1] of the upper cell's lower value; the normal field's goes into lps.
+// Bound by the vector units and by latency: 2579 vector instructions a face (138 us
+// of issue for the 128^3 box) at two waves per SIMD, the states of both sides being
+// live across HLL; 305 us (790 us with the fluxes formed component by component,
+// the partials of both parabolas per face and the sums by atomics).  The metric's
+// loads moved up among the parabolas spill more: 342 us.
 template <int DIR>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_adj_flux(AdjArgs A, const double *__restrict__ p, const double *__restrict__ ps,
-                                                  const double *__restrict__ lF, double *lP, double *lps)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_adj_face(AdjArgs A, const double *__restrict__ p, const double *__restrict__ ps, const double *__restrict__ w,
+           const double *__restrict__ lE, const double *__restrict__ F1, const double *__restrict__ F2,
+           const double *__restrict__ F3, double *__restrict__ X, double *__restrict__ lps)
 {
-    const int e1 = A.bs[0] + (DIR == 1 ? 1 : 2), e2 = A.bs[1] + (DIR == 2 ? 1 : 2), e3 = A.bs[2] + (DIR == 3 ? 1 : 2);
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= (int64_t)e1 * e2 * e3) return;
-    int a, b, c;
-    decode(t, e1, e2, e3, a, b, c);
-    const int i = a + (DIR == 1 ? NG : NG - 1), j = b + (DIR == 2 ? NG : NG - 1), z = c + (DIR == 3 ? NG : NG - 1);
-    const int64_t K = A.K, cell = cell_of(A, i, j, z);
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= A.n) return;
+    int i, j, z;
+    decode(A, t, i, j, z);
+    const uint32_t g = cell_of(A, i, j, z), sj = A.D[2], si = sj * A.D[1];
+    const uint32_t sd = DIR == 1 ? si : DIR == 2 ? sj : 1;
+    double y[kAdjRec][6];
+#pragma unroll
+    for (int v = 0; v < kAdjRec; v++)
+#pragma unroll
+        for (int m = 0; m < 6; m++) y[v][m] = gld(p + rec_comp<DIR>(v) * A.K, g + (m - 3) * sd);
+    const double bn = gld(ps + (DIR - 1) * A.K, g);
+    const uint32_t gm = cell_of(A, DIR == 1 ? wrap1(i - 1, A.bs[0]) : i, DIR == 2 ? wrap1(j - 1, A.bs[1]) : j,
+                                DIR == 3 ? wrap1(z - 1, A.bs[2]) : z);
+    const double rate = A.Dt / A.dx[DIR - 1];
     double lf[NPR];
     bool any = false;
-    for (int k = 0; k < NPR; k++) {
-        lf[k] = lF[k * K + cell];
-        any |= (lf[k] != 0.);
+#pragma unroll
+    for (int k = 0; k < NPR; k++)
+        if (k < B1 || k == KTOT) lf[k] = rate * (gld(w + k * A.Kw, g) - gld(w + k * A.Kw, gm));
+    lf[B1 + DIR - 1] = 0.;
+    if (DIR == 1) {
+        lf[B2] = -field_flux(lE + 2 * A.K, F2, g, si, sj);
+        lf[B3] = field_flux(lE + A.K, F3, g, si, 1);
+    } else if (DIR == 2) {
+        lf[B3] = -field_flux(lE, F3, g, sj, 1);
+        lf[B1] = field_flux(lE + 2 * A.K, F1, g, sj, si);
+    } else {
+        lf[B1] = -field_flux(lE + A.K, F1, g, 1, si);
+        lf[B2] = field_flux(lE, F2, g, 1, sj);
     }
-    if (!any) return;
-    const int64_t sd = (DIR == 1) ? (int64_t)A.D[1] * A.D[2] : (DIR == 2) ? (int64_t)A.D[2] : 1;
-    // reconstruction (primal values only: the Jacobians are formed per
-    // primitive at the end, so that they are not live across the HLL part)
-    double pl[NPR], pr[NPR];
-    for (int k = 0; k < NPR; k++) {
-        const double *q = p + k * K + cell;
-        const double xm[5] = {q[-3 * sd], q[-2 * sd], q[-sd], q[0], q[sd]};
-        const double xc[5] = {q[-2 * sd], q[-sd], q[0], q[sd], q[2 * sd]};
-        double l, r, jl[5], jr[5];
-        para_jacobian(xm, &l, &r, jl, jr);
-        pl[k] = r;
-        para_jacobian(xc, &l, &r, jl, jr);
-        pr[k] = l;
+#pragma unroll
+    for (int k = 0; k < NPR; k++) any |= lf[k] != 0.;
+    if (!any) {  // nothing reaches the face: its states may be invalid
+        for (int v = 0; v < 2 * kAdjRec; v++) gst(X + v * A.K, g, 0.);
+        return;
     }
-    const double bn = ps[(DIR - 1) * K + cell];
-    pl[B1 + DIR - 1] = bn;
-    pr[B1 + DIR - 1] = bn;
-    const int pos = DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3;
-    const Geom<double> G = geom_at(A, pos, (int64_t)i * A.D[1] + j);
-    // primal HLL
-    double FL[NPR], UL[NPR], FR[NPR], UR[NPR], vxl = 0., vnl = 0., vxr = 0., vnr = 0., dum;
-    {
-        State<double> q;
-        get_state(pl, G, q);
-        primtoflux(pl, q, DIR, G, A.gam, FL, &vxl, &vnl);
-        primtoflux(pl, q, 0, G, A.gam, UL, &dum, &dum);
-        get_state(pr, G, q);
-        primtoflux(pr, q, DIR, G, A.gam, FR, &vxr, &vnr);
-        primtoflux(pr, q, 0, G, A.gam, UR, &dum, &dum);
+    double pl[NPR], pr[NPR], lpl[NPR], lpr[NPR], dum;
+    pl[KTOT] = pr[KTOT] = 0.;
+#pragma unroll
+    for (int v = 0; v < kAdjRec; v++) {
+        const int k = rec_comp<DIR>(v);
+        para(y[v][0], y[v][1], y[v][2], y[v][3], y[v][4], dum, pl[k]);
+        para(y[v][1], y[v][2], y[v][3], y[v][4], y[v][5], pr[k], dum);
     }
-    const double m1 = mymax(0., vxl), cmax = fabs(mymax(m1, vxr));
-    const double n1 = mymax(0., -vnl), cmin = fabs(mymax(n1, -vnr));
-    const double den = cmax + cmin + kSMALL;
-    // reverse of F = (cmax FL + cmin FR - cmax cmin (UR - UL)) / den
-    double lFL[NPR], lFR[NPR], lUL[NPR], lUR[NPR], lcmax = 0., lcmin = 0.;
-    for (int k = 0; k < NPR; k++) {
-        const double F = (cmax * FL[k] + cmin * FR[k] - cmax * cmin * (UR[k] - UL[k])) / den;
-        lFL[k] = lf[k] * cmax / den;
-        lFR[k] = lf[k] * cmin / den;
-        lUR[k] = -lf[k] * cmax * cmin / den;
-        lUL[k] = -lUR[k];
-        lcmax += lf[k] * ((FL[k] - cmin * (UR[k] - UL[k])) - F) / den;
-        lcmin += lf[k] * ((FR[k] - cmax * (UR[k] - UL[k])) - F) / den;
+    pl[B1 + DIR - 1] = pr[B1 + DIR - 1] = bn;
+    const Geom<double> G = geom_at(A, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (uint32_t)i * A.D[1] + j);
+    hll_vjp(pl, pr, G, DIR, A.gam, lf, lpl, lpr);
+    double *n = lps + (DIR - 1) * A.Kg;
+    gst(n, g, gld(n, g) + (lpl[B1 + DIR - 1] + lpr[B1 + DIR - 1]));
+#pragma unroll
+    for (int v = 0; v < kAdjRec; v++) {
+        gst(X + 2 * v * A.K, g, lpl[rec_comp<DIR>(v)]);
+        gst(X + (2 * v + 1) * A.K, g, lpr[rec_comp<DIR>(v)]);
     }
-    double lvxl = 0., lvxr = 0., lvnl = 0., lvnr = 0.;
-    if (m1 > vxr) { if (!(0. > vxl)) lvxl = lcmax; }
-    else lvxr = lcmax;
-    if (n1 > -vnr) { if (!(0. > -vnl)) lvnl = -lcmin; }
-    else lvnr = -lcmin;
-    double lpl[NPR], lpr[NPR];
-    for (int k = 0; k < NPR; k++) lpl[k] = lpr[k] = 0.;
-    face_state_vjp(pl, G, DIR, A.gam, lFL, lUL, lvxl, lvnl, lpl);
-    face_state_vjp(pr, G, DIR, A.gam, lFR, lUR, lvxr, lvnr, lpr);
-    // normal face field
-    {
-        const double v = lpl[B1 + DIR - 1] + lpr[B1 + DIR - 1];
-        if (v != 0.) atomicAdd(&lps[(DIR - 1) * K + fold(A, i, j, z)], v);
-        lpl[B1 + DIR - 1] = lpr[B1 + DIR - 1] = 0.;
-    }
-    // reconstruction: pl from cells c-3..c+1, pr from c-2..c+2 along DIR
-    int64_t fg[6];
-    for (int m = -3; m <= 2; m++)
-        fg[m + 3] = fold(A, i + (DIR == 1 ? m : 0), j + (DIR == 2 ? m : 0), z + (DIR == 3 ? m : 0));
-    for (int k = 0; k < NPR; k++) {
-        if (lpl[k] == 0. && lpr[k] == 0.) continue;
-        const double *q = p + k * K + cell;
-        const double xm[5] = {q[-3 * sd], q[-2 * sd], q[-sd], q[0], q[sd]};
-        const double xc[5] = {q[-2 * sd], q[-sd], q[0], q[sd], q[2 * sd]};
-        double l, r, jl[5], Jr[5], Jl[5];
-        para_jacobian(xm, &l, &r, jl, Jr);
-        para_jacobian(xc, &l, &r, Jl, jl);
-        for (int m = -3; m <= 2; m++) {
-            double v = 0.;
-            if (m <= 1) v += lpl[k] * Jr[m + 3];
-            if (m >= -2) v += lpr[k] * Jl[m + 2];
-            if (v != 0.) atomicAdd(&lP[k * K + fg[m + 3]], v);
+}
+
+// Reconstruction along x1 or x2, reverse: adds to lP what the face adjoints X of
+// k_adj_face give through each cell's parabola, one component per blockIdx.y.  A
+// thread takes `seg` cells of a line along DIR (lanes along z) and the two cells on
+// either side, with the five sums that a parabola's stencil reaches in registers.
+// Bound by memory: 128^3, 139 us for 0.6 GB (4.4 TB/s).  Tiles with the sums in LDS
+// (28 cells of 16 z-lanes) took 194 us, segments of 16 cells with their loads not
+// sent ahead 173.
+template <int DIR>
+__global__ void __launch_bounds__(256) k_adj_rec(AdjArgs A, const double *__restrict__ p, const double *__restrict__ X,
+                                                 double *__restrict__ lP, int seg, int nseg)
+{
+    const int d = DIR - 1, o = 1 - d;  // this direction, the other of x1 and x2
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= nseg * A.bs[o] * A.bs[2]) return;
+    int sg, a, z;
+    region_index(t, A.bs[o], A.bs[2], sg, a, z);
+    const int v = blockIdx.y, k = rec_comp<DIR>(v), n = A.bs[d];
+    const double *q = p + k * A.K, *Xl = X + 2 * v * A.K, *Xr = Xl + A.K;
+    double *out = lP + k * A.Kg;
+    const uint32_t sj = A.D[2], si = sj * A.D[1], sd = DIR == 1 ? si : sj;
+    const uint32_t base = cell_of(A, DIR == 1 ? NG : a + NG, DIR == 1 ? a + NG : NG, z + NG);
+    const int c0 = sg * seg, len = n - c0 < seg ? n - c0 : seg;
+    auto at = [&](int c) { return base + (c < 0 ? c + n : c >= n ? c - n : c) * sd; };
+    double x[5], r[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+    for (int s = 0; s < 5; s++) x[s] = gld(q, at(c0 + s - 4));
+    double ll = gld(Xr, at(c0 - 2)), lr = gld(Xl, at(c0 - 1));
+#pragma unroll 2
+    for (int m = -2; m < len + 2; m++) {
+        // the next cell's values are on their way while this one's are worked on
+        const double xn = gld(q, at(c0 + m + 3)), lln = gld(Xr, at(c0 + m + 1)), lrn = gld(Xl, at(c0 + m + 2));
+        if (ll != 0. || lr != 0.) para_vjp(x, ll, lr, r);
+        if (m >= 2) {
+            const uint32_t g = base + (c0 + m - 2) * sd;
+            gst(out, g, gld(out, g) + r[0]);
         }
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            r[s] = r[s + 1];
+            x[s] = x[s + 1];
+        }
+        r[4] = 0.;
+        x[4] = xn;
+        ll = lln;
+        lr = lrn;
     }
+}
+
+// The same along x3, a block taking `nrow` z-rows as a whole (len = bs3, halo = 0),
+// or a window of len - 4 cells of one row with two on either side (halo = 2) where
+// a row is longer than a block.
+// Bound by memory: 128^3, 141 us (groups of 47 lanes with the sums by shuffles: 180).
+constexpr int kAdjRow3 = 256;
+__global__ void __launch_bounds__(kAdjRow3) k_adj_rec3(AdjArgs A, const double *__restrict__ p,
+                                                       const double *__restrict__ X, double *__restrict__ lP, int len,
+                                                       int nrow, int nwin, int halo)
+{
+    __shared__ double sh[4][kAdjRow3];
+    const int t = threadIdx.x, sub = t / len, l = t - sub * len;
+    const int row = blockIdx.x * nrow + sub;  // (i, j, window of the row)
+    const bool live = sub < nrow && row < A.bs[0] * A.bs[1] * nwin;
+    int i = 0, j = 0, win = 0;
+    if (live) region_index(row, A.bs[1], nwin, i, j, win);
+    const int v = blockIdx.y, k = rec_comp<3>(v);
+    const int o = win * (len - 2 * halo) + l - halo;
+    const int z = wrap1(NG + o, A.bs[2]);
+    const uint32_t g = cell_of(A, i + NG, j + NG, z), gn = z + 1 == NG + A.bs[2] ? g + 1 - A.bs[2] : g + 1;
+    double x[5], r[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+    for (int s = 0; s < 5; s++) x[s] = gld(p + k * A.K, g + s - 2);
+    const double ll = gld(X + (2 * v + 1) * A.K, g), lr = gld(X + 2 * v * A.K, gn);
+    if (ll != 0. || lr != 0.) para_vjp(x, ll, lr, r);
+    sh[0][t] = r[0];
+    sh[1][t] = r[1];
+    sh[2][t] = r[3];
+    sh[3][t] = r[4];
+    __syncthreads();
+    if (!live || l < halo || l >= len - halo || o >= A.bs[2]) return;
+    // lanes of the cells at -2 .. 2: the row is periodic where the block holds all of it
+    auto at = [&](int m) { const int q = l + m; return sub * len + (q < 0 ? q + len : q >= len ? q - len : q); };
+    double sum = r[2] + (sh[3][at(-2)] + sh[2][at(-1)]);
+    sum += sh[1][at(1)] + sh[0][at(2)];
+    double *out = lP + k * A.Kg;
+    gst(out, g, gld(out, g) + sum);
 }
 
 // ---------------------------------------------------------------------------
 static inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-// Zeroes n doubles of each of a, b and c (the accumulators of the adjoint).  A
-// kernel rather than hipMemsetAsync, so that a caller may capture the adjoint
-// in a HIP graph.
-__global__ void __launch_bounds__(256) k_adj_zero3(double *a, double *b, double *c, int64_t n)
-{
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    a[t] = 0.;
-    b[t] = 0.;
-    c[t] = 0.;
-}
-
 void launch_adjoint(const KParams &P, const BlockDev &B, double Dt, const double *p, const double *ps,
-                    const double *F1, const double *F2, const double *F3, const double *w, double *lP, double *lps,
-                    double *lpsf, double *lE, double *lEc, double *lF1, double *lF2, double *lF3, hipStream_t s)
+                    const double *F1, const double *F2, const double *F3, const double *w, int64_t Kw, double *lP,
+                    double *lps, int64_t Kg, double *lE, double *X, hipStream_t s)
 {
     AdjArgs A;
     for (int k = 0; k < 3; k++) {
@@ -399,7 +336,10 @@ void launch_adjoint(const KParams &P, const BlockDev &B, double Dt, const double
         A.bs[k] = B.bs[k];
         A.dx[k] = B.dx[k];
     }
+    A.n = B.bs[0] * B.bs[1] * B.bs[2];
     A.K = B.ks;
+    A.Kw = Kw;
+    A.Kg = Kg;
     A.Dt = Dt;
     A.gam = P.gam;
     A.kcol = B.kcol;
@@ -407,21 +347,30 @@ void launch_adjoint(const KParams &P, const BlockDev &B, double Dt, const double
     A.gcon = P.gcon + B.moff * NPOS * 10;
     A.gdet = P.gdet + B.moff * NPOS;
     const int64_t N = (int64_t)A.D[0] * A.D[1] * A.D[2];
-    hipLaunchKernelGGL(k_adj_zero3, g1(3 * A.K), dim3(256), 0, s, lps, lE, lEc, 3 * A.K);
-    hipLaunchKernelGGL(k_adj_seed, g1(N), dim3(256), 0, s, A, w, lpsf);
-    hipLaunchKernelGGL(k_adj_ct, g1(N), dim3(256), 0, s, A, lpsf, lE, lps);
-    hipLaunchKernelGGL(k_adj_div, g1(N), dim3(256), 0, s, A, w, lF1, lF2, lF3);
-    hipLaunchKernelGGL(k_adj_u0, g1(N), dim3(256), 0, s, A, p, w, lP);
-    const int64_t nc = (int64_t)(A.bs[0] + 1) * (A.bs[1] + 1) * (A.bs[2] + 1);
-    hipLaunchKernelGGL(k_adj_emf, g1(nc), dim3(256), 0, s, A, F1, F2, F3, lE, lF1, lF2, lF3, lEc);
-    const int64_t ne = (int64_t)(A.bs[0] + 2) * (A.bs[1] + 2) * (A.bs[2] + 2);
-    hipLaunchKernelGGL(k_adj_ecent, g1(ne), dim3(256), 0, s, A, p, lEc, lP);
-    const int64_t f1 = (int64_t)(A.bs[0] + 1) * (A.bs[1] + 2) * (A.bs[2] + 2);
-    const int64_t f2 = (int64_t)(A.bs[0] + 2) * (A.bs[1] + 1) * (A.bs[2] + 2);
-    const int64_t f3 = (int64_t)(A.bs[0] + 2) * (A.bs[1] + 2) * (A.bs[2] + 1);
-    hipLaunchKernelGGL(k_adj_flux<1>, g1(f1), dim3(256), 0, s, A, p, ps, lF1, lP, lps);
-    hipLaunchKernelGGL(k_adj_flux<2>, g1(f2), dim3(256), 0, s, A, p, ps, lF2, lP, lps);
-    hipLaunchKernelGGL(k_adj_flux<3>, g1(f3), dim3(256), 0, s, A, p, ps, lF3, lP, lps);
+    // mass fluxes only: RHO is the first component
+    hipLaunchKernelGGL(k_adj_edge, g1(N), dim3(256), 0, s, A, w, lE, lps);
+    hipLaunchKernelGGL(k_adj_cell, g1(N), dim3(256), 0, s, A, p, w, lE, F1, F2, F3, lP);
+    // the longest segments that still give the chip 4 wavefronts a SIMD, from 32
+    // cells (4 cells of overlap in 32) down to 4: on 20x27x14 cells segments of 16
+    // take 30 us, of 4 8 us; on 128^3 16 to 32 are alike
+    int seg = 32;
+    while (seg > 4 && (int64_t)kAdjRec * A.n / seg < 256 * 16 * 64) seg /= 2;
+    int nseg[2];
+    dim3 grec[2];
+    for (int d = 0; d < 2; d++) {
+        nseg[d] = (A.bs[d] + seg - 1) / seg;
+        grec[d] = dim3((unsigned)(((int64_t)nseg[d] * A.bs[1 - d] * A.bs[2] + 255) / 256), kAdjRec);
+    }
+    hipLaunchKernelGGL(k_adj_face<1>, g1(A.n), dim3(256), 0, s, A, p, ps, w, lE, F1, F2, F3, X, lps);
+    hipLaunchKernelGGL(k_adj_rec<1>, grec[0], dim3(256), 0, s, A, p, X, lP, seg, nseg[0]);
+    hipLaunchKernelGGL(k_adj_face<2>, g1(A.n), dim3(256), 0, s, A, p, ps, w, lE, F1, F2, F3, X, lps);
+    hipLaunchKernelGGL(k_adj_rec<2>, grec[1], dim3(256), 0, s, A, p, X, lP, seg, nseg[1]);
+    hipLaunchKernelGGL(k_adj_face<3>, g1(A.n), dim3(256), 0, s, A, p, ps, w, lE, F1, F2, F3, X, lps);
+    const int nwin = A.bs[2] <= kAdjRow3 ? 1 : (A.bs[2] + kAdjRow3 - 5) / (kAdjRow3 - 4), halo = nwin > 1 ? 2 : 0;
+    const int len = (A.bs[2] + nwin - 1) / nwin + 2 * halo, nrow = kAdjRow3 / len;
+    const int64_t nr = (int64_t)A.bs[0] * A.bs[1] * nwin;
+    hipLaunchKernelGGL(k_adj_rec3, dim3((unsigned)((nr + nrow - 1) / nrow), kAdjRec), dim3((nrow * len + 63) / 64 * 64), 0,
+                       s, A, p, X, lP, len, nrow, nwin, halo);
 }
 
 }  // namespace hamr

@@ -110,8 +110,7 @@ struct hamr_ctx {
     int las_graph_maxtl = 0;
     int prec = HAMR_PREC_FP64;     // arithmetic of reconstruction, fluxes and EMFs
     // adjoint scratch (allocated by the first adjoint call)
-    double *aw = nullptr, *alP = nullptr, *alps = nullptr, *alpsf = nullptr, *alE = nullptr, *alEc = nullptr;
-    double *alF[3] = {nullptr, nullptr, nullptr};
+    double *aw = nullptr, *alP = nullptr, *alps = nullptr, *alE = nullptr, *alX = nullptr;
     std::vector<void *> allocs;
     void *stage = nullptr;         // pinned host staging of whole-array copies
     size_t stage_bytes = 0;
@@ -2303,13 +2302,15 @@ int hamr_stage_forward(hamr_ctx *c, double Dt)
     return check_launch(c, "hamr_stage_forward");
 }
 
-// The adjoint's work arrays: weights, lambda of P, ps, the updated face field,
-// the corner and centre EMFs and the three fluxes (57 doubles per cell of the
-// padded slab).
+// The adjoint's work arrays: weights, lambda of P, ps, the corner EMFs and the
+// reconstructed face states of one direction.  They take 38 doubles per cell of
+// the padded slab; hamr_stage_adjoint_dev_noalloc accepts the boxes it is
+// documented for, 57 doubles per cell of the scratch.
 struct AdjBufs {
-    double *w, *lP, *lps, *lpsf, *lE, *lEc, *lF[3];
+    double *w, *lP, *lps, *lE, *X;
 };
-constexpr int64_t kAdjDoublesPerCell = NPR + NPR + 3 + 3 + 3 + 3 + 3 * NPR;
+constexpr int64_t kAdjDoublesPerCell = 57;
+static_assert(NPR + NPR + 3 + 3 + kAdjXSlabs <= kAdjDoublesPerCell, "the adjoint's work arrays fit the scratch");
 
 // w, grad_p, grad_ps: pointers of `kind` (host or device), unpadded layout.
 static int stage_adjoint(hamr_ctx *c, double Dt, const double *w, double *gp, double *gps, hipMemcpyKind in,
@@ -2331,8 +2332,8 @@ static int stage_adjoint(hamr_ctx *c, double Dt, const double *w, double *gp, do
     for (int dir = 1; dir <= 3; dir++)
         launch_flux(c->P, dir, flux_block_launch(c, dir, 0), c->p, c->ps, c->F[dir - 1], nullptr,
                     HAMR_PREC_FP64, c->s);
-    launch_adjoint(c->P, B, Dt, c->p, c->ps, c->F[0], c->F[1], c->F[2], A.w, A.lP, A.lps, A.lpsf, A.lE, A.lEc,
-                   A.lF[0], A.lF[1], A.lF[2], c->s);
+    launch_adjoint(c->P, B, Dt, c->p, c->ps, (const double *)c->F[0], (const double *)c->F[1],
+                   (const double *)c->F[2], A.w, B.ks, A.lP, A.lps, B.ks, A.lE, A.X, c->s);
     if (check_launch(c, "hamr_stage_adjoint")) return -1;
     double *sp = hout ? (double *)c->stage : gp, *sps = hout ? (double *)c->stage + NPR * N : gps;
     if (gp)
@@ -2362,13 +2363,12 @@ static int adjoint_ok(hamr_ctx *c, const double *w, const char *what)
 static int adjoint_bufs(hamr_ctx *c, AdjBufs &A)
 {
     const size_t K = (size_t)c->blocks[0].ks;
-    if (!c->aw) {
+    if (!c->alX) {
         if (dalloc(c, &c->aw, NPR * K) || dalloc(c, &c->alP, NPR * K) || dalloc(c, &c->alps, 3 * K) ||
-            dalloc(c, &c->alpsf, 3 * K) || dalloc(c, &c->alE, 3 * K) || dalloc(c, &c->alEc, 3 * K) ||
-            dalloc(c, &c->alF[0], NPR * K) || dalloc(c, &c->alF[1], NPR * K) || dalloc(c, &c->alF[2], NPR * K))
+            dalloc(c, &c->alE, 3 * K) || dalloc(c, &c->alX, kAdjXSlabs * K))
             return -1;
     }
-    A = AdjBufs{c->aw, c->alP, c->alps, c->alpsf, c->alE, c->alEc, {c->alF[0], c->alF[1], c->alF[2]}};
+    A = AdjBufs{c->aw, c->alP, c->alps, c->alE, c->alX};
     return 0;
 }
 
@@ -2387,8 +2387,7 @@ int hamr_stage_adjoint_dev(hamr_ctx *c, double Dt, const double *w, double *gp, 
 }
 
 // The work arrays carved from this device's `scratch` (c->scratch, resolved at
-// hamr_create): no allocation.  Every accumulator is cleared by a fill kernel
-// inside launch_adjoint; the rest is written before it is read.
+// hamr_create): no allocation.  Everything in them is written before it is read.
 int hamr_stage_adjoint_dev_noalloc(hamr_ctx *c, double Dt, const double *w, double *gp, double *gps)
 {
     if (adjoint_ok(c, w, "hamr_stage_adjoint_dev_noalloc")) return -1;
@@ -2409,10 +2408,8 @@ int hamr_stage_adjoint_dev_noalloc(hamr_ctx *c, double Dt, const double *w, doub
     A.w = take(NPR);
     A.lP = take(NPR);
     A.lps = take(3);
-    A.lpsf = take(3);
     A.lE = take(3);
-    A.lEc = take(3);
-    for (int d = 0; d < 3; d++) A.lF[d] = take(NPR);
+    A.X = take(kAdjXSlabs);
     return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice, A);
 }
 

@@ -162,11 +162,13 @@ void launch_update_part(const KParams &P, int part, const Launch &L, int full, d
                         const double *psf, const void *F1, const void *F2, const void *F3, int *pflag, int *failcnt,
                         int mixed, hipStream_t s);
 // Adjoint of one forward stage of a single periodic flat block (FP64): from the
-// weights w of U' (9 slabs) to lP (9 slabs, dL/dP) and lps (3 slabs, dL/d face
-// field); F1-F3 are the stage's fluxes; lpsf, lE, lEc, lF1-lF3 are scratch.
+// weights w of U' (9 slabs of Kw) to lP (9 slabs of Kg, dL/dP) and lps (3 slabs
+// of Kg, dL/d face field); F1-F3 are the stage's fluxes; lE (3 slabs) and X
+// (kAdjXSlabs) are scratch.
+constexpr int kAdjXSlabs = 14;
 void launch_adjoint(const KParams &P, const BlockDev &B, double Dt, const double *p, const double *ps,
-                    const double *F1, const double *F2, const double *F3, const double *w, double *lP, double *lps,
-                    double *lpsf, double *lE, double *lEc, double *lF1, double *lF2, double *lF3, hipStream_t s);
+                    const double *F1, const double *F2, const double *F3, const double *w, int64_t Kw, double *lP,
+                    double *lps, int64_t Kg, double *lE, double *X, hipStream_t s);
 
 // Ghost fill of direction dir (1 or 2) of a multi-level set over the faces whose
 // kind is FK_COPY, FK_OUTFLOW or FK_POLE (FK_AMR faces are left to the exchange
