@@ -185,6 +185,8 @@ def load_library(path=None):
         "hamr_stage_forward": [ctxp, C.c_double],
         "hamr_stage_adjoint": [ctxp, C.c_double, _dp, _dp, _dp],
         "hamr_stage_adjoint_dev": [ctxp, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p],
+        "hamr_stage_forward_dev": [ctxp, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p],
+        "hamr_stage_grad_dev": [ctxp, C.c_double] + [C.c_void_p] * 5,
         "hamr_stage_adjoint_dev_noalloc": [ctxp, C.c_double, C.c_void_p, C.c_void_p, C.c_void_p],
         "hamr_create_amr": [D, C.POINTER(AmrDescC), C.POINTER(ctxp)],
         "hamr_desc_amr": [D, C.POINTER(AmrDescC), _llp, _ip, _ip, _ip],
@@ -616,6 +618,16 @@ class Context:
     def stage_adjoint_dev(self, Dt, w_ptr, gp_ptr, gps_ptr):
         self._chk(self.L.hamr_stage_adjoint_dev(self.h, Dt, C.c_void_p(w_ptr), C.c_void_p(gp_ptr),
                                                 C.c_void_p(gps_ptr)), "hamr_stage_adjoint_dev")
+
+    def stage_forward_dev(self, Dt, p_ptr, ps_ptr, u_ptr):
+        """The stage from device arrays (unpadded layout); ghosts of U' are zero."""
+        self._chk(self.L.hamr_stage_forward_dev(self.h, Dt, C.c_void_p(p_ptr), C.c_void_p(ps_ptr),
+                                                C.c_void_p(u_ptr)), "hamr_stage_forward_dev")
+
+    def stage_grad_dev(self, Dt, p_ptr, ps_ptr, w_ptr, gp_ptr, gps_ptr):
+        """stage_adjoint_dev of the state in p_ptr, ps_ptr."""
+        self._chk(self.L.hamr_stage_grad_dev(self.h, Dt, *map(C.c_void_p, (p_ptr, ps_ptr, w_ptr, gp_ptr, gps_ptr))),
+                  "hamr_stage_grad_dev")
 
     def stage_adjoint_dev_noalloc(self, Dt, w_ptr, gp_ptr, gps_ptr):
         """stage_adjoint_dev with the work arrays in the library's static device

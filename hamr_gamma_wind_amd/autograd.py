@@ -4,20 +4,14 @@ hand-written adjoint (libhamr_hip.so).
 torch holds the device memory; the library computes on its own stream.  The
 forward copies the primitives and face fields from the given device tensors
 into the context, runs the stage and returns U' (interior cells; ghost cells
-are zero).  The backward runs the adjoint for the incoming gradient of U' and
-returns dL/dP and dL/d(face field).  Both synchronise torch's current stream
-before the library reads torch memory and the library's stream before torch
-reads its results.
+are zero).  The backward runs the adjoint for the incoming gradient of U', which
+the library reads in place, and returns dL/dP and dL/d(face field).  Both
+synchronise torch's current stream before the library reads torch memory, and the
+library's stream has finished when they return.
 """
 import torch
 
-from . import HAMR_P, HAMR_PS, HAMR_UNEW, NG, HamrError
-
-
-def _interior_mask(shape, device):
-    m = torch.zeros(shape, dtype=torch.float64, device=device)
-    m[..., NG:-NG, NG:-NG, NG:-NG] = 1.0
-    return m
+from . import HamrError
 
 
 class Stage(torch.autograd.Function):
@@ -31,12 +25,8 @@ class Stage(torch.autograd.Function):
             if tuple(t.shape) != (hctx.nblk, nc) + tuple(hctx.D):
                 raise HamrError("Stage: tensor shape does not match the context layout")
         torch.cuda.current_stream().synchronize()
-        hctx.set_dev(HAMR_P, P.data_ptr())
-        hctx.set_dev(HAMR_PS, PS.data_ptr())
-        hctx.stage_forward(Dt)
         U = torch.empty_like(P)
-        hctx.get_dev(HAMR_UNEW, U.data_ptr())
-        U = U * _interior_mask(U.shape, U.device)
+        hctx.stage_forward_dev(Dt, P.data_ptr(), PS.data_ptr(), U.data_ptr())
         ctx.hctx = hctx
         ctx.Dt = Dt
         ctx.save_for_backward(P, PS)
@@ -46,13 +36,11 @@ class Stage(torch.autograd.Function):
     def backward(ctx, gU):
         P, PS = ctx.saved_tensors
         hctx = ctx.hctx
-        w = (gU * _interior_mask(gU.shape, gU.device)).contiguous()
+        w = gU.contiguous()  # the weights of ghost cells are not read
         gP = torch.empty_like(P)
         gPS = torch.empty_like(PS)
         torch.cuda.current_stream().synchronize()
-        hctx.set_dev(HAMR_P, P.data_ptr())
-        hctx.set_dev(HAMR_PS, PS.data_ptr())
-        hctx.stage_adjoint_dev(ctx.Dt, w.data_ptr(), gP.data_ptr(), gPS.data_ptr())
+        hctx.stage_grad_dev(ctx.Dt, P.data_ptr(), PS.data_ptr(), w.data_ptr(), gP.data_ptr(), gPS.data_ptr())
         return gP, gPS, None, None
 
 

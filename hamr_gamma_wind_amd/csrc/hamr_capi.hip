@@ -109,7 +109,7 @@ struct hamr_ctx {
     hipGraphExec_t las_graph = nullptr;  // one time-level cycle (hamr_step_las_graph)
     int las_graph_maxtl = 0;
     int prec = HAMR_PREC_FP64;     // arithmetic of reconstruction, fluxes and EMFs
-    // adjoint scratch (allocated by the first adjoint call)
+    // adjoint scratch (each allocated by the first adjoint call that needs it)
     double *aw = nullptr, *alP = nullptr, *alps = nullptr, *alE = nullptr, *alX = nullptr;
     std::vector<void *> allocs;
     void *stage = nullptr;         // pinned host staging of whole-array copies
@@ -2312,20 +2312,55 @@ struct AdjBufs {
 constexpr int64_t kAdjDoublesPerCell = 57;
 static_assert(NPR + NPR + 3 + 3 + kAdjXSlabs <= kAdjDoublesPerCell, "the adjoint's work arrays fit the scratch");
 
-// w, grad_p, grad_ps: pointers of `kind` (host or device), unpadded layout.
+// Whether kernels of the context's device can use ptr as it is: device memory of
+// that device (not another device's, host or managed memory).
+static bool on_device(const hamr_ctx *c, const void *ptr)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == c->device;
+}
+
+// Which of the caller's buffers the adjoint reads and writes in place: device
+// buffers of this device, the gradients only where nothing overlaps them.  The
+// rest passes through the work arrays.
+struct AdjDirect {
+    bool w, g;
+};
+static AdjDirect adjoint_direct(const hamr_ctx *c, const double *w, const double *gp, const double *gps)
+{
+    const int64_t N = ncell_of(c->blocks[0]);
+    auto apart = [](const double *a, int64_t na, const double *b, int64_t nb) {
+        return !a || !b || (uintptr_t)(a + na) <= (uintptr_t)b || (uintptr_t)(b + nb) <= (uintptr_t)a;
+    };
+    AdjDirect d;
+    d.w = on_device(c, w);
+    d.g = gp && gps && on_device(c, gp) && on_device(c, gps) && apart(gp, NPR * N, gps, 3 * N) &&
+          apart(gp, NPR * N, w, NPR * N) && apart(gps, 3 * N, w, NPR * N);
+    return d;
+}
+
+// w, gp, gps: pointers of `kind` (host or device), unpadded layout; `d` says which
+// are used in place.  Copying 21 slabs took 195 us of the 128^3 box's gradient.
 static int stage_adjoint(hamr_ctx *c, double Dt, const double *w, double *gp, double *gps, hipMemcpyKind in,
-                         hipMemcpyKind out, const AdjBufs &A)
+                         hipMemcpyKind out, AdjDirect d, const AdjBufs &A)
 {
     const BlockDev &B = c->blocks[0];
     const size_t K = (size_t)B.ks, N = (size_t)ncell_of(B);
-    HIPCHK(c, hipStreamSynchronize(c->s));
     // host buffers pass through the pinned staging buffer (w in, then the gradients out)
     const bool hin = in == hipMemcpyHostToDevice, hout = out == hipMemcpyDeviceToHost;
-    if ((hin || hout) && stage_reserve(c, (NPR + 3) * N * sizeof(double))) return -1;
+    if (hin || hout) {
+        HIPCHK(c, hipStreamSynchronize(c->s));
+        if (stage_reserve(c, (NPR + 3) * N * sizeof(double))) return -1;
+    }
     double *sw = (double *)c->stage;
     if (hin) std::memcpy(sw, w, NPR * N * sizeof(double));
-    HIPCHK(c, hipMemcpy2DAsync(A.w, K * sizeof(double), hin ? sw : w, N * sizeof(double), N * sizeof(double), NPR,
-                               in, c->s));
+    if (!d.w)
+        HIPCHK(c, hipMemcpy2DAsync(A.w, K * sizeof(double), hin ? sw : w, N * sizeof(double), N * sizeof(double), NPR,
+                                   in, c->s));
     if (hin) HIPCHK(c, hipStreamSynchronize(c->s));
     // the fluxes of the stage (their mass-flux signs select the EMF upwinding)
     bound_all(c, c->p, c->ps);
@@ -2333,12 +2368,13 @@ static int stage_adjoint(hamr_ctx *c, double Dt, const double *w, double *gp, do
         launch_flux(c->P, dir, flux_block_launch(c, dir, 0), c->p, c->ps, c->F[dir - 1], nullptr,
                     HAMR_PREC_FP64, c->s);
     launch_adjoint(c->P, B, Dt, c->p, c->ps, (const double *)c->F[0], (const double *)c->F[1],
-                   (const double *)c->F[2], A.w, B.ks, A.lP, A.lps, B.ks, A.lE, A.X, c->s);
+                   (const double *)c->F[2], d.w ? w : A.w, d.w ? (int64_t)N : B.ks, d.g ? gp : A.lP,
+                   d.g ? gps : A.lps, d.g ? (int64_t)N : B.ks, A.lE, A.X, c->s);
     if (check_launch(c, "hamr_stage_adjoint")) return -1;
     double *sp = hout ? (double *)c->stage : gp, *sps = hout ? (double *)c->stage + NPR * N : gps;
-    if (gp)
+    if (gp && !d.g)
         HIPCHK(c, hipMemcpy2DAsync(sp, N * sizeof(double), A.lP, K * sizeof(double), N * sizeof(double), NPR, out, c->s));
-    if (gps)
+    if (gps && !d.g)
         HIPCHK(c, hipMemcpy2DAsync(sps, N * sizeof(double), A.lps, K * sizeof(double), N * sizeof(double), 3, out, c->s));
     HIPCHK(c, hipStreamSynchronize(c->s));
     if (hout) {
@@ -2358,16 +2394,15 @@ static int adjoint_ok(hamr_ctx *c, const double *w, const char *what)
     return 0;
 }
 
-// The work arrays of the allocating entry points: the context's own, allocated
-// by the first adjoint call.
-static int adjoint_bufs(hamr_ctx *c, AdjBufs &A)
+// The work arrays of the allocating entry points: the context's own, each
+// allocated by the first adjoint call that needs it.
+static int adjoint_bufs(hamr_ctx *c, AdjDirect d, AdjBufs &A)
 {
     const size_t K = (size_t)c->blocks[0].ks;
-    if (!c->alX) {
-        if (dalloc(c, &c->aw, NPR * K) || dalloc(c, &c->alP, NPR * K) || dalloc(c, &c->alps, 3 * K) ||
-            dalloc(c, &c->alE, 3 * K) || dalloc(c, &c->alX, kAdjXSlabs * K))
-            return -1;
-    }
+    auto need = [&](double **q, size_t ncomp) { return *q ? 0 : dalloc(c, q, ncomp * K); };
+    if (need(&c->alE, 3) || need(&c->alX, kAdjXSlabs) || (!d.w && need(&c->aw, NPR)) ||
+        (!d.g && (need(&c->alP, NPR) || need(&c->alps, 3))))
+        return -1;
     A = AdjBufs{c->aw, c->alP, c->alps, c->alE, c->alX};
     return 0;
 }
@@ -2375,15 +2410,61 @@ static int adjoint_bufs(hamr_ctx *c, AdjBufs &A)
 int hamr_stage_adjoint(hamr_ctx *c, double Dt, const double *w, double *gp, double *gps)
 {
     AdjBufs A;
-    if (adjoint_ok(c, w, "hamr_stage_adjoint") || adjoint_bufs(c, A)) return -1;
-    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyHostToDevice, hipMemcpyDeviceToHost, A);
+    const AdjDirect none{false, false};
+    if (adjoint_ok(c, w, "hamr_stage_adjoint") || adjoint_bufs(c, none, A)) return -1;
+    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyHostToDevice, hipMemcpyDeviceToHost, none, A);
 }
 
 int hamr_stage_adjoint_dev(hamr_ctx *c, double Dt, const double *w, double *gp, double *gps)
 {
     AdjBufs A;
-    if (adjoint_ok(c, w, "hamr_stage_adjoint_dev") || adjoint_bufs(c, A)) return -1;
-    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice, A);
+    if (adjoint_ok(c, w, "hamr_stage_adjoint_dev")) return -1;
+    const AdjDirect d = adjoint_direct(c, w, gp, gps);
+    if (adjoint_bufs(c, d, A)) return -1;
+    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice, d, A);
+}
+
+// p and ps of every block of a uniform grid from the caller's unpadded arrays, in
+// one launch where they are this device's memory.
+static int state_in(hamr_ctx *c, const double *p, const double *ps)
+{
+    if (on_device(c, p) && on_device(c, ps)) {
+        launch_box_in(c->P, nblk_of(c), c->blocks[0], p, ps, c->p, c->ps, c->s);
+        return 0;
+    }
+    return copy_array(c, HAMR_P, const_cast<double *>(p), 1, hipMemcpyDeviceToDevice) ||
+           copy_array(c, HAMR_PS, const_cast<double *>(ps), 1, hipMemcpyDeviceToDevice);
+}
+
+int hamr_stage_forward_dev(hamr_ctx *c, double Dt, const double *p, const double *ps, double *u)
+{
+    if (!c) return -1;
+    if (!p || !ps || !u) return fail(c, "hamr_stage_forward_dev: no array");
+    if (c->amr) return fail(c, "hamr_stage_forward_dev: uniform grids only");
+    HIPCHK(c, hipSetDevice(c->device));
+    if (state_in(c, p, ps)) return -1;
+    enqueue_stage_forward(c, Dt);
+    double *out = u;
+    const size_t bytes = (size_t)nblk_of(c) * NPR * ncell_of(c->blocks[0]) * sizeof(double);
+    if (!on_device(c, u)) HIPCHK(c, hipMalloc((void **)&out, bytes));
+    launch_box_out(c->P, nblk_of(c), c->blocks[0], c->Un, out, c->s);
+    int r = check_launch(c, "hamr_stage_forward_dev");
+    hipError_t e = out == u || r ? hipSuccess : hipMemcpyAsync(u, out, bytes, hipMemcpyDeviceToDevice, c->s);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->s);
+    if (out != u) (void)hipFree(out);
+    HIPCHK(c, e);
+    return r;
+}
+
+int hamr_stage_grad_dev(hamr_ctx *c, double Dt, const double *p, const double *ps, const double *w, double *gp,
+                        double *gps)
+{
+    AdjBufs A;
+    if (adjoint_ok(c, w, "hamr_stage_grad_dev")) return -1;
+    if (!p || !ps) return fail(c, "hamr_stage_grad_dev: no state");
+    const AdjDirect d = adjoint_direct(c, w, gp, gps);
+    if (adjoint_bufs(c, d, A) || state_in(c, p, ps)) return -1;
+    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice, d, A);
 }
 
 // The work arrays carved from this device's `scratch` (c->scratch, resolved at
@@ -2410,7 +2491,8 @@ int hamr_stage_adjoint_dev_noalloc(hamr_ctx *c, double Dt, const double *w, doub
     A.lps = take(3);
     A.lE = take(3);
     A.X = take(kAdjXSlabs);
-    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice, A);
+    return stage_adjoint(c, Dt, w, gp, gps, hipMemcpyDeviceToDevice, hipMemcpyDeviceToDevice,
+                         adjoint_direct(c, w, gp, gps), A);
 }
 
 int hamr_copy_probe(hamr_ctx *c, long long bytes, int nrep, double *avg_ms)

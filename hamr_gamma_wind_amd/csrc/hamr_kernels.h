@@ -230,6 +230,11 @@ void launch_dt_finalize(int nblk, unsigned long long *dtmin, double *dt, hipStre
 void launch_las_corr(const KParams &P, const LasCorr *e, int64_t n, int dir, int stage, void *FE, double *acc,
                      const double *dt_ptr, int mixed, hipStream_t s);
 void launch_dt_reset(int nblk, unsigned long long *dtmin, hipStream_t s);
+// Unpadded arrays of nblk equal blocks (like B): 9 and 3 components into the slabs p
+// and ps; the interior of the 9-component slabs U out, zeros in its ghosts.
+void launch_box_in(const KParams &P, int nblk, const BlockDev &B, const double *sp, const double *sps, double *p,
+                   double *ps, hipStream_t s);
+void launch_box_out(const KParams &P, int nblk, const BlockDev &B, const double *U, double *dst, hipStream_t s);
 void launch_copy(const void *src, void *dst, int64_t bytes, hipStream_t s);
 
 // Multi-level ghost exchange of stage dir (1..3): copy/restriction entries,

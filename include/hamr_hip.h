@@ -431,6 +431,13 @@ int hamr_time_kernel(hamr_ctx *ctx, int slot, int nrep, double *avg_ms);
 int hamr_stage_forward(hamr_ctx *ctx, double Dt);
 int hamr_stage_adjoint(hamr_ctx *ctx, double Dt, const double *w, double *grad_p, double *grad_ps);
 int hamr_stage_adjoint_dev(hamr_ctx *ctx, double Dt, const double *w_dev, double *grad_p_dev, double *grad_ps_dev);
+/* The stage on device arrays in the unpadded layout of hamr_set_array_dev: the
+ * state is read from p_dev and ps_dev (and left in HAMR_P and HAMR_PS with its
+ * ghosts filled); u_dev gets HAMR_UNEW with zeros in the ghosts.  Uniform grids. */
+int hamr_stage_forward_dev(hamr_ctx *ctx, double Dt, const double *p_dev, const double *ps_dev, double *u_dev);
+/* hamr_stage_adjoint_dev of the state p_dev, ps_dev. */
+int hamr_stage_grad_dev(hamr_ctx *ctx, double Dt, const double *p_dev, const double *ps_dev, const double *w_dev,
+                        double *grad_p_dev, double *grad_ps_dev);
 
 /* hamr_stage_adjoint_dev without any allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under

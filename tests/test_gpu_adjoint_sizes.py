@@ -50,3 +50,55 @@ def test_gradient_equals_reference(n):
     print(n, "dL/dP", np.array2string(eP, precision=2), "dL/dB", np.array2string(eS, precision=2), flush=True)
     assert np.all(eP[:8] <= 1e-9) and np.abs(gp[0][8]).max() == 0.0
     assert np.all(eS <= 1e-9)
+
+
+def _dev(a):
+    return torch.tensor(a, device="cuda:0")
+
+
+def test_buffers_in_place_and_overlapping():
+    """The gradients are written in place where nothing overlaps them, else through
+    the work arrays: over the weights, without dL/d(face field), and apart."""
+    n = (9, 6, 11)
+    ctx = H.Context(H.make_desc(n, (1, 1, 1), gam=GAM, minkowski=1, rho_floor=0.0, u_floor=0.0))
+    try:
+        ctx.set_grid()
+        p, ps = (_dev(a) for a in W.to_block(*W.minkowski_box(n, gam=GAM, seed=33)))
+        w = _dev(np.random.default_rng(34).normal(size=tuple(p.shape)))
+        w[..., :NG] = float("nan")  # weights of ghosts are not read
+        gp, gps = torch.full_like(p, float("nan")), torch.full_like(ps, float("nan"))
+        torch.cuda.synchronize()
+        state = (1e-3, p.data_ptr(), ps.data_ptr())
+        ctx.stage_grad_dev(*state, w.data_ptr(), gp.data_ptr(), gps.data_ptr())
+        assert torch.isfinite(gp).all() and torch.isfinite(gps).all()
+        only, over = torch.zeros_like(p), w.clone()
+        torch.cuda.synchronize()
+        ctx.stage_grad_dev(*state, w.data_ptr(), only.data_ptr(), None)
+        ctx.stage_grad_dev(*state, over.data_ptr(), over.data_ptr(), gps.data_ptr())
+        assert torch.equal(only, gp) and torch.equal(over, gp)
+    finally:
+        ctx.close()
+
+
+def test_stage_from_device_arrays_equals_the_steps():
+    """hamr_stage_forward_dev of several blocks: set, forward, get, ghosts zeroed."""
+    ctx = H.Context(H.make_desc((9, 10, 7), (2, 2, 2)))
+    try:
+        ctx.set_grid()
+        ctx.init_torus(H.torus_desc())
+        p, ps = _dev(ctx.get(H.HAMR_P)), _dev(ctx.get(H.HAMR_PS))
+        U, V = torch.full_like(p, float("nan")), torch.empty_like(p)
+        torch.cuda.synchronize()
+        ctx.stage_forward_dev(1e-3, p.data_ptr(), ps.data_ptr(), U.data_ptr())
+        got = ctx.get(H.HAMR_P), ctx.get(H.HAMR_PSH)
+        ctx.set_dev(H.HAMR_P, p.data_ptr())
+        ctx.set_dev(H.HAMR_PS, ps.data_ptr())
+        ctx.stage_forward(1e-3)
+        ctx.get_dev(H.HAMR_UNEW, V.data_ptr())
+        I = (Ellipsis,) + (slice(NG, -NG),) * 3
+        assert torch.equal(U[I], V[I])
+        U[I] = 0.0
+        assert not U.any()
+        assert np.array_equal(got[0], ctx.get(H.HAMR_P)) and np.array_equal(got[1], ctx.get(H.HAMR_PSH))
+    finally:
+        ctx.close()
