@@ -1466,14 +1466,13 @@ int hamr_emf_correct(hamr_ctx *c, int flag, double dt)
 int hamr_block_dt(hamr_ctx *c, int n, int dir, double *out)
 {
     if (!c || !valid_block(c, n) || dir < 1 || dir > 3 || !out) return fail(c, "hamr_block_dt: bad arguments");
-    unsigned long long v;
+    // one kernel moves the minimum to pinned memory and resets it, so the call waits
+    // for the stream once (a copy out and a copy in waited four times: 16 us more a call)
+    if (stage_reserve(c, sizeof(double))) return -1;
+    launch_dt_take(c->dtmin + n * 3 + dir - 1, (double *)c->stage, c->s);
+    if (check_launch(c, "hamr_block_dt")) return -1;
     HIPCHK(c, hipStreamSynchronize(c->s));
-    if (d2h(c, &v, c->dtmin + n * 3 + dir - 1, sizeof v)) return -1;
-    double d;
-    std::memcpy(&d, &v, sizeof d);
-    *out = d;
-    const unsigned long long init = 0x41CDCD6500000000ULL;
-    if (h2d(c, c->dtmin + n * 3 + dir - 1, &init, sizeof init)) return -1;
+    std::memcpy(out, c->stage, sizeof(double));
     return 0;
 }
 

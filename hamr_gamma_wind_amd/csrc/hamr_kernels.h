@@ -229,6 +229,8 @@ void launch_dt_finalize(int nblk, unsigned long long *dtmin, double *dt, hipStre
 // writes acc / (dt tl) into every receiver at its corrector.
 void launch_las_corr(const KParams &P, const LasCorr *e, int64_t n, int dir, int stage, void *FE, double *acc,
                      const double *dt_ptr, int mixed, hipStream_t s);
+// One direction minimum into *out (host-coherent memory), and its reset.
+void launch_dt_take(unsigned long long *dtmin, double *out, hipStream_t s);
 void launch_dt_reset(int nblk, unsigned long long *dtmin, hipStream_t s);
 // Unpadded arrays of nblk equal blocks (like B): 9 and 3 components into the slabs p
 // and ps; the interior of the 9-component slabs U out, zeros in its ghosts.

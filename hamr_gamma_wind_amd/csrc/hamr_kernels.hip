@@ -1535,6 +1535,17 @@ void launch_las_corr(const KParams &P, const LasCorr *e, int64_t n, int dir, int
                            dt_ptr);
 }
 
+static __global__ void k_dt_take(unsigned long long *__restrict__ dtmin, double *__restrict__ out)
+{
+    *out = __longlong_as_double((long long)*dtmin);
+    *dtmin = (unsigned long long)__double_as_longlong(1.e9);
+}
+
+void launch_dt_take(unsigned long long *dtmin, double *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_dt_take, dim3(1), dim3(1), 0, s, dtmin, out);
+}
+
 void launch_dt_reset(int nblk, unsigned long long *dtmin, hipStream_t s)
 {
     const int n = nblk * 3;
