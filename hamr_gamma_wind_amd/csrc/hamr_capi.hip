@@ -494,10 +494,17 @@ static void emf_correct_all(hamr_ctx *c, double dt_val, const double *dt_ptr)
     launch_amr_emf(c->P, c->emfx, c->nemfx, c->E, dt_val, dt_ptr, c->prec, c->s);
 }
 
-static void emf_all(hamr_ctx *c, const double *p)
+// Fluxes and centre EMFs of every block, and the corner EMFs from them.
+static void front_all(hamr_ctx *c, const double *p, const double *ps, unsigned long long *dtmin)
 {
-    launch_emf(c->P, all_launch(c, TS_ECENT), all_launch(c, TS_ECORNER), p, c->F[0], c->F[1], c->F[2], c->Ec, c->E,
-               c->prec, c->s);
+    const Launch L[4] = {all_launch(c, TS_FLUX1), all_launch(c, TS_FLUX2), all_launch(c, TS_FLUX3),
+                         all_launch(c, TS_ECENT)};
+    launch_front(c->P, L, p, ps, c->F, dtmin, c->Ec, c->prec, c->s);
+}
+
+static void corner_all(hamr_ctx *c)
+{
+    launch_emf_corner(c->P, all_launch(c, TS_ECORNER), c->Ec, c->F[0], c->F[1], c->F[2], c->E, c->prec, c->s);
 }
 
 static int max_plane(const hamr_ctx *c)
@@ -1479,8 +1486,8 @@ int hamr_block_dt(hamr_ctx *c, int n, int dir, double *out)
 int hamr_ct_emf(hamr_ctx *c, int flag, int n)
 {
     if (!c || !valid_block(c, n)) return fail(c, "hamr_ct_emf: bad block");
-    launch_emf(c->P, block_launch(c, KC_ECENT, n), block_launch(c, KC_CORNER, n), flag ? c->ph : c->p, c->F[0],
-               c->F[1], c->F[2], c->Ec, c->E, c->prec, c->s);
+    launch_emf_centre(c->P, block_launch(c, KC_ECENT, n), flag ? c->ph : c->p, c->Ec, c->prec, c->s);
+    launch_emf_corner(c->P, block_launch(c, KC_CORNER, n), c->Ec, c->F[0], c->F[1], c->F[2], c->E, c->prec, c->s);
     return check_launch(c, "hamr_ct_emf");
 }
 
@@ -1557,12 +1564,11 @@ static void enqueue_step(hamr_ctx *c)
     // predictor: p/ps -> ph/psh with Dt = dt/2
     {
         StageRange r("predictor: fluxes");
-        for (int dir = 1; dir <= 3; dir++)
-            launch_flux(P, dir, all_launch(c, TS_FLUX1 + dir - 1), c->p, c->ps, c->F[dir - 1], nullptr, c->prec, s);
+        front_all(c, c->p, c->ps, nullptr);
     }
     {
         StageRange r("predictor: EMFs and face field");
-        emf_all(c, c->p);
+        corner_all(c);
         pole(c, 0., c->dt);
         launch_ct_update(P, all_launch(c, TS_CT), 0., c->dt, 0.5, c->ps, c->psh, c->E, c->prec, s);
     }
@@ -1577,14 +1583,12 @@ static void enqueue_step(hamr_ctx *c)
     // corrector: U0 -> p/ps with Dt = dt, fluxes from ph/psh, Courant minima recorded
     {
         StageRange r("corrector: fluxes and corrections");
-        for (int dir = 1; dir <= 3; dir++)
-            launch_flux(P, dir, all_launch(c, TS_FLUX1 + dir - 1), c->ph, c->psh, c->F[dir - 1], c->dtmin, c->prec,
-                        s);
+        front_all(c, c->ph, c->psh, c->dtmin);
         reflux_all(c, 0., c->dt);
     }
     {
         StageRange r("corrector: EMFs and face field");
-        emf_all(c, c->ph);
+        corner_all(c);
         pole(c, 0., c->dt);
         emf_correct_all(c, 0., c->dt);
         launch_ct_update(P, all_launch(c, TS_CT), 0., c->dt, 1.0, c->ps, c->ps, c->E, c->prec, s);
@@ -1893,20 +1897,16 @@ static void enqueue_las_cycle(hamr_ctx *c, int maxtl)
         P.las_s = s;
         P.las_want = LAS_IDLE;
         const bool last = s == 2 * maxtl - 1;
-        for (int ph = LAS_HALF; ph <= LAS_FULL; ph++)
-            for (int dir = 1; dir <= 3; dir++) {
-                const Launch L = las_launch(c, KC_FLUX1 + dir - 1, s, ph);
-                if (L.wl.n)
-                    launch_flux(P, dir, L, las_in(c, ph), las_ins(c, ph), c->F[dir - 1], last ? c->dtmin : nullptr,
-                                mixed, st);
-            }
+        for (int ph = LAS_HALF; ph <= LAS_FULL; ph++) {
+            const Launch L[4] = {las_launch(c, KC_FLUX1, s, ph), las_launch(c, KC_FLUX2, s, ph),
+                                 las_launch(c, KC_FLUX3, s, ph), las_launch(c, KC_ECENT, s, ph)};
+            launch_front(P, L, las_in(c, ph), las_ins(c, ph), c->F, last ? c->dtmin : nullptr, c->Ec, mixed, st);
+        }
         for (int d = 0; d < 3; d++)
             for (int stage = 0; stage < 2; stage++)
                 launch_las_corr(P, c->las_f[d], c->nlas_f[d], d + 1, stage, c->F[d], c->acc_f[d], c->dt, mixed, st);
         for (int ph = LAS_HALF; ph <= LAS_FULL; ph++) {
-            const Launch Lc = las_launch(c, KC_ECENT, s, ph), Le = las_launch(c, KC_CORNER, s, ph);
-            if (Lc.wl.n && Le.wl.n)
-                launch_emf(P, Lc, Le, las_in(c, ph), c->F[0], c->F[1], c->F[2], c->Ec, c->E, mixed, st);
+            launch_emf_corner(P, las_launch(c, KC_CORNER, s, ph), c->Ec, c->F[0], c->F[1], c->F[2], c->E, mixed, st);
         }
         for (int ph = LAS_HALF; ph <= LAS_FULL; ph++) {
             P.las_want = ph;
@@ -2141,6 +2141,49 @@ static int restore_flags(hamr_ctx *c, const FlagCopy &k, const char *what)
     return 0;
 }
 
+// The fluxes and centre EMFs run as one kernel where their launches have one form:
+// the fastest such form, if it beats the four slots' own best launches in turn.
+static int tune_front(hamr_ctx *c, int nrep)
+{
+    hipEvent_t e0, e1;
+    HIPCHK(c, hipEventCreate(&e0));
+    HIPCHK(c, hipEventCreate(&e1));
+    auto front_ms = [&](float *ms) -> int {
+        front_all(c, c->p, c->ps, nullptr);  // warm-up
+        HIPCHK(c, hipEventRecord(e0, c->s));
+        for (int r = 0; r < nrep; r++) front_all(c, c->p, c->ps, nullptr);
+        HIPCHK(c, hipEventRecord(e1, c->s));
+        HIPCHK(c, hipEventSynchronize(e1));
+        HIPCHK(c, hipEventElapsedTime(ms, e0, e1));
+        return check_launch(c, "autotune");
+    };
+    TuneCfg best[4];
+    std::copy(c->tune + TS_FLUX1, c->tune + TS_ECENT + 1, best);
+    float best_ms;
+    if (front_ms(&best_ms)) return -1;
+    for (int ti = 0; ti < 3; ti++)
+        for (int swz = 0; swz < 2; swz++) {
+            float ms;
+            for (int k = 0; k < 4; k++) {
+                c->tune[TS_FLUX1 + k] = TuneCfg();
+                c->tune[TS_FLUX1 + k].tile = ti;
+                c->tune[TS_FLUX1 + k].swz = swz;
+            }
+            if (front_ms(&ms)) return -1;
+            if (ms >= best_ms) continue;
+            best_ms = ms;
+            for (int k = 0; k < 4; k++) {
+                const int slot = TS_FLUX1 + k;
+                if (time_launches(c, slot, all_launch(c, slot), 0, 0, nrep, &c->tune[slot].ms)) return -1;
+                best[k] = c->tune[slot];
+            }
+        }
+    std::copy(best, best + 4, c->tune + TS_FLUX1);
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    return 0;
+}
+
 int hamr_autotune(hamr_ctx *c, int nrep)
 {
     if (!c || nrep < 1) return fail(c, "hamr_autotune: bad arguments");
@@ -2190,6 +2233,7 @@ int hamr_autotune(hamr_ctx *c, int nrep)
         }
         c->tune[slot] = best;
     }
+    if (tune_front(c, nrep)) return -1;
     if (restore_flags(c, keepf, "autotune")) return -1;
     drop_graphs(c);
     return 0;
@@ -2263,7 +2307,10 @@ int hamr_time_stage(hamr_ctx *c, int stage, int nrep, double *avg_ms)
         case 2:
             launch_flux(c->P, stage + 1, all_launch(c, TS_FLUX1 + stage), c->p, c->ps, c->F[stage], nullptr, c->prec, c->s);
             break;
-        case 3: emf_all(c, c->p); break;
+        case 3:
+            launch_emf_centre(c->P, all_launch(c, TS_ECENT), c->p, c->Ec, c->prec, c->s);
+            corner_all(c);
+            break;
         case 4: pole(c, 0., c->dt); break;
         case 5: launch_ct_update(c->P, all_launch(c, TS_CT), 0., c->dt, 0.5, c->ps, c->psh, c->E, c->prec, c->s); break;
         case 6: update_all(c, 0, 0., c->dt, 0.5, c->p, c->p, c->ph, c->psh); break;
@@ -2285,9 +2332,8 @@ int hamr_time_stage(hamr_ctx *c, int stage, int nrep, double *avg_ms)
 static void enqueue_stage_forward(hamr_ctx *c, double Dt)
 {
     bound_all(c, c->p, c->ps);
-    for (int dir = 1; dir <= 3; dir++)
-        launch_flux(c->P, dir, all_launch(c, TS_FLUX1 + dir - 1), c->p, c->ps, c->F[dir - 1], nullptr, c->prec, c->s);
-    emf_all(c, c->p);
+    front_all(c, c->p, c->ps, nullptr);
+    corner_all(c);
     pole(c, Dt, nullptr);
     launch_ct_update(c->P, all_launch(c, TS_CT), Dt, nullptr, 1.0, c->ps, c->psh, c->E, c->prec, c->s);
     launch_cons(c->P, all_launch(c, TS_CONS), Dt, c->p, c->U0, c->Un, c->psh, c->F[0], c->F[1], c->F[2], c->prec, c->s);

@@ -64,6 +64,14 @@ struct WorkList {
     int swz;
 };
 
+// The lists of the merged launch of KC_FLUX1 .. KC_FLUX3 and KC_ECENT; the first
+// `chunked` items of each are taken chunk by chunk in turn (whole chunks), the rest
+// class by class.
+struct FrontLists {
+    WorkList wl[4];
+    int chunked;
+};
+
 // One launch configuration: the work list built for `threads` per tile, the
 // workgroup count (<= wl.n) and the LDS the update kernel stages per tile.
 struct Launch {
@@ -131,9 +139,11 @@ inline int cons_max_cols(int bs3, int threads) { return (threads - 1) / bs3 + 2;
 // (F, Ec, E are double arrays), 1 = FP32 (float arrays with the same slab layout).
 void launch_flux(const KParams &P, int dir, const Launch &L, const double *p, const double *ps, void *F,
                  unsigned long long *dtmin, int mixed, hipStream_t s);
-void launch_emf(const KParams &P, const Launch &centre, const Launch &corner, const double *p, const void *F1,
-                const void *F2, const void *F3, void *Ec, void *E, int mixed, hipStream_t s);
-// Its two kernels one at a time (for timing and tuning).
+// The three fluxes and the centre EMFs of a set of blocks.  L: the launches of KC_FLUX1
+// .. KC_FLUX3 and KC_ECENT; one kernel where they take one tile size, a thread per face
+// and a workgroup per tile, else one after the other.
+void launch_front(const KParams &P, const Launch *L, const double *p, const double *ps, double *const *F,
+                  unsigned long long *dtmin, void *Ec, int mixed, hipStream_t s);
 void launch_emf_centre(const KParams &P, const Launch &L, const double *p, void *Ec, int mixed, hipStream_t s);
 void launch_emf_corner(const KParams &P, const Launch &L, const void *Ec, const void *F1, const void *F2,
                        const void *F3, void *E, int mixed, hipStream_t s);

@@ -1383,12 +1383,24 @@ void launch_emf_corner(const KParams &P, const Launch &L, const void *Ec, const 
                          (double *)E, s);
 }
 
-void launch_emf(const KParams &P, const Launch &centre, const Launch &corner, const double *p, const void *F1,
-                const void *F2, const void *F3, void *Ec, void *E, int mixed, hipStream_t s)
+static bool front_merges(const Launch *L)
 {
-    if (centre.wl.n <= 0) return;
-    launch_emf_centre(P, centre, p, Ec, mixed, s);
-    launch_emf_corner(P, corner, Ec, F1, F2, F3, E, mixed, s);
+    for (int k = 0; k < 4; k++)
+        if (L[k].line || L[k].threads != L[0].threads || L[k].grid != L[k].wl.n) return false;
+    return true;
+}
+
+void launch_front(const KParams &P, const Launch *L, const double *p, const double *ps, double *const *F,
+                  unsigned long long *dtmin, void *Ec, int mixed, hipStream_t s)
+{
+    if (!front_merges(L)) {
+        for (int d = 0; d < 3; d++) launch_flux(P, d + 1, L[d], p, ps, F[d], dtmin, mixed, s);
+        launch_emf_centre(P, L[3], p, Ec, mixed, s);
+    } else if (mixed) {
+        launch_front_f32(P, L, p, ps, (float *)F[0], (float *)F[1], (float *)F[2], dtmin, (float *)Ec, s);
+    } else {
+        recon_front(P, L, p, ps, (double *)F[0], (double *)F[1], (double *)F[2], dtmin, (double *)Ec, s);
+    }
 }
 
 void launch_pole(const KParams &P, const int *ring, const int *rside, int nring, int len, int ni_max, double dt_val,

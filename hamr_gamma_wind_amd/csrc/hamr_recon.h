@@ -130,60 +130,64 @@ __device__ __forceinline__ void dt_reduce(double vdt, unsigned long long *__rest
 // faster than one wave with none spilled.  The FP32 HLLC kernel at four waves
 // (128 VGPRs, 9 spilled) ran 4% faster than at three (139, none spilled).
 template <int DIR, class R, int RS>
+__device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const double *__restrict__ p,
+                                          const double *__restrict__ ps, R *__restrict__ F,
+                                          unsigned long long *__restrict__ dtmin)
+{
+    const int n = it.x;
+    const BlockDev &B = P.blk[n];
+    const int e1 = B.bs[0] + (DIR == 1 ? 1 : 2), e2 = B.bs[1] + (DIR == 2 ? 1 : 2), e3 = B.bs[2] + (DIR == 3 ? 1 : 2);
+    const int t = it.y * blockDim.x + threadIdx.x;
+    double vdt = 1.e9;
+    if (t < e1 * e2 * e3) {
+        int a, b, c;
+        region_index(t, e2, e3, a, b, c);
+        const int i = a + (DIR == 1 ? NG : NG - 1);
+        const int j = b + (DIR == 2 ? NG : NG - 1);
+        const int z = c + (DIR == 3 ? NG : NG - 1);
+        const int64_t K = B.ks;
+        const int64_t cell = ((int64_t)i * B.D[1] + j) * B.D[2] + z;
+        const int64_t sd = (DIR == 1) ? (int64_t)B.D[1] * B.D[2] : (DIR == 2) ? (int64_t)B.D[2] : 1;
+        const double *pb = p + NPR * B.off;
+        R pl[NPR], pr[NPR];
+        // every stencil value first, then the parabolas (KTOT enters no flux)
+        double y[KTOT][6];
+#pragma unroll
+        for (int k = 0; k < KTOT; k++) {
+            if (k == B1 + DIR - 1) continue;
+            const double *q = pb + (int64_t)k * K;
+#pragma unroll
+            for (int m = 0; m < 6; m++) y[k][m] = gld(q + (m - 3) * sd, (uint32_t)cell);
+        }
+        auto one = [&](int k) {
+            if (k == B1 + DIR - 1) return;  // the face-normal field comes from ps
+            const R ym3 = (R)y[k][0], ym2 = (R)y[k][1], ym1 = (R)y[k][2], y0 = (R)y[k][3], yp1 = (R)y[k][4],
+                    yp2 = (R)y[k][5];
+            R l, r;
+            para(ym3, ym2, ym1, y0, yp1, l, r);
+            pl[k] = r;
+            para(ym2, ym1, y0, yp1, yp2, l, r);
+            pr[k] = l;
+        };
+#pragma unroll
+        for (int k = 0; k < 4; k++) one(k);
+        // the metric while the rest is reconstructed, in the registers the first stencils left
+        const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
+        const R bn = (R)gld(ps + 3 * B.off + (DIR - 1) * K, (uint32_t)cell);
+#pragma unroll
+        for (int k = 4; k < KTOT; k++) one(k);
+        if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+        else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+    }
+    if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
+}
+
+template <int DIR, class R, int RS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
 k_flux(KParams P, WorkList wl, const double *__restrict__ p, const double *__restrict__ ps, R *__restrict__ F,
        unsigned long long *__restrict__ dtmin)
 {
-    FOR_ITEMS(wl)
-    {
-        const int2 it = wl_get(wl, w_);
-        const int n = it.x;
-        const BlockDev &B = P.blk[n];
-        const int e1 = B.bs[0] + (DIR == 1 ? 1 : 2), e2 = B.bs[1] + (DIR == 2 ? 1 : 2), e3 = B.bs[2] + (DIR == 3 ? 1 : 2);
-        const int t = it.y * blockDim.x + threadIdx.x;
-        double vdt = 1.e9;
-        if (t < e1 * e2 * e3) {
-            int a, b, c;
-            region_index(t, e2, e3, a, b, c);
-            const int i = a + (DIR == 1 ? NG : NG - 1);
-            const int j = b + (DIR == 2 ? NG : NG - 1);
-            const int z = c + (DIR == 3 ? NG : NG - 1);
-            const int64_t K = B.ks;
-            const int64_t cell = ((int64_t)i * B.D[1] + j) * B.D[2] + z;
-            const int64_t sd = (DIR == 1) ? (int64_t)B.D[1] * B.D[2] : (DIR == 2) ? (int64_t)B.D[2] : 1;
-            const double *pb = p + NPR * B.off;
-            R pl[NPR], pr[NPR];
-            // every stencil value first, then the parabolas (KTOT enters no flux)
-            double y[KTOT][6];
-#pragma unroll
-            for (int k = 0; k < KTOT; k++) {
-                if (k == B1 + DIR - 1) continue;
-                const double *q = pb + (int64_t)k * K;
-#pragma unroll
-                for (int m = 0; m < 6; m++) y[k][m] = gld(q + (m - 3) * sd, (uint32_t)cell);
-            }
-            auto one = [&](int k) {
-                if (k == B1 + DIR - 1) return;  // the face-normal field comes from ps
-                const R ym3 = (R)y[k][0], ym2 = (R)y[k][1], ym1 = (R)y[k][2], y0 = (R)y[k][3], yp1 = (R)y[k][4],
-                        yp2 = (R)y[k][5];
-                R l, r;
-                para(ym3, ym2, ym1, y0, yp1, l, r);
-                pl[k] = r;
-                para(ym2, ym1, y0, yp1, yp2, l, r);
-                pr[k] = l;
-            };
-#pragma unroll
-            for (int k = 0; k < 4; k++) one(k);
-            // the metric while the rest is reconstructed, in the registers the first stencils left
-            const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
-            const R bn = (R)gld(ps + 3 * B.off + (DIR - 1) * K, (uint32_t)cell);
-#pragma unroll
-            for (int k = 4; k < KTOT; k++) one(k);
-            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
-            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
-        }
-        if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
-    }
+    FOR_ITEMS(wl) flux_item<DIR, R, RS>(P, wl_get(wl, w_), p, ps, F, dtmin);
 }
 
 // ---------------------------------------------------------------------------
@@ -318,35 +322,75 @@ k_flux_lines(KParams P, WorkList wl, const double *__restrict__ p, const double 
 // ---------------------------------------------------------------------------
 // Cell-centre EMF, consttransport1 (GPU_const_trans.h:63-119), cells [NG-1, NG+BS].
 template <class R>
+__device__ __forceinline__ void emf_centre_item(const KParams &P, const int2 it, const double *__restrict__ p,
+                                                R *__restrict__ Ec)
+{
+    const BlockDev &B = P.blk[it.x];
+    const int e1 = B.bs[0] + 2, e2 = B.bs[1] + 2, e3 = B.bs[2] + 2;
+    const int t = it.y * blockDim.x + threadIdx.x;
+    if (t >= e1 * e2 * e3) return;
+    int a, b, c;
+    region_index(t, e2, e3, a, b, c);
+    const int i = a + NG - 1, j = b + NG - 1, z = c + NG - 1;
+    const int64_t K = B.ks;
+    const int64_t cell = ((int64_t)i * B.D[1] + j) * B.D[2] + z;
+    const double *pb = p + NPR * B.off + cell;
+    R pr[NPR];
+#pragma unroll
+    for (int k = 0; k < NPR; k++) pr[k] = (R)pb[(int64_t)k * K];
+    const Geom<R> G = load_geom<R>(P, B, CENT, (int64_t)i * B.D[1] + j);
+    R ucon[4], ucov[4], bcon[4];
+    ucon_calc(pr, G, ucon);
+    lower10(ucon, G.gcov, ucov);
+    bcon_calc(pr, ucon, ucov, bcon);
+    R *E = Ec + 3 * B.off + cell;
+    E[0] = -G.g * (ucon[2] * bcon[3] - ucon[3] * bcon[2]);
+    E[K] = -G.g * (ucon[3] * bcon[1] - ucon[1] * bcon[3]);
+    E[2 * K] = -G.g * (ucon[1] * bcon[2] - ucon[2] * bcon[1]);
+}
+
+template <class R>
 __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, const double *__restrict__ p,
                                                     R *__restrict__ Ec)
 {
-    FOR_ITEMS(wl)
-    {
-        const int2 it = wl_get(wl, w_);
-        const BlockDev &B = P.blk[it.x];
-        const int e1 = B.bs[0] + 2, e2 = B.bs[1] + 2, e3 = B.bs[2] + 2;
-        const int t = it.y * blockDim.x + threadIdx.x;
-        if (t >= e1 * e2 * e3) continue;
-        int a, b, c;
-        region_index(t, e2, e3, a, b, c);
-        const int i = a + NG - 1, j = b + NG - 1, z = c + NG - 1;
-        const int64_t K = B.ks;
-        const int64_t cell = ((int64_t)i * B.D[1] + j) * B.D[2] + z;
-        const double *pb = p + NPR * B.off + cell;
-        R pr[NPR];
-#pragma unroll
-        for (int k = 0; k < NPR; k++) pr[k] = (R)pb[(int64_t)k * K];
-        const Geom<R> G = load_geom<R>(P, B, CENT, (int64_t)i * B.D[1] + j);
-        R ucon[4], ucov[4], bcon[4];
-        ucon_calc(pr, G, ucon);
-        lower10(ucon, G.gcov, ucov);
-        bcon_calc(pr, ucon, ucov, bcon);
-        R *E = Ec + 3 * B.off + cell;
-        E[0] = -G.g * (ucon[2] * bcon[3] - ucon[3] * bcon[2]);
-        E[K] = -G.g * (ucon[3] * bcon[1] - ucon[1] * bcon[3]);
-        E[2 * K] = -G.g * (ucon[1] * bcon[2] - ucon[2] * bcon[1]);
+    FOR_ITEMS(wl) emf_centre_item(P, wl_get(wl, w_), p, Ec);
+}
+
+// The three fluxes and the centre EMFs in one launch.  They depend on nothing of each
+// other, so that a class's blocks start while the last ones of the class before
+// still run, where as four launches each waited for the slowest block of the one
+// before with the chip draining (a flux block runs 10 us or more on its own, and a
+// grid of 64x32x32 zones fills the chip once).  The classes follow one another, the
+// light one last; FP32 launches of four chunks or more per class go chunk by chunk,
+// so that the primitives of a region come from the memory-side cache for three of
+// their four readings (FP64 fluxes issue too long for that to show: 256x128x128
+// 3.86 and 3.88 ms a step).  Classes in turn from one workgroup to the next run 8-20%
+// slower: the three flux bodies do not fit the instruction cache together.
+// Per pass, four launches -> one: 64x32x32 FP64 1.93 -> 1.66 ms, 42x25x39 blocks 4.82
+// -> 4.28, 256x128x128 17.0 -> 16.5, HLLC 96x72x60 3.11 -> 2.71; mixed 384x192x192
+// 42.5 -> 40.1, HLLC 256x128x128 14.8 -> 13.4; the step of 384x192x192 by chunk
+// (items): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
+constexpr int kFrontChunk = 4096;
+template <class R, int RS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
+k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__restrict__ ps, R *__restrict__ F1,
+        R *__restrict__ F2, R *__restrict__ F3, unsigned long long *__restrict__ dtmin, R *__restrict__ Ec)
+{
+    const int w = blockIdx.x;
+    int cls, idx;
+    if (w < 4 * L.chunked) {
+        cls = (w / kFrontChunk) & 3;
+        idx = w / (4 * kFrontChunk) * kFrontChunk + w % kFrontChunk;
+    } else {
+        idx = w - 4 * L.chunked;
+        for (cls = 0; cls < 3 && idx >= L.wl[cls].n - L.chunked; cls++) idx -= L.wl[cls].n - L.chunked;
+        idx += L.chunked;
     }
+    const int2 it = wl_get(L.wl[cls], idx);
+    if (cls == 0) flux_item<1, R, RS>(P, it, p, ps, F1, dtmin);
+    else if (cls == 1) flux_item<2, R, RS>(P, it, p, ps, F2, dtmin);
+    else if (cls == 2) flux_item<3, R, RS>(P, it, p, ps, F3, dtmin);
+    else emf_centre_item(P, it, p, Ec);
 }
 
 // Corner EMF upwinded on the mass-flux sign, consttransport2
@@ -464,6 +508,26 @@ void recon_flux(const KParams &P, int dir, const Launch &L, const double *p, con
 }
 
 template <class R>
+void recon_front(const KParams &P, const Launch *L, const double *p, const double *ps, R *F1, R *F2, R *F3,
+                 unsigned long long *dtmin, R *Ec, hipStream_t s)
+{
+    FrontLists f;
+    int n = 0;
+    for (int k = 0; k < 4; k++) {
+        f.wl[k] = L[k].wl;
+        n += L[k].wl.n;
+    }
+    f.chunked = L[0].wl.n;
+    for (int k = 1; k < 4; k++) f.chunked = L[k].wl.n < f.chunked ? L[k].wl.n : f.chunked;
+    f.chunked = sizeof(R) == 4 && f.chunked >= 4 * kFrontChunk ? f.chunked / kFrontChunk * kFrontChunk : 0;
+    if (n <= 0) return;
+    if (P.riemann == 1)
+        hipLaunchKernelGGL((k_front<R, 1>), dim3((unsigned)n), bdim(L[0]), 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+    else
+        hipLaunchKernelGGL((k_front<R, 0>), dim3((unsigned)n), bdim(L[0]), 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+}
+
+template <class R>
 void recon_emf_centre(const KParams &P, const Launch &L, const double *p, R *Ec, hipStream_t s)
 {
     if (L.wl.n <= 0) return;
@@ -481,6 +545,8 @@ void recon_emf_corner(const KParams &P, const Launch &L, const R *Ec, const R *F
 // The FP32 instantiations (hamr_kernels_f32.hip).
 void launch_flux_f32(const KParams &P, int dir, const Launch &L, const double *p, const double *ps, float *F,
                      unsigned long long *dtmin, hipStream_t s);
+void launch_front_f32(const KParams &P, const Launch *L, const double *p, const double *ps, float *F1, float *F2,
+                      float *F3, unsigned long long *dtmin, float *Ec, hipStream_t s);
 void launch_emf_centre_f32(const KParams &P, const Launch &L, const double *p, float *Ec, hipStream_t s);
 void launch_emf_corner_f32(const KParams &P, const Launch &L, const float *Ec, const float *F1, const float *F2,
                            const float *F3, float *E, hipStream_t s);

@@ -402,8 +402,10 @@ int hamr_autotune(hamr_ctx *ctx, int nrep);
  * update and the 2D inversion in two kernels (k_cons, then HAMR_TUNE_INVERT's
  * k_invert) instead of one (k_update).  For HAMR_TUNE_CONS, workgroups = -1
  * selects the two-kernel form with the update's x1-marching k_cons (one thread
- * per (j, z) walking i).  The tuner tries every form; all give the same result
- * bit for bit. */
+ * per (j, z) walking i).  HAMR_TUNE_FLUX1-3 and the centre EMFs' slot run as one
+ * kernel in a step while all four have one workgroup size, a workgroup per item
+ * and a thread per face, as by default.  The tuner tries every form; all give the
+ * same result bit for bit. */
 int hamr_tune_get(const hamr_ctx *ctx, int slot, int *cfg, double *ms);
 int hamr_tune_set(hamr_ctx *ctx, int slot, const int *cfg);
 /* Average device time (ms, HIP events on the context stream) of one launch of
