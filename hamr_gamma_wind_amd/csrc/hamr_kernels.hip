@@ -95,6 +95,9 @@ __global__ void __launch_bounds__(64) k_pole_average(KParams P, const int *__res
 // Face-B update from the curl of the corner EMF, consttransport3
 // (GPU_const_trans.h:426-530); faces [NG, NG+BS] along their normal.  psi and
 // psf may alias (each thread reads only the faces it writes).
+// Bound by memory: 0.36 GB (256x128x128 FP64), 0.85 GB (384x192x192 mixed) in 101 and
+// 295 us; 113 and 320 with each component's loads behind the store of the one before
+// and nine separate divisions.
 template <class R, bool TILED>
 __global__ void __launch_bounds__(256) k_ct_update(KParams P, WorkList wl, double Dt_val,
                                                    const double *__restrict__ dt_ptr, double dt_mult, const double *psi,
@@ -104,23 +107,26 @@ __global__ void __launch_bounds__(256) k_ct_update(KParams P, WorkList wl, doubl
     {
         const int2 it = wl_get(wl, w_);
         const BlockDev &B = P.blk[it.x];
-        const int e1 = B.bs[0] + 1, e2 = B.bs[1] + 1, e3 = B.bs[2] + 1;
+        const int n2 = B.bs[1] + 1, n3 = B.bs[2] + 1;
         const int t = it.y * blockDim.x + threadIdx.x;
-        if (t >= e1 * e2 * e3) continue;
+        if (t >= (B.bs[0] + 1) * n2 * n3) continue;
         int a, b, c;
-        region_index(t, e2, e3, a, b, c);
+        region_index(t, n2, n3, a, b, c);
         const int i = a + NG, j = b + NG, z = c + NG;
         const double Dt = block_Dt(P, B, Dt_val, dt_ptr, dt_mult);
         const int64_t K = B.ks, si = (int64_t)B.D[1] * B.D[2], sj = B.D[2];
         const int64_t g = ((int64_t)i * B.D[1] + j) * B.D[2] + z, col = (int64_t)i * B.D[1] + j;
-        const double gF1 = P.gdet[mg1(B, FACE1) + col], gF2 = P.gdet[mg1(B, FACE2) + col],
-                     gF3 = P.gdet[mg1(B, FACE3) + col];
-        const R *Ebr = E + 3 * B.off + g;
-        auto Eb = [&](int64_t o) { return (double)Ebr[o]; };
-        const double *si_ = psi + 3 * B.off + g;
-        double *sf = psf + 3 * B.off + g;
-        const double dx1 = B.dx[0], dx2 = B.dx[1], dx3 = B.dx[2];
-        double temp;
+        // every load first: psf may be psi, so none is moved above a store
+        const uint32_t o = (uint32_t)g;
+        const double gF1 = gld(P.gdet + mg1(B, FACE1), (uint32_t)col), gF2 = gld(P.gdet + mg1(B, FACE2), (uint32_t)col),
+                     gF3 = gld(P.gdet + mg1(B, FACE3), (uint32_t)col);
+        const R *E1 = E + 3 * B.off, *E2 = E1 + K, *E3 = E2 + K;
+        const double e1 = (double)gld(E1, o), e1j = (double)gld(E1 + sj, o), e1z = (double)gld(E1 + 1, o);
+        const double e2 = (double)gld(E2, o), e2i = (double)gld(E2 + si, o), e2z = (double)gld(E2 + 1, o);
+        const double e3 = (double)gld(E3, o), e3i = (double)gld(E3 + si, o), e3j = (double)gld(E3 + sj, o);
+        const double *sb = psi + 3 * B.off;
+        const double b1 = gld(sb, o), b2 = gld(sb + K, o), b3 = gld(sb + 2 * K, o);
+        double *sf = psf + 3 * B.off;
         // the x3 ghosts of the push table's receiver, as in finish_cell: B1 and
         // B2 of the NG lowest / highest cells of the z-row, B3 of the faces
         // that are not the block's own x3 boundary faces (each block forms those)
@@ -138,31 +144,34 @@ __global__ void __launch_bounds__(256) k_ct_update(KParams P, WorkList wl, doubl
             }
         }
         const int64_t KM = sm ? T.ks : 0;
+        const Div<double> by_g1(gF1), by_g2(gF2), by_g3(gF3);
+        const double r1 = Div<double>(B.dx[0])(Dt), r2 = Div<double>(B.dx[1])(Dt), r3 = Div<double>(B.dx[2])(Dt);
         if (j < NG + B.bs[1] && z < NG + B.bs[2]) {
-            temp = 0.;
-            temp += 1.0 / 1.0 * si_[0] * gF1;
-            temp += -Dt / (1.0 * dx2) * (Eb(2 * K + sj) - Eb(2 * K));
-            temp += Dt / (1.0 * dx3) * (Eb(K + 1) - Eb(K));
-            sf[0] = temp / gF1;
-            if (sm) sm[0] = sf[0];
-            if (sm2) sm2[0] = sf[0];
+            double temp = b1 * gF1;
+            temp += -r2 * (e3j - e3);
+            temp += r3 * (e2z - e2);
+            temp = by_g1(temp);
+            gst(sf, o, temp);
+            if (sm) sm[0] = temp;
+            if (sm2) sm2[0] = temp;
         }
         if (i < NG + B.bs[0] && j < NG + B.bs[1]) {
-            temp = si_[2 * K] * gF3;
-            temp += -Dt / dx1 * (Eb(K + si) - Eb(K));
-            temp += Dt / dx2 * (Eb(sj) - Eb(0));
-            sf[2 * K] = temp / gF3;
-            if (sm && z != NG) sm[2 * KM] = sf[2 * K];
-            if (sm2 && z != NG) sm2[2 * KM] = sf[2 * K];
+            double temp = b3 * gF3;
+            temp += -r1 * (e2i - e2);
+            temp += r2 * (e1j - e1);
+            temp = by_g3(temp);
+            gst(sf + 2 * K, o, temp);
+            if (sm && z != NG) sm[2 * KM] = temp;
+            if (sm2 && z != NG) sm2[2 * KM] = temp;
         }
         if (i < NG + B.bs[0] && z < NG + B.bs[2]) {
-            temp = 0.;
-            temp += 1.0 / 1.0 * si_[K] * gF2;
-            temp += Dt / (1.0 * dx1) * (Eb(2 * K + si) - Eb(2 * K));
-            temp += -Dt / (1.0 * dx3) * (Eb(1) - Eb(0));
-            sf[K] = temp / gF2;
-            if (sm) sm[KM] = sf[K];
-            if (sm2) sm2[KM] = sf[K];
+            double temp = b2 * gF2;
+            temp += r1 * (e3i - e3);
+            temp += -r3 * (e1z - e1);
+            temp = by_g2(temp);
+            gst(sf + K, o, temp);
+            if (sm) sm[KM] = temp;
+            if (sm2) sm2[KM] = temp;
         }
     }
 }
@@ -849,7 +858,8 @@ __global__ void __launch_bounds__(256) k_fill(KParams P, WorkList wl, double *p,
             }
         }
         auto cell = [&](const FillSrc &s) { return (s.i * d2 + s.j) * d3 + s.z; };
-        const int64_t K = B.ks, oa = P.blk[a.blk].off, o1 = P.blk[f1.blk].off, o2 = P.blk[f2.blk].off;
+        // (the slabs of a uniform grid follow one another)
+        const int64_t K = B.ks, oa = a.blk * K, o1 = f1.blk * K, o2 = f2.blk * K;
         const int cg = (i * d2 + j) * d3 + z, ca = cell(a), c1 = cell(f1), c2 = cell(f2);
         double pr[NPR];
 #pragma unroll
