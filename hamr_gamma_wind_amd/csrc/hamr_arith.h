@@ -62,6 +62,17 @@ template <> struct Div<double> {
 };
 #endif
 
+// a / 3, correctly rounded: Div's last step by a constant reciprocal, without its
+// treatment of infinite a (the quotient is then NaN, not infinite).
+template <class R> HD R third(R a) { return Div<R>(R(3.))(a); }
+#if HAMR_DEVICE_ARITH
+template <> HD double third<double>(double a)
+{
+    const double y = 1. / 3., q = a * y;
+    return fma(fma(-3., q, a), y, q);
+}
+#endif
+
 #if HAMR_DEVICE_ARITH
 // x^e in FP64 on the device, for the entropy of a state (x = rho).  The library
 // pow is 226 VALU instructions, 18% of the FP64 flux kernel, for two per face;
