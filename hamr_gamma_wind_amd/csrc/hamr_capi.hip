@@ -263,7 +263,7 @@ static int build_class_lists(hamr_ctx *c)
             if (c->amr) {
                 if (cls == KC_BOUND1) use = B.kind[0] == FK_OUTFLOW || B.kind[1] == FK_OUTFLOW;
                 else if (cls == KC_BOUND2) use = B.kind[2] == FK_POLE || B.kind[3] == FK_POLE;
-                else if (cls == KC_FILL || cls == KC_FILLROWS) use = false;
+                else if (cls == KC_FILL || cls == KC_FILLROWS || (cls >= KC_SFLUX1 && cls <= KC_SFLUX3)) use = false;
             } else if (cls == KC_BOUND1 || cls == KC_BOUND2) {
                 use = false;
             }
@@ -497,9 +497,11 @@ static void emf_correct_all(hamr_ctx *c, double dt_val, const double *dt_ptr)
 // Fluxes and centre EMFs of every block, and the corner EMFs from them.
 static void front_all(hamr_ctx *c, const double *p, const double *ps, unsigned long long *dtmin)
 {
-    const Launch L[4] = {all_launch(c, TS_FLUX1), all_launch(c, TS_FLUX2), all_launch(c, TS_FLUX3),
-                         all_launch(c, TS_ECENT)};
-    launch_front(c->P, L, p, ps, c->F, dtmin, c->Ec, c->prec, c->s);
+    Launch L[4] = {all_launch(c, TS_FLUX1), all_launch(c, TS_FLUX2), all_launch(c, TS_FLUX3), all_launch(c, TS_ECENT)};
+    const bool share = !c->amr && front_merges(L);
+    if (share)
+        for (int d = 0; d < 3; d++) L[d] = all_launch(c, TS_FLUX1 + d, KC_SFLUX1 + d);
+    launch_front(c->P, L, share, p, ps, c->F, dtmin, c->Ec, c->prec, c->s);
 }
 
 static void corner_all(hamr_ctx *c)
@@ -1900,7 +1902,7 @@ static void enqueue_las_cycle(hamr_ctx *c, int maxtl)
         for (int ph = LAS_HALF; ph <= LAS_FULL; ph++) {
             const Launch L[4] = {las_launch(c, KC_FLUX1, s, ph), las_launch(c, KC_FLUX2, s, ph),
                                  las_launch(c, KC_FLUX3, s, ph), las_launch(c, KC_ECENT, s, ph)};
-            launch_front(P, L, las_in(c, ph), las_ins(c, ph), c->F, last ? c->dtmin : nullptr, c->Ec, mixed, st);
+            launch_front(P, L, false, las_in(c, ph), las_ins(c, ph), c->F, last ? c->dtmin : nullptr, c->Ec, mixed, st);
         }
         for (int d = 0; d < 3; d++)
             for (int stage = 0; stage < 2; stage++)

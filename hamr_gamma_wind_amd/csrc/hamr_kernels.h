@@ -125,6 +125,8 @@ enum KClass : int {
     KC_FILL, KC_FILLROWS,              // ghost cells of a uniform grid's block: all, or without the x3 ghosts
                                        // inside its x1 and x2 range
     KC_LINE1, KC_LINE2, KC_LINE3,      // line-staged flux tiles of one direction (line_tiles)
+    KC_SFLUX1, KC_SFLUX2, KC_SFLUX3,   // faces of one direction (+ one transverse ghost layer along x3, and along x1
+                                       // and x2 where the side has no block beyond it), uniform grids
     KC_FLAGS,                          // the flag slab, kFlagsPerThread cells per thread (fallback)
     KC_N
 };
@@ -141,8 +143,13 @@ void launch_flux(const KParams &P, int dir, const Launch &L, const double *p, co
                  unsigned long long *dtmin, int mixed, hipStream_t s);
 // The three fluxes and the centre EMFs of a set of blocks.  L: the launches of KC_FLUX1
 // .. KC_FLUX3 and KC_ECENT; one kernel where they take one tile size, a thread per face
-// and a workgroup per tile, else one after the other.
-void launch_front(const KParams &P, const Launch *L, const double *p, const double *ps, double *const *F,
+// and a workgroup per tile (front_merges), else one after the other.  share (one kernel
+// only): all blocks of a uniform grid, KC_SFLUX1 .. KC_SFLUX3 for the fluxes; ghost
+// faces beyond an x1 or x2 side with a block get the fluxes that the corner EMFs read
+// from that block; their other fluxes, and faces beyond both an x1 and an x2 side, are
+// left alone.
+bool front_merges(const Launch *L);
+void launch_front(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, double *const *F,
                   unsigned long long *dtmin, void *Ec, int mixed, hipStream_t s);
 void launch_emf_centre(const KParams &P, const Launch &L, const double *p, void *Ec, int mixed, hipStream_t s);
 void launch_emf_corner(const KParams &P, const Launch &L, const void *Ec, const void *F1, const void *F2,

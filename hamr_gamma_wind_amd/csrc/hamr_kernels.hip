@@ -22,6 +22,14 @@ int64_t class_work(const BlockDev &B, int cls)
     case KC_FLUX1: return (b1 + 1) * (b2 + 2) * (b3 + 2);
     case KC_FLUX2: return (b1 + 2) * (b2 + 1) * (b3 + 2);
     case KC_FLUX3: return (b1 + 2) * (b2 + 2) * (b3 + 1);
+    case KC_SFLUX1:
+    case KC_SFLUX2:
+    case KC_SFLUX3: {
+        int64_t w = 1;
+        for (int d = 0; d < 3; d++)
+            w *= B.bs[d] + (d == cls - KC_SFLUX1 ? 1 : d == 2 ? 2 : (B.kind[2 * d] != FK_COPY) + (B.kind[2 * d + 1] != FK_COPY));
+        return w;
+    }
     case KC_ECENT: return (b1 + 2) * (b2 + 2) * (b3 + 2);
     case KC_CORNER: return (b1 + 1) * (b2 + 1) * (b3 + 1);
     case KC_INTERIOR: return b1 * b2 * b3;
@@ -1393,23 +1401,23 @@ void launch_emf_corner(const KParams &P, const Launch &L, const void *Ec, const 
                          (double *)E, s);
 }
 
-static bool front_merges(const Launch *L)
+bool front_merges(const Launch *L)
 {
     for (int k = 0; k < 4; k++)
         if (L[k].line || L[k].threads != L[0].threads || L[k].grid != L[k].wl.n) return false;
     return true;
 }
 
-void launch_front(const KParams &P, const Launch *L, const double *p, const double *ps, double *const *F,
+void launch_front(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, double *const *F,
                   unsigned long long *dtmin, void *Ec, int mixed, hipStream_t s)
 {
     if (!front_merges(L)) {
         for (int d = 0; d < 3; d++) launch_flux(P, d + 1, L[d], p, ps, F[d], dtmin, mixed, s);
         launch_emf_centre(P, L[3], p, Ec, mixed, s);
     } else if (mixed) {
-        launch_front_f32(P, L, p, ps, (float *)F[0], (float *)F[1], (float *)F[2], dtmin, (float *)Ec, s);
+        launch_front_f32(P, L, share, p, ps, (float *)F[0], (float *)F[1], (float *)F[2], dtmin, (float *)Ec, s);
     } else {
-        recon_front(P, L, p, ps, (double *)F[0], (double *)F[1], (double *)F[2], dtmin, (double *)Ec, s);
+        recon_front(P, L, share, p, ps, F[0], F[1], F[2], dtmin, (double *)Ec, s);
     }
 }
 

@@ -10,10 +10,10 @@ void launch_flux_f32(const KParams &P, int dir, const Launch &L, const double *p
     recon_flux<float>(P, dir, L, p, ps, F, dtmin, s);
 }
 
-void launch_front_f32(const KParams &P, const Launch *L, const double *p, const double *ps, float *F1, float *F2,
-                      float *F3, unsigned long long *dtmin, float *Ec, hipStream_t s)
+void launch_front_f32(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, float *F1,
+                      float *F2, float *F3, unsigned long long *dtmin, float *Ec, hipStream_t s)
 {
-    recon_front<float>(P, L, p, ps, F1, F2, F3, dtmin, Ec, s);
+    recon_front<float>(P, L, share, p, ps, F1, F2, F3, dtmin, Ec, s);
 }
 
 void launch_emf_centre_f32(const KParams &P, const Launch &L, const double *p, float *Ec, hipStream_t s)

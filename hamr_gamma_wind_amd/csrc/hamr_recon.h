@@ -26,12 +26,14 @@ namespace hamr {
 // HLL flux through face `cell` (cell index of the face's upper cell; (i, j) its
 // metric column) from the reconstructed states pl (lower side) and pr (upper
 // side), fluxcalc2D2's flux and speed part (GPU_program1.cu:811-1045).  G: the
-// metric at the face, bn: the face's normal field.  Stores the 9 fluxes and returns the face's Courant dt, or 1e9 where it is not a
-// valid bound (no signal speed).
+// metric at the face, bn: the face's normal field.  Stores the 9 fluxes, hands those
+// that the corner EMFs use to emf (mass, B of the next direction, B of the one after)
+// and returns the face's Courant dt, or 1e9 where it is not a valid bound (no signal
+// speed).
 template <int DIR, class R>
 __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
                                            R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                           const R bn)
+                                           const R bn, R *emf)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -55,8 +57,13 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
     R *Fb = F + NPR * B.off;
     const Div<R> by_c(cmax + cmin + R(kSMALL));
 #pragma unroll
-    for (int k = 0; k < NPR; k++)
-        gst(Fb + (int64_t)k * K, (uint32_t)cell, by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k])));
+    for (int k = 0; k < NPR; k++) {
+        const R f = by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]));
+        gst(Fb + (int64_t)k * K, (uint32_t)cell, f);
+        if (k == RHO) emf[0] = f;
+        if (k == B1 + DIR % 3) emf[1] = f;
+        if (k == B1 + (DIR + 1) % 3) emf[2] = f;
+    }
     const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
     return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
 }
@@ -67,7 +74,7 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
 template <int DIR, class R>
 __device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
                                             R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                            const R bn)
+                                            const R bn, R *emf)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -99,7 +106,13 @@ __device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B,
                          sizeof(R) == 4 ? G.oma : R(0.), F1);
     R *Fb = F + NPR * B.off + cell;
 #pragma unroll
-    for (int k = 0; k < NPR; k++) Fb[(int64_t)k * K] = G.g * F1[k];
+    for (int k = 0; k < NPR; k++) {
+        const R f = G.g * F1[k];
+        Fb[(int64_t)k * K] = f;
+        if (k == RHO) emf[0] = f;
+        if (k == B1 + DIR % 3) emf[1] = f;
+        if (k == B1 + (DIR + 1) % 3) emf[2] = f;
+    }
     const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
     return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
 }
@@ -108,6 +121,49 @@ __device__ __forceinline__ void dt_reduce(double vdt, unsigned long long *__rest
 {
     vdt = wave_min(vdt);
     if ((threadIdx.x & 63) == 0 && vdt < 1.e9) atomicMin(&dtmin[slot], (unsigned long long)__double_as_longlong(vdt));
+}
+
+// The face's part in the blocks beside it along x1 and x2 (uniform grids): a face in
+// the first or last row of a transverse direction is a ghost face of the block across
+// that side, which does not compute it.  That block's corner EMFs read its mass flux
+// and transverse field fluxes (share_face), and its Courant minimum counts the face, as
+// it does the ghost faces beyond two sides, whose fluxes nothing reads (share_dt, by
+// the whole wavefront; side[d]: the sides of direction d that the lane's face lies at,
+// bit 0 the lower, bit 1 the upper).
+template <int DIR, class R>
+__device__ __forceinline__ void share_face(const BlockDev &B, const int side[2], int cell, const R *emf,
+                                           R *__restrict__ F)
+{
+    const int64_t K = B.ks;
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+        if (d == DIR - 1 || !side[d]) continue;
+        const bool lo = side[d] & 1;
+        const int64_t st = d == 0 ? (int64_t)B.D[1] * B.D[2] : B.D[2];
+        R *f = F + NPR * ((lo ? B.nbr[2 * d] : B.nbr[2 * d + 1]) * K) + (cell + (lo ? B.bs[d] : -B.bs[d]) * st);
+        f[RHO * K] = emf[0];
+        f[(B1 + DIR % 3) * K] = emf[1];
+        f[(B1 + (DIR + 1) % 3) * K] = emf[2];
+    }
+}
+template <int DIR>
+__device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, const int side[2], double vdt,
+                                         unsigned long long *__restrict__ dtmin)
+{
+    if (!__any(side[0] | side[1])) return;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {      // x1: beside, below, above
+        if (DIR == 1 && a) continue;
+#pragma unroll
+        for (int b = 0; b < 3; b++) {  // x2
+            if ((DIR == 2 && b) || (!a && !b)) continue;
+            const bool in = (!a || (side[0] & a)) && (!b || (side[1] & b));
+            if (!__any(in)) continue;
+            int n = a ? B.nbr[a - 1] : B.nbr[2 + b - 1];
+            if (a && b) n = P.blk[n].nbr[2 + b - 1];
+            dt_reduce(in ? vdt : 1.e9, dtmin, n * 3 + DIR - 1);
+        }
+    }
 }
 
 // One thread per face: both parabolas of the face's two cells.
@@ -129,22 +185,30 @@ __device__ __forceinline__ void dt_reduce(double vdt, unsigned long long *__rest
 // at two waves per SIMD: 256 VGPRs with about 20 spilled to scratch ran 1.4x
 // faster than one wave with none spilled.  The FP32 HLLC kernel at four waves
 // (128 VGPRs, 9 spilled) ran 4% faster than at three (139, none spilled).
-template <int DIR, class R, int RS>
+template <int DIR, class R, int RS, bool SHARE = false>
 __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const double *__restrict__ p,
                                           const double *__restrict__ ps, R *__restrict__ F,
                                           unsigned long long *__restrict__ dtmin)
 {
     const int n = it.x;
     const BlockDev &B = P.blk[n];
-    const int e1 = B.bs[0] + (DIR == 1 ? 1 : 2), e2 = B.bs[1] + (DIR == 2 ? 1 : 2), e3 = B.bs[2] + (DIR == 3 ? 1 : 2);
+    // first face and number of faces along each direction: across DIR one ghost layer, with
+    // SHARE along x1 and x2 only where no block of the grid is beyond that side
+    int f0[3], nf[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const bool lo = d != DIR - 1 && !(SHARE && d < 2 && B.kind[2 * d] == FK_COPY);
+        const bool hi = d != DIR - 1 && !(SHARE && d < 2 && B.kind[2 * d + 1] == FK_COPY);
+        f0[d] = lo ? NG - 1 : NG;
+        nf[d] = B.bs[d] + (d == DIR - 1 ? 1 : (int)lo + (int)hi);
+    }
     const int t = it.y * blockDim.x + threadIdx.x;
     double vdt = 1.e9;
-    if (t < e1 * e2 * e3) {
+    int side[2] = {0, 0};
+    if (t < nf[0] * nf[1] * nf[2]) {
         int a, b, c;
-        region_index(t, e2, e3, a, b, c);
-        const int i = a + (DIR == 1 ? NG : NG - 1);
-        const int j = b + (DIR == 2 ? NG : NG - 1);
-        const int z = c + (DIR == 3 ? NG : NG - 1);
+        region_index(t, nf[1], nf[2], a, b, c);
+        const int i = a + f0[0], j = b + f0[1], z = c + f0[2];
         const int64_t K = B.ks;
         const int64_t cell = ((int64_t)i * B.D[1] + j) * B.D[2] + z;
         const int64_t sd = (DIR == 1) ? (int64_t)B.D[1] * B.D[2] : (DIR == 2) ? (int64_t)B.D[2] : 1;
@@ -176,10 +240,23 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
         const R bn = (R)gld(ps + 3 * B.off + (DIR - 1) * K, (uint32_t)cell);
 #pragma unroll
         for (int k = 4; k < KTOT; k++) one(k);
-        if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
-        else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+        R emf[3];
+        if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+        else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+        if constexpr (SHARE) {
+            const int x[2] = {i, j};
+#pragma unroll
+            for (int d = 0; d < 2; d++)
+                if (d != DIR - 1)
+                    side[d] = (x[d] == NG && B.kind[2 * d] == FK_COPY ? 1 : 0)
+                        | (x[d] == NG + B.bs[d] - 1 && B.kind[2 * d + 1] == FK_COPY ? 2 : 0);
+            share_face<DIR>(B, side, (int)cell, emf, F);
+        }
     }
-    if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
+    if (dtmin) {
+        dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
+        if constexpr (SHARE) share_dt<DIR>(P, B, side, vdt, dtmin);
+    }
 }
 
 template <int DIR, class R, int RS>
@@ -311,8 +388,9 @@ k_flux_lines(KParams P, WorkList wl, const double *__restrict__ p, const double 
         if (fact) {
             const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
             const R bn = (R)ps[3 * B.off + (DIR - 1) * (int64_t)B.ks + cell];
-            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
-            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn);
+            R emf[3];
+            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
         }
         if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
         // the next item's first barrier orders its LDS writes after these reads
@@ -371,7 +449,7 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // 42.5 -> 40.1, HLLC 256x128x128 14.8 -> 13.4; the step of 384x192x192 by chunk
 // (items): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
 constexpr int kFrontChunk = 4096;
-template <class R, int RS>
+template <class R, int RS, bool SHARE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
 k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__restrict__ ps, R *__restrict__ F1,
         R *__restrict__ F2, R *__restrict__ F3, unsigned long long *__restrict__ dtmin, R *__restrict__ Ec)
@@ -387,9 +465,9 @@ k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__r
         idx += L.chunked;
     }
     const int2 it = wl_get(L.wl[cls], idx);
-    if (cls == 0) flux_item<1, R, RS>(P, it, p, ps, F1, dtmin);
-    else if (cls == 1) flux_item<2, R, RS>(P, it, p, ps, F2, dtmin);
-    else if (cls == 2) flux_item<3, R, RS>(P, it, p, ps, F3, dtmin);
+    if (cls == 0) flux_item<1, R, RS, SHARE>(P, it, p, ps, F1, dtmin);
+    else if (cls == 1) flux_item<2, R, RS, SHARE>(P, it, p, ps, F2, dtmin);
+    else if (cls == 2) flux_item<3, R, RS, SHARE>(P, it, p, ps, F3, dtmin);
     else emf_centre_item(P, it, p, Ec);
 }
 
@@ -508,8 +586,8 @@ void recon_flux(const KParams &P, int dir, const Launch &L, const double *p, con
 }
 
 template <class R>
-void recon_front(const KParams &P, const Launch *L, const double *p, const double *ps, R *F1, R *F2, R *F3,
-                 unsigned long long *dtmin, R *Ec, hipStream_t s)
+void recon_front(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, R *F1, R *F2,
+                 R *F3, unsigned long long *dtmin, R *Ec, hipStream_t s)
 {
     FrontLists f;
     int n = 0;
@@ -521,10 +599,14 @@ void recon_front(const KParams &P, const Launch *L, const double *p, const doubl
     for (int k = 1; k < 4; k++) f.chunked = L[k].wl.n < f.chunked ? L[k].wl.n : f.chunked;
     f.chunked = sizeof(R) == 4 && f.chunked >= 4 * kFrontChunk ? f.chunked / kFrontChunk * kFrontChunk : 0;
     if (n <= 0) return;
-    if (P.riemann == 1)
-        hipLaunchKernelGGL((k_front<R, 1>), dim3((unsigned)n), bdim(L[0]), 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
-    else
-        hipLaunchKernelGGL((k_front<R, 0>), dim3((unsigned)n), bdim(L[0]), 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+    const dim3 g((unsigned)n), b = bdim(L[0]);
+    if (P.riemann == 1) {
+        if (share) hipLaunchKernelGGL((k_front<R, 1, true>), g, b, 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+        else hipLaunchKernelGGL((k_front<R, 1, false>), g, b, 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+    } else {
+        if (share) hipLaunchKernelGGL((k_front<R, 0, true>), g, b, 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+        else hipLaunchKernelGGL((k_front<R, 0, false>), g, b, 0, s, P, f, p, ps, F1, F2, F3, dtmin, Ec);
+    }
 }
 
 template <class R>
@@ -545,8 +627,8 @@ void recon_emf_corner(const KParams &P, const Launch &L, const R *Ec, const R *F
 // The FP32 instantiations (hamr_kernels_f32.hip).
 void launch_flux_f32(const KParams &P, int dir, const Launch &L, const double *p, const double *ps, float *F,
                      unsigned long long *dtmin, hipStream_t s);
-void launch_front_f32(const KParams &P, const Launch *L, const double *p, const double *ps, float *F1, float *F2,
-                      float *F3, unsigned long long *dtmin, float *Ec, hipStream_t s);
+void launch_front_f32(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, float *F1,
+                      float *F2, float *F3, unsigned long long *dtmin, float *Ec, hipStream_t s);
 void launch_emf_centre_f32(const KParams &P, const Launch &L, const double *p, float *Ec, hipStream_t s);
 void launch_emf_corner_f32(const KParams &P, const Launch &L, const float *Ec, const float *F1, const float *F2,
                            const float *F3, float *E, hipStream_t s);
