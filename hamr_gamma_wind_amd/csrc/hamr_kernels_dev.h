@@ -1,5 +1,5 @@
 // hamr_kernels_dev.h -- device helpers shared by the kernel translation units:
-// work-list walking, metric addressing and loads, wavefront reductions.
+// work-list walking, metric addressing and loads.
 #pragma once
 
 #include "hamr_kernels.h"
@@ -90,13 +90,6 @@ __device__ __forceinline__ double block_Dt(const KParams &P, const BlockDev &B, 
 {
     const double Dt = dt_ptr ? dt_ptr[0] * dt_mult : Dt_val;
     return P.las_s >= 0 ? Dt * (double)(B.tl > 0 ? B.tl : 1) : Dt;
-}
-
-__device__ __forceinline__ double wave_min(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    return v;
 }
 
 // Where the update and face-field kernels also write cell (i, j, z) (index g)

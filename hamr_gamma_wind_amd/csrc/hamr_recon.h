@@ -28,12 +28,11 @@ namespace hamr {
 // side), fluxcalc2D2's flux and speed part (GPU_program1.cu:811-1045).  G: the
 // metric at the face, bn: the face's normal field.  Stores the 9 fluxes, hands those
 // that the corner EMFs use to emf (mass, B of the next direction, B of the one after)
-// and returns the face's Courant dt, or 1e9 where it is not a valid bound (no signal
-// speed).
+// and returns the face's largest signal speed.
 template <int DIR, class R>
-__device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
-                                           R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                           const R bn, R *emf)
+__device__ __forceinline__ R hll_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
+                                      R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
+                                      const R bn, R *emf)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -64,17 +63,16 @@ __device__ __forceinline__ double hll_face(const KParams &P, const BlockDev &B, 
         if (k == B1 + DIR % 3) emf[1] = f;
         if (k == B1 + (DIR + 1) % 3) emf[2] = f;
     }
-    const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
-    return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
+    return ctop;
 }
 
-// HLLC flux through the same face (fluxcalc2D_FT, GPU_hllc.h:3-247): the
-// Courant dt from the coordinate speeds as in hll_face, the flux from the
+// HLLC flux through the same face (fluxcalc2D_FT, GPU_hllc.h:3-247): the largest
+// signal speed from the coordinate speeds as in hll_face, the flux from the
 // orthonormal-frame solver of hamr_hllc.h with the face's tetrad.
 template <int DIR, class R>
-__device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
-                                            R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                            const R bn, R *emf)
+__device__ __forceinline__ R hllc_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
+                                       R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
+                                       const R bn, R *emf)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -113,14 +111,23 @@ __device__ __forceinline__ double hllc_face(const KParams &P, const BlockDev &B,
         if (k == B1 + DIR % 3) emf[1] = f;
         if (k == B1 + (DIR + 1) % 3) emf[2] = f;
     }
-    const double v = P.cour * B.dx[DIR - 1] / (double)ctop;
-    return (v < 1.e9 && v > 1.e-6) ? v : 1.e9;
+    return ctop;
 }
 
-__device__ __forceinline__ void dt_reduce(double vdt, unsigned long long *__restrict__ dtmin, int slot)
+// A wavefront's part in a Courant minimum, from its faces' largest signal speeds c (0:
+// none): the step cour dx / c where it lies between 1e-6 and 1e9.  The quotient falls
+// with c, so the faces' largest c gives their smallest step and one division serves the
+// wavefront.
+template <class R>
+__device__ __forceinline__ void dt_reduce(const KParams &P, double dx, R c, unsigned long long *__restrict__ dtmin,
+                                          int slot)
 {
-    vdt = wave_min(vdt);
-    if ((threadIdx.x & 63) == 0 && vdt < 1.e9) atomicMin(&dtmin[slot], (unsigned long long)__double_as_longlong(vdt));
+    const double cd = P.cour * dx;
+    c = ((double)c > cd * 1.e-9 && (double)c < cd * 1.e6) ? c : R(0.);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) c = mymax(c, (R)__shfl_xor(c, off, 64));
+    const double v = cd / (double)c;
+    if ((threadIdx.x & 63) == 0 && v < 1.e9) atomicMin(&dtmin[slot], (unsigned long long)__double_as_longlong(v));
 }
 
 // The face's part in the blocks beside it along x1 and x2 (uniform grids): a face in
@@ -146,8 +153,8 @@ __device__ __forceinline__ void share_face(const BlockDev &B, const int side[2],
         f[(B1 + (DIR + 1) % 3) * K] = emf[2];
     }
 }
-template <int DIR>
-__device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, const int side[2], double vdt,
+template <int DIR, class R>
+__device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, const int side[2], R c,
                                          unsigned long long *__restrict__ dtmin)
 {
     if (!__any(side[0] | side[1])) return;
@@ -161,7 +168,7 @@ __device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, co
             if (!__any(in)) continue;
             int n = a ? B.nbr[a - 1] : B.nbr[2 + b - 1];
             if (a && b) n = P.blk[n].nbr[2 + b - 1];
-            dt_reduce(in ? vdt : 1.e9, dtmin, n * 3 + DIR - 1);
+            dt_reduce(P, B.dx[DIR - 1], in ? c : R(0.), dtmin, n * 3 + DIR - 1);
         }
     }
 }
@@ -203,7 +210,7 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
         nf[d] = B.bs[d] + (d == DIR - 1 ? 1 : (int)lo + (int)hi);
     }
     const int t = it.y * blockDim.x + threadIdx.x;
-    double vdt = 1.e9;
+    R ctop = R(0.);
     int side[2] = {0, 0};
     if (t < nf[0] * nf[1] * nf[2]) {
         int a, b, c;
@@ -241,8 +248,8 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
 #pragma unroll
         for (int k = 4; k < KTOT; k++) one(k);
         R emf[3];
-        if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
-        else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+        if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+        else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
         if constexpr (SHARE) {
             const int x[2] = {i, j};
 #pragma unroll
@@ -254,8 +261,8 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
         }
     }
     if (dtmin) {
-        dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
-        if constexpr (SHARE) share_dt<DIR>(P, B, side, vdt, dtmin);
+        dt_reduce(P, B.dx[DIR - 1], ctop, dtmin, n * 3 + DIR - 1);
+        if constexpr (SHARE) share_dt<DIR>(P, B, side, ctop, dtmin);
     }
 }
 
@@ -384,15 +391,15 @@ k_flux_lines(KParams P, WorkList wl, const double *__restrict__ p, const double 
         if (nfd == 33 || nfd == 65) line_tile_states<DIR, R, 33>(B, it.y, p, sm, pl, pr, fact, cell, i, j);
         else if (nfd == 17) line_tile_states<DIR, R, 17>(B, it.y, p, sm, pl, pr, fact, cell, i, j);
         else line_tile_states<DIR, R, 0>(B, it.y, p, sm, pl, pr, fact, cell, i, j);
-        double vdt = 1.e9;
+        R ctop = R(0.);
         if (fact) {
             const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
             const R bn = (R)ps[3 * B.off + (DIR - 1) * (int64_t)B.ks + cell];
             R emf[3];
-            if constexpr (RS == 1) vdt = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
-            else vdt = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+            if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+            else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
         }
-        if (dtmin) dt_reduce(vdt, dtmin, n * 3 + DIR - 1);
+        if (dtmin) dt_reduce(P, B.dx[DIR - 1], ctop, dtmin, n * 3 + DIR - 1);
         // the next item's first barrier orders its LDS writes after these reads
     }
 }
@@ -448,6 +455,13 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // -> 4.28, 256x128x128 17.0 -> 16.5, HLLC 96x72x60 3.11 -> 2.71; mixed 384x192x192
 // 42.5 -> 40.1, HLLC 256x128x128 14.8 -> 13.4; the step of 384x192x192 by chunk
 // (items): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
+//
+// SHARE (uniform grids): ghost faces along x1 and x2 beyond a side with a block are
+// computed by that block only and written to both: 8% fewer faces on 32^3 blocks, 20%
+// on 16x8x8.  256x128x128 FP64 16.17 -> 15.80 ms a pass, HLLC 96x72x60 2.68 -> 2.59,
+// 42x25x39 blocks 4.24 -> 4.18, 384x192x192 mixed 39.85 -> 39.57.  Along x3 as well the
+// blocks would write single values into the rows beside them: no faster than computing
+// the two faces more per row (384x192x192 2.09 and 2.07 ms a launch).
 constexpr int kFrontChunk = 4096;
 template <class R, int RS, bool SHARE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
