@@ -62,14 +62,14 @@ template <> struct Div<double> {
 };
 #endif
 
-// a / 3, correctly rounded: Div's last step by a constant reciprocal, without its
-// treatment of infinite a (the quotient is then NaN, not infinite).
-template <class R> HD R third(R a) { return Div<R>(R(3.))(a); }
+// a / 6: Div's quotient by a constant reciprocal, without its treatment of infinite a
+// (the quotient is then NaN, not infinite).
+template <class R> HD R sixth(R a) { return Div<R>(R(6.))(a); }
 #if HAMR_DEVICE_ARITH
-template <> HD double third<double>(double a)
+template <> HD double sixth<double>(double a)
 {
-    const double y = 1. / 3., q = a * y;
-    return fma(fma(-3., q, a), y, q);
+    const double y = 1. / 6., q = a * y;
+    return fma(fma(-6., q, a), y, q);
 }
 #endif
 

@@ -255,7 +255,7 @@ template <class R> HD R mc_slope(R ym, R y0, R yp)
 // (GPU_interp.h:89-90): a_{c+1/2} = (y_c + y_{c+1})/2 - (dq_{c+1} - dq_c)/6.
 template <class R> HD R ppm_face(R ym, R yp, R dqm, R dqp)
 {
-    return R(0.5) * (yp + ym) - Div<R>(R(6.0))(dqp - dqm);
+    return R(0.5) * (yp + ym) - sixth(dqp - dqm);
 }
 
 // CW84 monotonicity limits of the parabola of a cell with mean x3 and interface
@@ -272,26 +272,11 @@ template <class R> HD void ppm_limit(R x3, R l, R r, R &lout, R &rout)
     rout = r;
 }
 
-// Half of mc_slope, and ppm_face from half slopes: the same values with a power of
-// two taken out (2 dq_-, 2 dq_+ and dq_c / 2 are compared as dq_-, dq_+ and dq_c / 4,
-// (dq_{c+1} - dq_c) / 6 is a third of the halves' difference), 5 products fewer per
-// six-point stencil.
-template <class R> HD R half_slope(R ym, R y0, R yp)
-{
-    const R dm = y0 - ym, dp = yp - y0, dc = yp - ym;
-    const R v = copysign(fmin(R(0.25) * fabs(dc), fmin(fabs(dm), fabs(dp))), dc);
-    return (dm * dp > R(0.)) ? v : R(0.);
-}
-template <class R> HD R ppm_face_half(R ym, R yp, R hm, R hp)
-{
-    return R(0.5) * (yp + ym) - third(hp - hm);
-}
-
 // GPU_interp.h:60-111: CW84 PPM with MC (factor 2) slopes; l = a_L, r = a_R.
 template <class R> HD void para(R x1, R x2, R x3, R x4, R x5, R &lout, R &rout)
 {
-    const R h1 = half_slope(x1, x2, x3), h2 = half_slope(x2, x3, x4), h3 = half_slope(x3, x4, x5);
-    ppm_limit(x3, ppm_face_half(x2, x3, h1, h2), ppm_face_half(x3, x4, h2, h3), lout, rout);
+    const R dq1 = mc_slope(x1, x2, x3), dq2 = mc_slope(x2, x3, x4), dq3 = mc_slope(x3, x4, x5);
+    ppm_limit(x3, ppm_face(x2, x3, dq1, dq2), ppm_face(x3, x4, dq2, dq3), lout, rout);
 }
 
 // ---------------------------------------------------------------------------

@@ -339,7 +339,7 @@ __device__ __forceinline__ void line_tile_states(const BlockDev &B, int item, co
             ym[v] = (R)y[-sdir];
             y0[v] = (R)y[0];
             yp[v] = (R)y[sdir];
-            dq[v] = half_slope(ym[v], y0[v], yp[v]);
+            dq[v] = mc_slope(ym[v], y0[v], yp[v]);
             DQ[v * T + t] = dq[v];
         }
         v++;
@@ -350,8 +350,8 @@ __device__ __forceinline__ void line_tile_states(const BlockDev &B, int item, co
     for (int v = 0; v < NV; v++) {
         if (edge) {
             R l, r;
-            ppm_limit(y0[v], ppm_face_half(ym[v], y0[v], DQ[v * T + t - sn], dq[v]),
-                      ppm_face_half(y0[v], yp[v], dq[v], DQ[v * T + t + sn]), l, r);
+            ppm_limit(y0[v], ppm_face(ym[v], y0[v], DQ[v * T + t - sn], dq[v]),
+                      ppm_face(y0[v], yp[v], dq[v], DQ[v * T + t + sn]), l, r);
             le[v] = l;
             RE[v * T + t] = r;
         }
