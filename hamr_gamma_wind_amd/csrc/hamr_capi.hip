@@ -252,6 +252,8 @@ static int d2h(hamr_ctx *c, void *dst, const void *src, size_t bytes)
 static int build_class_lists(hamr_ctx *c)
 {
     const int nb = nblk_of(c);
+    std::vector<int2> all;
+    size_t first[KC_N][3];
     for (int cls = 0; cls < KC_N; cls++) {
         // block list of the class: every block, except that the ghost fill of a
         // multi-level set has its own kernels, which serve only the outflow and
@@ -293,12 +295,16 @@ static int build_class_lists(hamr_ctx *c)
             }
             L.n[ti] = (int)items.size();
             L.lds_cols[ti] = cols;
-            if (!items.empty()) {
-                if (dalloc(c, &L.items[ti], items.size())) return -1;
-                if (h2d(c, L.items[ti], items.data(), items.size() * sizeof(int2))) return -1;
-            }
+            first[cls][ti] = all.size();
+            all.insert(all.end(), items.begin(), items.end());
         }
     }
+    // one allocation and one copy for all lists
+    int2 *dev = nullptr;
+    if (dalloc(c, &dev, all.size()) || h2d(c, dev, all.data(), all.size() * sizeof(int2))) return -1;
+    for (int cls = 0; cls < KC_N; cls++)
+        for (int ti = 0; ti < 3; ti++)
+            if (c->cl[cls].n[ti]) c->cl[cls].items[ti] = dev + first[cls][ti];
     return 0;
 }
 
