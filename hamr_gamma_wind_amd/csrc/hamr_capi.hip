@@ -46,6 +46,13 @@ constexpr int kSlotClass[TS_N] = {KC_FLUX1, KC_FLUX2, KC_FLUX3, KC_ECENT, KC_COR
 // unequal times.
 static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_FLAGS ? 0 : 1; }
 
+// Default tile of the fluxes and centre EMFs (index into kTiles, 128 threads): smaller
+// tiles leave fewer lanes idle at the end of a block and of the launch.  256, 128, 64
+// threads, ms a step: 42x25x39 blocks FP64 0.980, 0.968, 0.970; 256x128x128 FP64 3.74, 3.68,
+// 3.69, mixed 2.76, 2.74, 2.77, HLLC mixed 3.09, 3.07, 3.09; HLLC 96x72x60 FP64 0.614, 0.601,
+// 0.594; 384x192x192 mixed 9.24, 9.21, 9.31.
+constexpr int kFrontTile = 1;
+
 struct TuneCfg {
     int tile = kDefaultTile;  // index into kTiles
     int grid = 0;             // workgroups; 0: one per item
@@ -413,8 +420,10 @@ static int init_device(hamr_ctx *c)
     if (h2d(c, c->io_roff, c->roff.data(), (nb + 1) * sizeof(int64_t))) return -1;
     if (h2d(c, c->io_doff, c->doff.data(), (nb + 1) * sizeof(int64_t))) return -1;
     if (build_class_lists(c)) return -1;
-    for (int slot = 0; slot < TS_N; slot++)
+    for (int slot = 0; slot < TS_N; slot++) {
         if (kSlotClass[slot] >= 0) c->tune[slot].swz = default_swz(kSlotClass[slot]);
+        if (slot <= TS_ECENT) c->tune[slot].tile = kFrontTile;
+    }
     KParams &P = c->P;
     P.gam = c->d.gam;
     P.cour = c->d.cour;

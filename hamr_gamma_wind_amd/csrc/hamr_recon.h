@@ -462,7 +462,7 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // 42x25x39 blocks 4.24 -> 4.18, 384x192x192 mixed 39.85 -> 39.57.  Along x3 as well the
 // blocks would write single values into the rows beside them: no faster than computing
 // the two faces more per row (384x192x192 2.09 and 2.07 ms a launch).
-constexpr int kFrontChunk = 4096;
+constexpr int kFrontChunk = 1 << 20;  // threads: 4096 items of 256
 template <class R, int RS, bool SHARE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
 k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__restrict__ ps, R *__restrict__ F1,
@@ -471,8 +471,9 @@ k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__r
     const int w = blockIdx.x;
     int cls, idx;
     if (w < 4 * L.chunked) {
-        cls = (w / kFrontChunk) & 3;
-        idx = w / (4 * kFrontChunk) * kFrontChunk + w % kFrontChunk;
+        const int chunk = kFrontChunk / (int)blockDim.x, q = w / chunk;
+        cls = q & 3;
+        idx = (q >> 2) * chunk + (w - q * chunk);
     } else {
         idx = w - 4 * L.chunked;
         for (cls = 0; cls < 3 && idx >= L.wl[cls].n - L.chunked; cls++) idx -= L.wl[cls].n - L.chunked;
@@ -611,7 +612,8 @@ void recon_front(const KParams &P, const Launch *L, bool share, const double *p,
     }
     f.chunked = L[0].wl.n;
     for (int k = 1; k < 4; k++) f.chunked = L[k].wl.n < f.chunked ? L[k].wl.n : f.chunked;
-    f.chunked = sizeof(R) == 4 && f.chunked >= 4 * kFrontChunk ? f.chunked / kFrontChunk * kFrontChunk : 0;
+    const int chunk = kFrontChunk / L[0].threads;
+    f.chunked = sizeof(R) == 4 && f.chunked >= 4 * chunk ? f.chunked / chunk * chunk : 0;
     if (n <= 0) return;
     const dim3 g((unsigned)n), b = bdim(L[0]);
     if (P.riemann == 1) {
