@@ -144,10 +144,9 @@ void launch_flux(const KParams &P, int dir, const Launch &L, const double *p, co
 // The three fluxes and the centre EMFs of a set of blocks.  L: the launches of KC_FLUX1
 // .. KC_FLUX3 and KC_ECENT; one kernel where they take one tile size, a thread per face
 // and a workgroup per tile (front_merges), else one after the other.  share (one kernel
-// only): all blocks of a uniform grid, KC_SFLUX1 .. KC_SFLUX3 for the fluxes; ghost
-// faces beyond an x1 or x2 side with a block get the fluxes that the corner EMFs read
-// from that block; their other fluxes, and faces beyond both an x1 and an x2 side, are
-// left alone.
+// only): all blocks of a uniform grid, their ghosts filled, KC_SFLUX1 .. KC_SFLUX3 for
+// the fluxes; ghost faces beyond an x1 or x2 side with a block get their fluxes from
+// that block.  F, Ec and dtmin are the same in every form.
 bool front_merges(const Launch *L);
 void launch_front(const KParams &P, const Launch *L, bool share, const double *p, const double *ps, double *const *F,
                   unsigned long long *dtmin, void *Ec, int mixed, hipStream_t s);

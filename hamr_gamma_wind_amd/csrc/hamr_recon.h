@@ -26,13 +26,12 @@ namespace hamr {
 // HLL flux through face `cell` (cell index of the face's upper cell; (i, j) its
 // metric column) from the reconstructed states pl (lower side) and pr (upper
 // side), fluxcalc2D2's flux and speed part (GPU_program1.cu:811-1045).  G: the
-// metric at the face, bn: the face's normal field.  Stores the 9 fluxes, hands those
-// that the corner EMFs use to emf (mass, B of the next direction, B of the one after)
-// and returns the face's largest signal speed.
+// metric at the face, bn: the face's normal field.  Stores the 9 fluxes, returns them
+// in f and the face's largest signal speed.
 template <int DIR, class R>
 __device__ __forceinline__ R hll_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
                                       R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                      const R bn, R *emf)
+                                      const R bn, R *f)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -57,11 +56,8 @@ __device__ __forceinline__ R hll_face(const KParams &P, const BlockDev &B, const
     const Div<R> by_c(cmax + cmin + R(kSMALL));
 #pragma unroll
     for (int k = 0; k < NPR; k++) {
-        const R f = by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]));
-        gst(Fb + (int64_t)k * K, (uint32_t)cell, f);
-        if (k == RHO) emf[0] = f;
-        if (k == B1 + DIR % 3) emf[1] = f;
-        if (k == B1 + (DIR + 1) % 3) emf[2] = f;
+        f[k] = by_c(cmax * t1[k] + cmin * t3[k] - cmax * cmin * (t4[k] - t2[k]));
+        gst(Fb + (int64_t)k * K, (uint32_t)cell, f[k]);
     }
     return ctop;
 }
@@ -72,7 +68,7 @@ __device__ __forceinline__ R hll_face(const KParams &P, const BlockDev &B, const
 template <int DIR, class R>
 __device__ __forceinline__ R hllc_face(const KParams &P, const BlockDev &B, const double *__restrict__ ps, R *pl,
                                        R *pr, int i, int j, int64_t cell, R *__restrict__ F, const Geom<R> &G,
-                                       const R bn, R *emf)
+                                       const R bn, R *f)
 {
     const int64_t K = B.ks;
     pl[B1 + DIR - 1] = bn;
@@ -105,11 +101,8 @@ __device__ __forceinline__ R hllc_face(const KParams &P, const BlockDev &B, cons
     R *Fb = F + NPR * B.off + cell;
 #pragma unroll
     for (int k = 0; k < NPR; k++) {
-        const R f = G.g * F1[k];
-        Fb[(int64_t)k * K] = f;
-        if (k == RHO) emf[0] = f;
-        if (k == B1 + DIR % 3) emf[1] = f;
-        if (k == B1 + (DIR + 1) % 3) emf[2] = f;
+        f[k] = G.g * F1[k];
+        Fb[(int64_t)k * K] = f[k];
     }
     return ctop;
 }
@@ -132,26 +125,30 @@ __device__ __forceinline__ void dt_reduce(const KParams &P, double dx, R c, unsi
 
 // The face's part in the blocks beside it along x1 and x2 (uniform grids): a face in
 // the first or last row of a transverse direction is a ghost face of the block across
-// that side, which does not compute it.  That block's corner EMFs read its mass flux
-// and transverse field fluxes (share_face), and its Courant minimum counts the face, as
-// it does the ghost faces beyond two sides, whose fluxes nothing reads (share_dt, by
-// the whole wavefront; side[d]: the sides of direction d that the lane's face lies at,
-// bit 0 the lower, bit 1 the upper).
+// that side, which does not compute it, and an x3 face at two sides one of the block
+// across both.  Those blocks get its fluxes (share_face), and their Courant minima
+// count it (share_dt, by the whole wavefront).  side[d]: the sides of direction d that
+// the lane's face lies at, bit 0 the lower, bit 1 the upper.
 template <int DIR, class R>
-__device__ __forceinline__ void share_face(const BlockDev &B, const int side[2], int cell, const R *emf,
+__device__ __forceinline__ void share_face(const KParams &P, const BlockDev &B, const int side[2], int cell, const R *f,
                                            R *__restrict__ F)
 {
     const int64_t K = B.ks;
+    int n[2], shift[2];
+    auto put = [&](int m, int sh) {
+        R *o = F + NPR * (m * K) + (cell + sh);
+#pragma unroll
+        for (int k = 0; k < NPR; k++) o[k * K] = f[k];
+    };
 #pragma unroll
     for (int d = 0; d < 2; d++) {
         if (d == DIR - 1 || !side[d]) continue;
         const bool lo = side[d] & 1;
-        const int64_t st = d == 0 ? (int64_t)B.D[1] * B.D[2] : B.D[2];
-        R *f = F + NPR * ((lo ? B.nbr[2 * d] : B.nbr[2 * d + 1]) * K) + (cell + (lo ? B.bs[d] : -B.bs[d]) * st);
-        f[RHO * K] = emf[0];
-        f[(B1 + DIR % 3) * K] = emf[1];
-        f[(B1 + (DIR + 1) % 3) * K] = emf[2];
+        n[d] = lo ? B.nbr[2 * d] : B.nbr[2 * d + 1];
+        shift[d] = (lo ? B.bs[d] : -B.bs[d]) * (d == 0 ? B.D[1] * B.D[2] : B.D[2]);
+        put(n[d], shift[d]);
     }
+    if (DIR == 3 && side[0] && side[1]) put(P.blk[n[0]].nbr[side[1] & 1 ? 2 : 3], shift[0] + shift[1]);
 }
 template <int DIR, class R>
 __device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, const int side[2], R c,
@@ -247,9 +244,9 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
         const R bn = (R)gld(ps + 3 * B.off + (DIR - 1) * K, (uint32_t)cell);
 #pragma unroll
         for (int k = 4; k < KTOT; k++) one(k);
-        R emf[3];
-        if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
-        else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+        R f[NPR];
+        if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, f);
+        else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, f);
         if constexpr (SHARE) {
             const int x[2] = {i, j};
 #pragma unroll
@@ -257,7 +254,7 @@ __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const
                 if (d != DIR - 1)
                     side[d] = (x[d] == NG && B.kind[2 * d] == FK_COPY ? 1 : 0)
                         | (x[d] == NG + B.bs[d] - 1 && B.kind[2 * d + 1] == FK_COPY ? 2 : 0);
-            share_face<DIR>(B, side, (int)cell, emf, F);
+            share_face<DIR>(P, B, side, (int)cell, f, F);
         }
     }
     if (dtmin) {
@@ -395,9 +392,9 @@ k_flux_lines(KParams P, WorkList wl, const double *__restrict__ p, const double 
         if (fact) {
             const Geom<R> G = load_geom<R>(P, B, DIR == 1 ? FACE1 : DIR == 2 ? FACE2 : FACE3, (int64_t)i * B.D[1] + j);
             const R bn = (R)ps[3 * B.off + (DIR - 1) * (int64_t)B.ks + cell];
-            R emf[3];
-            if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
-            else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, emf);
+            R f[NPR];
+            if constexpr (RS == 1) ctop = hllc_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, f);
+            else ctop = hll_face<DIR>(P, B, ps, pl, pr, i, j, cell, F, G, bn, f);
         }
         if (dtmin) dt_reduce(P, B.dx[DIR - 1], ctop, dtmin, n * 3 + DIR - 1);
         // the next item's first barrier orders its LDS writes after these reads
@@ -457,11 +454,14 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // (items): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
 //
 // SHARE (uniform grids): ghost faces along x1 and x2 beyond a side with a block are
-// computed by that block only and written to both: 8% fewer faces on 32^3 blocks, 20%
-// on 16x8x8.  256x128x128 FP64 16.17 -> 15.80 ms a pass, HLLC 96x72x60 2.68 -> 2.59,
-// 42x25x39 blocks 4.24 -> 4.18, 384x192x192 mixed 39.85 -> 39.57.  Along x3 as well the
-// blocks would write single values into the rows beside them: no faster than computing
-// the two faces more per row (384x192x192 2.09 and 2.07 ms a launch).
+// computed by that block only, which writes all their fluxes to both: 8% fewer faces on
+// 32^3 blocks, 20% on 16x8x8.  Without and with it, ms a pass: 42x25x39 blocks FP64 4.18,
+// 4.13; 256x128x128 FP64 16.03, 15.75, HLLC mixed 13.31, 13.18; HLLC 96x72x60 2.64, 2.58;
+// 384x192x192 mixed 40.18, 39.86.  (With only the fluxes written that the face update's
+// EMFs read: 0.1-0.7% less time, but stale values left in HAMR_F1-F3 and on edges of
+// HAMR_EMF.)  Along x3 as well the blocks would write single values into the rows beside
+// them: no faster than computing the two faces more per row (384x192x192 2.09 and 2.07
+// ms a launch).
 constexpr int kFrontChunk = 1 << 20;  // threads: 4096 items of 256
 template <class R, int RS, bool SHARE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))

@@ -72,8 +72,7 @@ enum {
     HAMR_PS = 1,    /* face fields, 3 */
     HAMR_PH = 2,    /* half-step primitives, 9 */
     HAMR_PSH = 3,   /* half-step face fields, 3 */
-    HAMR_F1 = 4,    /* fluxes through the lower x1 faces, 9 (after a batched step of a uniform grid the
-                     * ghost faces hold only what the corner EMFs read: mass and transverse field) */
+    HAMR_F1 = 4,    /* fluxes through the lower x1 faces, 9 */
     HAMR_F2 = 5,
     HAMR_F3 = 6,
     HAMR_EMF = 7,   /* corner EMF E_1, E_2, E_3 */
