@@ -36,7 +36,9 @@ class Stage(torch.autograd.Function):
     def backward(ctx, gU):
         P, PS = ctx.saved_tensors
         hctx = ctx.hctx
-        w = gU.contiguous()  # the weights of ghost cells are not read
+        # the values themselves (a lazily negated view keeps its sign in a flag); the
+        # weights of ghost cells are not read
+        w = gU.resolve_neg().contiguous()
         gP = torch.empty_like(P)
         gPS = torch.empty_like(PS)
         torch.cuda.current_stream().synchronize()
