@@ -29,13 +29,17 @@ template <> HD float rpow<float>(float a, float e) { return __builtin_amdgcn_exp
 // and each quotient takes the last step of the IEEE division on it (product,
 // residual, correction, special values): 4 instructions instead of 11 with a
 // quarter-rate estimate among them.  These are the operations the compiler's
-// own division performs when it does not rescale its operands, so the result is
-// the same correctly rounded quotient; where it would rescale (a numerator below
-// 2^-969, a divisor or quotient at the ends of the exponent range) the result is
-// within one unit in the last place.  Zeros, infinities and NaNs divide as IEEE.
-// The FP64 flux kernel has 54 divisions by 32 divisors per face (24 of them by
-// the constant 6), the update 66 by 20 and 9 by 6 in every Newton iteration.
-// In FP32 the quotient is a * rcp(b), as dv.
+// own division performs when it does not rescale its operands, so for a numerator
+// from 2^-969 on and a divisor above 2^-1024 the result is the same correctly
+// rounded quotient, an overflowing one the same infinity (div_fixup makes it of the
+// NaN that the residual then is); a smaller numerator gives it within one unit in
+// the last place.  A divisor of 2^-1024 or less, whose reciprocal overflows, gives
+// an infinity also where the quotient is finite: no divisor of the step comes near
+// (densities, enthalpies, Lorentz factors, wave speeds with kSMALL added, metric
+// determinants).  Zeros, infinities and NaNs divide as IEEE.
+// The FP64 flux kernel forms 31 quotients by 10 divisors a face, the update 60 by 17
+// (9 by 6 of them in every Newton iteration).  In FP32 the quotient is a * rcp(b),
+// as dv.
 template <class R> struct Div {
     R d;
     HD explicit Div(R b) : d(b) {}
@@ -62,8 +66,8 @@ template <> struct Div<double> {
 };
 #endif
 
-// a / 6: Div's quotient by a constant reciprocal, without its treatment of infinite a
-// (the quotient is then NaN, not infinite).
+// a / 6, 21 of them a face: Div's quotient by a constant reciprocal, without its
+// treatment of infinite a (the quotient is then NaN, not infinite).
 template <class R> HD R sixth(R a) { return Div<R>(R(6.))(a); }
 #if HAMR_DEVICE_ARITH
 template <> HD double sixth<double>(double a)
