@@ -2311,7 +2311,7 @@ int hamr_tune_set(hamr_ctx *c, int slot, const int *cfg)
 
 int hamr_time_stage(hamr_ctx *c, int stage, int nrep, double *avg_ms)
 {
-    if (!c || !avg_ms || nrep < 1 || stage < 0 || stage > 7) return fail(c, "hamr_time_stage: bad arguments");
+    if (!c || !avg_ms || nrep < 1 || stage < 0 || stage > 9) return fail(c, "hamr_time_stage: bad arguments");
     HIPCHK(c, hipSetDevice(c->device));
     hipEvent_t e0, e1;
     HIPCHK(c, hipEventCreate(&e0));
@@ -2331,7 +2331,9 @@ int hamr_time_stage(hamr_ctx *c, int stage, int nrep, double *avg_ms)
         case 4: pole(c, 0., c->dt); break;
         case 5: launch_ct_update(c->P, all_launch(c, TS_CT), 0., c->dt, 0.5, c->ps, c->psh, c->E, c->prec, c->s); break;
         case 6: update_all(c, 0, 0., c->dt, 0.5, c->p, c->p, c->ph, c->psh); break;
-        default: bound_all(c, c->ph, c->psh, true); break;
+        case 7: bound_all(c, c->ph, c->psh, true); break;
+        case 8: front_all(c, c->p, c->ps, nullptr); break;
+        default: corner_all(c); break;
         }
     }
     HIPCHK(c, hipEventRecord(e1, c->s));

@@ -376,10 +376,12 @@ int hamr_step_las_graph(hamr_ctx *ctx, int maxtl, int ncycles, double *dt_inout)
 int hamr_las_info(const hamr_ctx *ctx, long long *info);
 /* Average device time (ms, HIP events on the context stream) of one launch of
  * a stage over all blocks, with predictor-step operands (p and ps are not
- * modified): 0-2 flux x1..x3, 3 EMF, 4 polar average, 5 face-B update,
- * 6 conserved update + inversion, 7 ghost fill (3 directions) as the step
- * runs it after the update (the x3 ghost rows that the update writes left
- * out). */
+ * modified): 4 polar average, 5 face-B update, 6 conserved update + inversion,
+ * 7 ghost fill (3 directions) as the step runs it after the update (the x3
+ * ghost rows that the update writes left out), 8 fluxes and centre EMFs as the
+ * step launches them (one kernel by default), 9 corner EMFs; a half step is 4-9.
+ * 0-2: the flux of x1..x3 alone, 3: centre and corner EMFs, in the separate
+ * kernels that a step runs only where their launch shapes differ. */
 int hamr_time_stage(hamr_ctx *ctx, int stage, int nrep, double *avg_ms);
 /* ---- launch autotuner (no reference counterpart) ----
  * Every kernel of the step walks a work list of (block, tile) items.  For each
