@@ -22,7 +22,9 @@ using ::fabs;
 using ::fmin;
 
 // ---------------------------------------------------------------------------
-// Forward-mode number with N tangents (PPM Jacobian w.r.t. its 5 inputs).
+// Forward-mode number with N tangents (PPM Jacobian w.r.t. its 5 inputs).  The Jacobian
+// forms, up to para_jacobian, are in no kernel: the host checks hold para_vjp, which
+// is, against them.
 template <int N> struct Dual {
     double v, d[N];
     HD Dual() : v(0.) { for (int k = 0; k < N; k++) d[k] = 0.; }

@@ -50,7 +50,9 @@ static int default_swz(int cls) { return cls == KC_INTERIOR || cls == KC_FLAGS ?
 // tiles leave fewer lanes idle at the end of a block and of the launch.  256, 128, 64
 // threads, ms a step: 42x25x39 blocks FP64 0.980, 0.968, 0.970; 256x128x128 FP64 3.74, 3.68,
 // 3.69, mixed 2.76, 2.74, 2.77, HLLC mixed 3.09, 3.07, 3.09; HLLC 96x72x60 FP64 0.614, 0.601,
-// 0.594; 384x192x192 mixed 9.24, 9.21, 9.31.
+// 0.594; 384x192x192 mixed 9.24, 9.21, 9.31.  Launches over part of the blocks (one block,
+// the stepping levels of a cycle, the adjoint's fluxes) take kDefaultTile, where the
+// smaller tile is not measured.
 constexpr int kFrontTile = 1;
 
 struct TuneCfg {

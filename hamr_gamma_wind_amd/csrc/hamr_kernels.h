@@ -54,10 +54,10 @@ __host__ __device__ inline int las_phase(int tl, int s)
 // the grid is smaller than the list).  With swz = 1 the item order is permuted
 // so that the workgroups one XCD runs (ids congruent mod 8) take chunks of 32
 // consecutive items, the chunks dealt to the XCDs in turn: tiles whose stencils
-// share data meet in the same L2 (32 tiles are 8 planes of a 32^3 block), while
-// regions of the grid that take longer than others (the inversions) spread over
-// all XCDs, which one contiguous eighth of the list per XCD does not do (10-20%
-// slower for the update).
+// share data meet in the same L2 (32 tiles of 128 threads are 4 planes of a 32^3
+// block), while regions of the grid that take longer than others (the inversions)
+// spread over all XCDs, which one contiguous eighth of the list per XCD does not do
+// (10-20% slower for the update).
 struct WorkList {
     const int2 *items;
     int n;

@@ -556,13 +556,14 @@ __global__ void __launch_bounds__(256) k_invert(KParams P, WorkList wl, int full
 // and k_fallback finishes it.  Same arithmetic as k_cons + k_invert, bit for
 // bit.
 //
-// Bound by memory: 6.8 GB per launch on 384x192x192 mixed (4.5 GB needed; the
+// Bound by memory: 6.8 GB per launch on 384x192x192 mixed (5.0 GB needed; the
 // ghost cells between the z-rows add a fifth, the upper x1 fluxes are read
-// twice) at 4.2 TB/s, where a plain copy runs at 4.5.  Three waves per SIMD and all
-// loads of a cell issued together: with the fluxes read as they are added it
-// moved the same bytes 1.4x slower.  The per-column values (lapse, shift,
+// twice) at 4.2 TB/s, where a plain copy runs at 4.5.  Three waves per SIMD (two with
+// the per-tile push lookup, whose FP64 form takes 172 registers) and all loads of a
+// cell issued together: with the fluxes read as they are added it moved the same
+// bytes 1.4x slower.  The per-column values (lapse, shift,
 // floors, reciprocals) come staged with the metric instead of being formed per
-// cell, 2592 -> 2010 VALU instructions, and the literals are left in the loop
+// cell, 2592 -> 1965 VALU instructions, and the literals are left in the loop
 // (build.py): 2.09 -> 1.60 ms.
 template <class R, bool TILED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TILED ? 2 : 3)))

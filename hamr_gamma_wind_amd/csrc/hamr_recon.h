@@ -172,10 +172,13 @@ __device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, co
 
 // One thread per face: both parabolas of the face's two cells.
 //
-// Bound by the VALU (FP32: 1.55e3 instructions per face, x3 fluxes at 97% of the
-// issue rate; FP64: 1.98e3) and, beside it, by the latency of the stencil loads:
-// the limiter's branches keep the compiler from moving a load above the previous
-// variable's parabola, so that the 7 variables' loads waited one after another.
+// Bound by the float units (FP32: 1471-1543 instructions per face, x1, x2, x3 fluxes
+// with the float unit busy 74, 78, 92% of the cycles, where float instructions alone
+// reach 86-96%; FP64: 1.9e3, 55%, too few waves) and, beside it, by the latency of the
+// stencil loads: the limiter's branches keep the compiler from moving a load above the
+// previous variable's parabola, so that the 7 variables' loads waited one after another.
+// The x1 faces read 2.8 GB where the others read 1.3-1.4 (384x192x192): a chunk of an XCD
+// holds 3.5 of the planes that their stencils reach across.
 // With all 42 issued first and the metric's 21 in the middle: x1, x2, x3 fluxes
 // 418, 435, 400 -> 339, 346, 320 us (FP64, 256x128x128), 818, 855, 690 -> 768, 727,
 // 594 us (mixed, 384x192x192).  At least 3 waves per SIMD (FP64: 162 VGPRs; FP32
@@ -186,9 +189,9 @@ __device__ __forceinline__ void share_dt(const KParams &P, const BlockDev &B, co
 // once issues 29% fewer FP32 VALU instructions per face, but its carried state
 // takes 157 registers (three waves) and it ran 7-35% slower.
 // RS selects the Riemann solver: 0 HLL, 1 HLLC.  The FP64 HLLC kernel is held
-// at two waves per SIMD: 256 VGPRs with about 20 spilled to scratch ran 1.4x
-// faster than one wave with none spilled.  The FP32 HLLC kernel at four waves
-// (128 VGPRs, 9 spilled) ran 4% faster than at three (139, none spilled).
+// at two waves per SIMD (240 VGPRs, none spilled): 1.4x faster than one wave.  The
+// FP32 HLLC kernel at four waves (128 VGPRs, 28 bytes of scratch) ran 4% faster than
+// at three (139, none).
 template <int DIR, class R, int RS, bool SHARE = false>
 __device__ __forceinline__ void flux_item(const KParams &P, const int2 it, const double *__restrict__ p,
                                           const double *__restrict__ ps, R *__restrict__ F,
@@ -365,8 +368,8 @@ __device__ __forceinline__ void line_tile_states(const BlockDev &B, int item, co
     }
 }
 
-// Occupancy: four waves per SIMD in FP32 (<= 128 VGPRs), two in FP64 (the
-// FP64 states, speeds and fluxes need ~220 VGPRs).  The LDS of one tile:
+// Occupancy: four waves per SIMD in FP32 (128 VGPRs), two in FP64 (256 VGPRs and
+// 360-552 bytes of scratch, HLLC 644-844).  The LDS of one tile:
 // 2 (NPR - 1) kLineT values of R.
 template <int DIR, class R, int RS>
 __global__ void __launch_bounds__(kLineT) __attribute__((amdgpu_waves_per_eu(RS || sizeof(R) == 8 ? 2 : 4)))
@@ -451,7 +454,7 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // Per pass, four launches -> one: 64x32x32 FP64 1.93 -> 1.66 ms, 42x25x39 blocks 4.82
 // -> 4.28, 256x128x128 17.0 -> 16.5, HLLC 96x72x60 3.11 -> 2.71; mixed 384x192x192
 // 42.5 -> 40.1, HLLC 256x128x128 14.8 -> 13.4; the step of 384x192x192 by chunk
-// (items): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
+// (items of 256): all 9.78 ms, 16384 9.72, 8192 9.53, 4096 9.32, 2048 9.40, 1024 9.45.
 //
 // SHARE (uniform grids): ghost faces along x1 and x2 beyond a side with a block are
 // computed by that block only, which writes all their fluxes to both: 8% fewer faces on
@@ -462,7 +465,7 @@ __global__ void __launch_bounds__(256) k_emf_centre(KParams P, WorkList wl, cons
 // HAMR_EMF.)  Along x3 as well the blocks would write single values into the rows beside
 // them: no faster than computing the two faces more per row (384x192x192 2.09 and 2.07
 // ms a launch).
-constexpr int kFrontChunk = 1 << 20;  // threads: 4096 items of 256
+constexpr int kFrontChunk = 1 << 20;  // threads: 8192 items of the default 128
 template <class R, int RS, bool SHARE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RS ? (sizeof(R) == 4 ? 4 : 2) : 3)))
 k_front(KParams P, FrontLists L, const double *__restrict__ p, const double *__restrict__ ps, R *__restrict__ F1,

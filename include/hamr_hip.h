@@ -322,8 +322,9 @@ int hamr_clear_flags(hamr_ctx *ctx);
 /* Courant dt of the current state p/ps (per-block harmonic, min over blocks). */
 int hamr_estimate_dt(hamr_ctx *ctx, double *dt);
 /* nsteps predictor+corrector steps over all blocks with the dt kept on the
- * device (next dt = min over blocks, clamped to 1.3 dt).  *dt_inout: the first
- * step's dt on input (<= 0: keep the device value), the next dt on output. */
+ * device (next dt = min over blocks, clamped to 1.3 dt), from p/ps with their
+ * ghosts filled (hamr_boundprim(ctx, 1)).  *dt_inout: the first step's dt on
+ * input (<= 0: keep the device value), the next dt on output. */
 int hamr_step(hamr_ctx *ctx, int nsteps, double *dt_inout);
 /* Capture one step into a HIP graph and replay it nsteps times (same result as
  * hamr_step). */
